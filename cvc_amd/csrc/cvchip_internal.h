@@ -152,6 +152,7 @@ struct cvchip_ctx {
   hipEvent_t pin_ev[2] = {nullptr, nullptr};
   // reduction scratch
   cvchip::Scratch red;
+  size_t red_off = 0;     // where the operator's next partials start in red (doubles)
   cvchip::Scratch red2;   // first-stage sums of the two-stage partial reduction
   // idle device buffers of freed temporaries (solver, propagator and
   // contraction workspaces), reused by exact size: repeated calls allocate

@@ -1142,8 +1142,8 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
   const unsigned nblk = tr.nblk;
   double *part = nullptr;
   if (dm != DOT_NONE) {
-    CVC_TRY(ensure_red(c, sizeof(double) * ((size_t)nblk * 3 * N + 64 * 256)));
-    part = (double *)c->red.ptr;
+    CVC_TRY(ensure_red(c, sizeof(double) * (c->red_off + (size_t)nblk * 3 * N + 64 * 256)));
+    part = (double *)c->red.ptr + c->red_off;
   }
   const cplx<R> *U;
   if constexpr (sizeof(R) == 8) U = (RECON == 18) ? c->gauge64 : c->gauge64r12;
@@ -1344,19 +1344,33 @@ __global__ void k_reduce_partials(const double *__restrict__ part, int nblk, int
   if (threadIdx.x == 0) res[blockIdx.x] = sh[0];
 }
 
-int reduce_partials(cvchip_ctx *c, const double *part, int nblk, int Q, int N, double *res) {
-  const int rows = Q * N;
-  // segments of at least 4096 partials, at most 64 per row
-  int G = nblk / 4096;
-  if (G > 64) G = 64;
-  if (G >= 2) {
-    CVC_TRY(ensure_red2(c, sizeof(double) * (size_t)rows * G));
-    double *seg = (double *)c->red2.ptr;
-    hipLaunchKernelGGL(k_reduce_seg, dim3(rows * G), dim3(256), 0, c->stream, part, nblk, G, seg);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(rows), dim3(256), 0, c->stream, seg, G, Q, N, res);
-  } else {
-    hipLaunchKernelGGL(k_reduce_partials, dim3(rows), dim3(256), 0, c->stream, part, nblk, Q, N, res);
+// segments of at least 4096 partials, at most kSegMax per row
+constexpr int kSegMax = 64;
+
+int reduce_stage1(cvchip_ctx *c, const double *part, int nblk, int rows, int slot, const double **out, int *n) {
+  const int G = std::min(nblk / 4096, kSegMax);
+  if (G < 2) {
+    *out = part;
+    *n = nblk;
+    return 0;
   }
+  // both halves at the size of a full set of rows, so that neither call grows
+  // the scratch under the other's result
+  const size_t half = (size_t)3 * 256 * kSegMax;
+  CVC_TRY(ensure_red2(c, sizeof(double) * 2 * half));
+  double *seg = (double *)c->red2.ptr + slot * half;
+  hipLaunchKernelGGL(k_reduce_seg, dim3(rows * G), dim3(256), 0, c->stream, part, nblk, G, seg);
+  CVC_HIP(hipGetLastError());
+  *out = seg;
+  *n = G;
+  return 0;
+}
+
+int reduce_partials(cvchip_ctx *c, const double *part, int nblk, int Q, int N, double *res) {
+  const double *p = nullptr;
+  int n = 0;
+  CVC_TRY(reduce_stage1(c, part, nblk, Q * N, 0, &p, &n));
+  hipLaunchKernelGGL(k_reduce_partials, dim3(Q * N), dim3(256), 0, c->stream, p, n, Q, N, res);
   CVC_HIP(hipGetLastError());
   return 0;
 }

@@ -295,42 +295,111 @@ __device__ __forceinline__ void cdiv(double o[2], const double a[2], const doubl
   o[1] = im;
 }
 
+constexpr int kMaxGap = 48;
+
+// Sums Q rows of n block partials (row q at p + q stride) over the block in a
+// fixed order; the totals are valid in thread 0.  Four independent chains per
+// thread keep several loads in flight; waves add by lane shuffles and meet in LDS once.
+constexpr int kScThreads = 512;
+template <int Q>
+__device__ __forceinline__ void sum_rows(const double *__restrict__ p, size_t stride, int n, double out[Q]) {
+  __shared__ double ws[Q][kScThreads / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double a[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const double *row = p + q * stride;
+    double c[4] = {0., 0., 0., 0.};
+    int b = (int)threadIdx.x;
+    for (; b + 3 * kScThreads < n; b += 4 * kScThreads) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) c[k] += row[b + k * kScThreads];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++, b += kScThreads)
+      if (b < n) c[k] += row[b];
+    a[q] = (c[0] + c[1]) + (c[2] + c[3]);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) a[q] += __shfl_down(a[q], (unsigned)off, 64);
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) ws[q][w] = a[q];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      out[q] = 0.;
+      for (int k = 0; k < kScThreads / 64; k++) out[q] += ws[q][k];
+    }
+  }
+}
+
+// One block per right-hand side sums its rows of the partial dot products and
+// forms the recurrence's scalars in the same launch (a reduction kernel, a
+// clearing kernel and one-block scalar kernels before).  Latency bound: an
+// iteration on a small lattice is a chain of short launches, 72 -> 61 us at 8^4
+// with one rhs, a whole source at 16x8^3 71.7 -> 68.2 ms; at 32x16^3 with 12 rhs
+// the 6000 partials of a row took 11 us with one load in flight per thread,
+// 1.935 -> 1.908 ms per iteration.
+// part: rows (q N + rhs) of n partials.
+
 // alpha = r0rn / <r2,p2>
-__global__ void k_sc_alpha(RhsState *st, const double *res, int N) {
-  const int r = threadIdx.x;
-  if (r >= N) return;
+__global__ void __launch_bounds__(kScThreads) k_sc_alpha(RhsState *st, const double *__restrict__ part, int n, int N) {
+  const int r = blockIdx.x;
+  double w[2];
+  sum_rows<2>(part + (size_t)r * n, (size_t)N * n, n, w);
+  if (threadIdx.x) return;
   RhsState &S = st[r];
   if (S.final_upd) {
     S.done = 1;
     S.final_upd = 0;
   }
   if (S.done) return;
-  const double w[2] = {res[r], res[N + r]};
   cdiv(S.alpha, S.r0rn, w);
 }
 
-// omega = <t,s>/<t,t>
-__global__ void k_sc_omega(RhsState *st, const double *res, int N) {
-  const int r = threadIdx.x;
-  if (r >= N) return;
+// omega = <t,s>/<t,t> from one launch's three rows
+__global__ void __launch_bounds__(kScThreads) k_sc_omega(RhsState *st, const double *__restrict__ part, int n, int N) {
+  const int r = blockIdx.x;
+  double w[3];
+  sum_rows<3>(part + (size_t)r * n, (size_t)N * n, n, w);
   RhsState &S = st[r];
-  if (S.done) return;
-  const double inv = 1. / res[2 * N + r];
-  S.omega[0] = res[r] * inv;
-  S.omega[1] = res[N + r] * inv;
+  if (threadIdx.x || S.done) return;
+  const double inv = 1. / w[2];
+  S.omega[0] = w[0] * inv;
+  S.omega[1] = w[1] * inv;
 }
 
-constexpr int kMaxGap = 48;
+// the same from the norms of the two halves of the gamma5-hermitian operator:
+// <t,s> = |B s|^2 (partials ts, real) and <t,t> (partials tt)
+__global__ void __launch_bounds__(kScThreads) k_sc_omega_her(RhsState *st, const double *__restrict__ ts, int nts,
+                                                             const double *__restrict__ tt, int ntt) {
+  const int r = blockIdx.x;
+  double a[1], b[1];
+  sum_rows<1>(ts + (size_t)r * nts, 0, nts, a);
+  __syncthreads();
+  sum_rows<1>(tt + (size_t)r * ntt, 0, ntt, b);
+  RhsState &S = st[r];
+  if (threadIdx.x || S.done) return;
+  S.omega[0] = a[0] * (1. / b[0]);
+  S.omega[1] = 0.;
+}
 
 // after r1: convergence test (or reliable-update trigger), beta, r0rn
-__global__ void k_sc_beta(RhsState *st, const double *res, int N, int it, int lagged, int mixed,
-                          double delta2) {
-  const int r = threadIdx.x;
-  if (r >= N) return;
+__global__ void __launch_bounds__(kScThreads) k_sc_beta(RhsState *st, const double *__restrict__ part, int n, int N,
+                                                        int it, int lagged, int mixed, double delta2) {
+  const int r = blockIdx.x;
+  double res[3];
+  sum_rows<3>(part + (size_t)r * n, (size_t)N * n, n, res);
   RhsState &S = st[r];
-  if (S.done) return;
-  S.norm = res[r];
-  const double w[2] = {res[N + r], res[2 * N + r]};
+  if (threadIdx.x || S.done) return;
+  S.norm = res[0];
+  const double w[2] = {res[1], res[2]};
   if (!mixed) {
     if (S.norm <= S.tol2) {
       S.iter = it;
@@ -506,7 +575,8 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   S.nt = (size_t)S.VN * 192 >= ((size_t)256 << 20) ? 1 : 0;
   // room for the operator's partials too (its traversal has its own block count)
   const size_t nb_max = std::max<size_t>(S.nblk, dslash_blocks(c, N));
-  CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 3 * N + 64 * 256)));
+  // (two launches' norms side by side in Op::apply_omega)
+  CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 4 * N + 64 * 256)));
   CVC_HIP(hipMalloc(&S.st, sizeof(RhsState) * N));
   CVC_HIP(hipMalloc(&S.res, sizeof(double) * 4 * N));
   CVC_HIP(hipHostMalloc(&S.hst, sizeof(RhsState) * N, hipHostMallocDefault));
@@ -522,6 +592,17 @@ static void solve_free(Solve &S) {
 
 static int reduce(Solve &S, int nblk, int Q) {
   return reduce_partials(S.c, (const double *)S.c->red.ptr, nblk, Q, S.N, S.res);
+}
+
+// the preceding kernel's Q N rows of partials, in the first stage's segments when
+// there are many, to the scalar kernel that f launches
+template <typename F> static int scalar_rows(Solve &S, int nblk, int Q, F f) {
+  const double *p = nullptr;
+  int n = 0;
+  CVC_TRY(reduce_stage1(S.c, (const double *)S.c->red.ptr, nblk, Q * S.N, 0, &p, &n));
+  f(p, n);
+  CVC_HIP(hipGetLastError());
+  return 0;
 }
 
 static int pull_state(Solve &S) {
@@ -560,10 +641,6 @@ static int true_residual(Solve &S, Field &x, const Field &b, Field &tmp, double 
   return 0;
 }
 
-__global__ void k_zero_doubles(double *p, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0.;
-}
-
 // The operator of the recurrence: D(mu), or for the gamma5-hermitian system
 // A = gamma5 D(mu) gamma5 D(-mu) = Qf5(mu) Qf5(-mu) (invert_Qtm.c:325-327).
 struct Op {
@@ -580,24 +657,36 @@ struct Op {
     return dslash_eo(c, out, *tmp, &in, mutm, 1, 0, -0.5, g5, dm,
                      dm == DOT_TS ? (partner ? partner : &in) : partner, nb);
   }
-  // t = A in with <t,in> (complex) in res[0..N) / res[N..2N) and <t,t> in
-  // res[2N..3N).  For the gamma5-hermitian operator A = B^dagger B with
-  // B = gamma5 D(-mu) (gamma5 M(-mu) on the even/odd system), so
-  // <t,in> = <B in, B in> is the norm of the first application's output: both
-  // applications fuse a norm, and neither reads the input again.
-  int apply_ts(Field &out, const Field &in, cvchip_ctx *cc, int N, double *res) {
+  // t = A in and omega = <t,in> / <t,t> into the state.  For the
+  // gamma5-hermitian operator A = B^dagger B with B = gamma5 D(-mu) (gamma5
+  // M(-mu) on the even/odd system), so <t,in> = <B in, B in> is the norm of the
+  // first application's output: both applications fuse a norm, and neither
+  // reads the input again.  The second one's partials follow the first one's in
+  // the reduction scratch (solve_setup makes room for both).
+  int apply_omega(Field &out, const Field &in, cvchip_ctx *cc, int N, RhsState *st) {
     int nb1 = 0, nb2 = 0;
+    const double *p1 = nullptr, *p2 = nullptr;
+    int n1 = 0, n2 = 0;
     if (!her) {
       CVC_TRY(apply(out, in, DOT_TS, nullptr, &nb1));
-      return reduce_partials(cc, (const double *)cc->red.ptr, nb1, 3, N, res);
+      CVC_TRY(reduce_stage1(cc, (const double *)cc->red.ptr, nb1, 3 * N, 0, &p1, &n1));
+      hipLaunchKernelGGL(k_sc_omega, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, N);
+      CVC_HIP(hipGetLastError());
+      return 0;
     }
     if (eo) CVC_TRY(applyM(*aux, in, -c->mu, 1, DOT_NN, nullptr, &nb1));
     else CVC_TRY(dslash(c, *aux, in, -c->mu, 1, DOT_NN, nullptr, &nb1));
-    CVC_TRY(reduce_partials(cc, (const double *)cc->red.ptr, nb1, 1, N, res));
-    hipLaunchKernelGGL(k_zero_doubles, dim3(1), dim3(256), 0, cc->stream, res + N, N);
-    if (eo) CVC_TRY(applyM(out, *aux, c->mu, 1, DOT_NN, nullptr, &nb2));
-    else CVC_TRY(dslash(c, out, *aux, c->mu, 1, DOT_NN, nullptr, &nb2));
-    return reduce_partials(cc, (const double *)cc->red.ptr, nb2, 1, N, res + 2 * N);
+    c->red_off = (size_t)nb1 * N;
+    int rc;
+    if (eo) rc = applyM(out, *aux, c->mu, 1, DOT_NN, nullptr, &nb2);
+    else rc = dslash(c, out, *aux, c->mu, 1, DOT_NN, nullptr, &nb2);
+    c->red_off = 0;
+    CVC_TRY(rc);
+    CVC_TRY(reduce_stage1(cc, (const double *)cc->red.ptr, nb1, N, 0, &p1, &n1));
+    CVC_TRY(reduce_stage1(cc, (const double *)cc->red.ptr + (size_t)nb1 * N, nb2, N, 1, &p2, &n2));
+    hipLaunchKernelGGL(k_sc_omega_her, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, p2, n2);
+    CVC_HIP(hipGetLastError());
+    return 0;
   }
   int apply(Field &out, const Field &in, DotMode dm, const Field *r2, int *nb) {
     if (eo) {
@@ -676,17 +765,18 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
   if (!all_done) {
     TRY(op.apply(p2, p, DOT_R2, &r2, &nb));
     dcalls++;
-    TRY(reduce(S, nb, 2));
     for (int it = 0; it <= niter_max; it++) {
-      hipLaunchKernelGGL(k_sc_alpha, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N);
+      TRY(scalar_rows(S, nb, 2, [&](const double *q, int n) {
+        hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
+      }));
       hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt);
-      TRY(op.apply_ts(t, s, c, N, S.res));
+      TRY(op.apply_omega(t, s, c, N, S.st));
       dcalls++;
-      hipLaunchKernelGGL(k_sc_omega, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N);
       hipLaunchKernelGGL((k_r1_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
                          S.VN, N, (double *)c->red.ptr, S.nt);
-      TRY(reduce(S, (int)S.nblk, 3));
-      hipLaunchKernelGGL(k_sc_beta, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N, it, lagged, 0, 0.0);
+      TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
+        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N, it, lagged, 0, 0.0);
+      }));
       hipLaunchKernelGGL((k_xp_update<IO, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ix, ip, is, ir1, ip2,
                          S.st, S.VN, N, S.nt);
       CVC_HIP(hipGetLastError());
@@ -700,7 +790,6 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
       if (all_done) break;
       TRY(op.apply(p2, p, DOT_R2, &r2, &nb));
       dcalls++;
-      TRY(reduce(S, nb, 2));
     }
   }
   // final state (final_upd counts as converged)
@@ -817,17 +906,18 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
   if (!all_done) {
     TRY(opl.apply(p2, p, DOT_R2, &r2, &nb));
     dcalls++;
-    TRY(reduce(S, nb, 2));
     for (int it = 0; it <= niter_max; it++) {
-      hipLaunchKernelGGL(k_sc_alpha, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N);
+      TRY(scalar_rows(S, nb, 2, [&](const double *q, int n) {
+        hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
+      }));
       hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt);
-      TRY(opl.apply_ts(t, s, c, N, S.res));
+      TRY(opl.apply_omega(t, s, c, N, S.st));
       dcalls++;
-      hipLaunchKernelGGL(k_sc_omega, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N);
       hipLaunchKernelGGL((k_r1_update<IO, IOR>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
                          S.VN, N, (double *)c->red.ptr, S.nt);
-      TRY(reduce(S, (int)S.nblk, 3));
-      hipLaunchKernelGGL(k_sc_beta, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N, it, 0, 1, delta2);
+      TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
+        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N, it, 0, 1, delta2);
+      }));
       // xl += omega s + alpha p ; p = r1 + beta (p - omega p2)
       hipLaunchKernelGGL((k_xp_update<IOPlain<float>, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ixl, ip, is, ir1, ip2,
                          S.st, S.VN, N, S.nt);
@@ -886,7 +976,6 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
       if (all_done) break;
       TRY(opl.apply(p2, p, DOT_R2, &r2, &nb));
       dcalls++;
-      TRY(reduce(S, nb, 2));
     }
   }
   TRY(pull_state(S));

@@ -248,6 +248,11 @@ __device__ __forceinline__ void block_reduce_store(const double v[Q], double *__
 __global__ void k_reduce_partials(const double *__restrict__ part, int nblk, int Q, int N,
                                   double *__restrict__ res);
 
+// First stage alone, for kernels that add the rest of each row themselves: *out / *n
+// are the rows and their length, either part itself or segment sums in the
+// context's second scratch (half `slot` of it: two results may be in use at once).
+int reduce_stage1(cvchip_ctx *c, const double *part, int nblk, int rows, int slot, const double **out, int *n);
+
 int reduce_partials(cvchip_ctx *c, const double *part, int nblk, int Q, int N, double *res);
 
 // Workgroups are dispatched to the 8 XCDs round-robin (block b runs on XCD b % 8).
