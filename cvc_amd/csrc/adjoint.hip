@@ -34,8 +34,6 @@ int source_links(cvchip_ctx *c, const int src[4], SrcLinks *out);
 int launch_psi(cvchip_ctx *c, double2 *psi, const Field &dn, const SrcLinks &L, int nu);
 int contract_fields(cvchip_ctx *c, double *conn, double contact[8], const Field &up, const Field &dn,
                     const int src[4]);
-int invert_her_fields(cvchip_ctx *c, Field &x, const Field &b, double sp, int niter_max, int prec,
-                      double delta, unsigned flags, cvchip_stats *stats);
 
 struct AdjParams {
   ConnParams P;
@@ -341,19 +339,15 @@ __global__ void __launch_bounds__(256) k_dot_g5(double *__restrict__ part, const
   block_reduce_store<2>(dv, part, 1);
 }
 
-// 12-column set <-> columns col0.. of a 60-column set, optionally times gamma5
-__global__ void k_cols(double2 *__restrict__ dst, const double2 *__restrict__ src, uint32_t V, int to60, int col0,
-                       int g5) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;   // over 12 comps * V * 12 cols
-  if (i >= 144u * V) return;
-  const uint32_t r = i % 12u;
-  const uint32_t cs = i / 12u;                                 // comp * V + site
-  const uint32_t comp = cs / V;
-  const size_t o60 = (size_t)cs * 60 + col0 + r;
-  double2 v = to60 ? src[i] : src[o60];
-  if (g5 && comp >= 6) { v.x = -v.x; v.y = -v.y; }
-  if (to60) dst[o60] = v;
-  else dst[i] = v;
+// dst (n columns) = gamma5 times columns col0 .. col0 + n - 1 of a 60-column set
+__global__ void k_cols_g5(double2 *__restrict__ dst, const double2 *__restrict__ src, uint32_t V, uint32_t n, int col0) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;   // over 12 comps * V * n cols
+  if (i >= 12u * n * V) return;
+  const uint32_t r = i % n;
+  const uint32_t cs = i / n;                                   // comp * V + site
+  double2 v = src[(size_t)cs * 60 + col0 + r];
+  if (cs / V >= 6) { v.x = -v.x; v.y = -v.y; }
+  dst[i] = v;
 }
 
 // one site's 12 x 60 block of a 60-column set: out[c][col]
@@ -428,7 +422,7 @@ extern "C" int cvchip_cvc_gradient(cvchip_ctx *c, const int src[4], double qmax,
       ysp[nu] = site_of(c, src[0] + d[0], src[1] + d[1], src[2] + d[2], src[3] + d[3]);
     }
 
-    Field up, dn, xu, xd, b12, x12;
+    Field up, dn, xu, xd;
     double *cw = nullptr, *dqs = nullptr;
     double2 *psi = nullptr, *K = nullptr, *blk = nullptr;
     std::vector<double> conn((size_t)32 * V);
@@ -439,8 +433,6 @@ extern "C" int cvchip_cvc_gradient(cvchip_ctx *c, const int src[4], double qmax,
     if (!rc) rc = field_alloc(c, dn, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, xu, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, xd, 60, CVCHIP_PREC_F64);
-    if (!rc) rc = field_alloc(c, b12, 12, CVCHIP_PREC_F64);
-    if (!rc) rc = field_alloc(c, x12, 12, CVCHIP_PREC_F64);
     auto hipok = [&](hipError_t e, const char *w) {
       if (e != hipSuccess && !rc) rc = hip_fail(e, w, __FILE__, __LINE__);
     };
@@ -593,29 +585,18 @@ extern "C" int cvchip_cvc_gradient(cvchip_ctx *c, const int src[4], double qmax,
       }
     }
     // ---- adjoint solves: Lambda_up = g5 D(-mu)^-1 g5 Xi_up, Lambda_dn = g5 D(mu)^-1 g5 Xi_dn (in place)
-    const double mu0 = c->mu;
     for (int f = 0; f < 2 && !rc; f++) {
       Field &xi = f == 0 ? xu : xd;
-      for (int s = 0; s < 5 && !rc; s++) {
-        hipLaunchKernelGGL(k_cols, dim3((144u * V + 255) / 256), dim3(256), 0, c->stream, (double2 *)b12.data,
-                           (const double2 *)xi.data, V, 0, 12 * s, 1);
-        hipok(hipMemsetAsync(x12.data, 0, x12.bytes, c->stream), "adjoint");
-        c->mu = f == 0 ? -mu0 : mu0;
-        cvchip_stats st;
-        memset(&st, 0, sizeof(st));
-        if (!rc) rc = invert_her_fields(c, x12, b12, sp, niter_max, prec, delta, 0, &st);
-        c->mu = mu0;
-        if (rc > 0) rc = 0;
-        if (rc) break;
-        tot.iterations += st.iterations;
-        tot.converged += st.converged;
-        tot.reliable_updates += st.reliable_updates;
-        tot.dslash_calls += st.dslash_calls;
-        tot.seconds += st.seconds;
-        hipLaunchKernelGGL(k_cols, dim3((144u * V + 255) / 256), dim3(256), 0, c->stream, (double2 *)xi.data,
-                           (const double2 *)x12.data, V, 1, 12 * s, 1);
-        hipok(hipGetLastError(), "adjoint columns");
-      }
+      rc = solve_five_sources(c, xi, f == 0 ? -c->mu : c->mu,
+                              [&](Field &b, int s0, int ns) {
+                                const uint32_t n = 12u * (uint32_t)ns;
+                                hipLaunchKernelGGL(k_cols_g5, dim3((12u * n * V + 255) / 256), dim3(256), 0, c->stream,
+                                                   (double2 *)b.data, (const double2 *)xi.data, V, n, 12 * s0);
+                                CVC_HIP(hipGetLastError());
+                                return 0;
+                              },
+                              sp, niter_max, prec, delta, &tot);
+      if (!rc) rc = gamma5_inplace(c, xi);
     }
     // ---- dL/dmu = Im<Lambda_up, g5 S_up> - Im<Lambda_dn, g5 S_dn>
     double dmu = 0.;
@@ -672,8 +653,6 @@ extern "C" int cvchip_cvc_gradient(cvchip_ctx *c, const int src[4], double qmax,
     field_free(dn);
     field_free(xu);
     field_free(xd);
-    field_free(b12);
-    field_free(x12);
     if (cw) (void)hipFree(cw);
     if (dqs) (void)hipFree(dqs);
     if (psi) (void)hipFree(psi);

@@ -30,6 +30,7 @@
 #include <stdio.h>
 #include <string.h>
 #include <math.h>
+#include <algorithm>
 #include <vector>
 
 #include "contract_common.h"
@@ -365,36 +366,6 @@ __global__ void k_wi(double2 *__restrict__ wi, const double2 *__restrict__ conn,
   }
 }
 
-// -------------------------------------------------- point sources, copies
-// b[c][site][r] = delta(site, ys) delta(c, r) for r = 0..11 (12-column set)
-__global__ void k_point_sources(double2 *__restrict__ b, uint32_t V, uint32_t ys) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;   // over 12 * V * 12
-  if (i >= 144u * V) return;
-  const uint32_t r = i % 12u;
-  const uint32_t c = i / (12u * V);
-  const uint32_t site = (i / 12u) % V;
-  b[i] = make_double2((site == ys && c == r) ? 1.0 : 0.0, 0.0);
-}
-
-// dst (ND columns) [.., col0 + r] = src (12 columns) [.., r]
-__global__ void k_put_columns(double2 *__restrict__ dst, const double2 *__restrict__ src, uint32_t V, int ND,
-                              int col0) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;   // over 12 * V * 12
-  if (i >= 144u * V) return;
-  const uint32_t r = i % 12u;
-  const uint32_t cs = i / 12u;                                 // c * V + site
-  dst[(size_t)cs * ND + col0 + r] = src[i];
-}
-
-// dst columns col0 .. col0 + 11 of an nd-column FP64 set = the 12 columns of src
-int put_columns(cvchip_ctx *c, Field &dst, const Field &src, int col0) {
-  const uint32_t V = (uint32_t)c->lat.V;
-  hipLaunchKernelGGL(k_put_columns, dim3((144u * V + 255) / 256), dim3(256), 0, c->stream, (double2 *)dst.data,
-                     (const double2 *)src.data, V, dst.nrhs, col0);
-  CVC_HIP(hipGetLastError());
-  return 0;
-}
-
 // ------------------------------------------------------------------ Pi(q)
 // One pass of a length-L DFT along a direction of stride `stride` (in sites):
 // out[.. n ..] = sum_x w[(n x) mod L] in[.. x ..],  w[k] = exp(-2 pi i k / L).
@@ -584,47 +555,74 @@ extern "C" int cvchip_pi_q(cvchip_ctx *c, double *piq, const double *conn, const
 
 namespace cvchip {
 
+// Up to kBatchSites sites one solve takes the five 12-column sources together:
+// 12 columns leave the chip idle there (a launch is then mostly latency) and
+// the FP64 updates of the mixed solvers are shared by 60 columns.  One source
+// point, five solves of 12 against one of 60 per flavour (even/odd, FP16 /
+// FP32 / FP64 inside): 8^4 48 / 55 / 69 -> 15 / 18 / 28 ms, 16x8^3 55 / 63 / 85
+// -> 22 / 27 / 55 ms, 16^3x8 90 / 112 / 202 -> 60 / 93 / 202 ms, 32x16^3 256 /
+// 356 / 824 -> 238 / 351 / 729 ms.  Beyond, five times the workspaces (23 GB
+// at 32x16^3) buy nothing more; without room for them the sources go one by one.
+constexpr int64_t kBatchSites = 1 << 17;
+
+int solve_five_sources(cvchip_ctx *c, Field &out, double mu, const std::function<int(Field &, int, int)> &source,
+                       double sp, int niter_max, int prec, double delta, cvchip_stats *tot) {
+  // solves the 12 ns columns of b into x
+  auto solve = [&](Field &x, const Field &b, int ns) -> int {
+    if (hipMemsetAsync(x.data, 0, x.bytes, c->stream) != hipSuccess) return CVCHIP_ERR_HIP;
+    cvchip_stats st;
+    memset(&st, 0, sizeof(st));
+    const double mu0 = c->mu;
+    c->mu = mu;
+    const int rc = invert_her_fields(c, x, b, sp, niter_max, prec, delta, 0, &st);
+    c->mu = mu0;
+    if (rc < 0) return rc;
+    if (tot) {
+      // the iterations of 12 columns are those of the slowest of them
+      for (int k = 0; k < ns; k++)
+        tot->iterations += *std::max_element(c->col_iters.begin() + 12 * k, c->col_iters.begin() + 12 * (k + 1));
+      tot->converged += st.converged;
+      tot->reliable_updates += st.reliable_updates;
+      tot->dslash_calls += st.dslash_calls;
+      tot->seconds += st.seconds;
+      if (st.true_res2_max > tot->true_res2_max) tot->true_res2_max = st.true_res2_max;
+    }
+    return 0;
+  };
+  Field all, b, x;
+  bool have_all = c->lat.V <= kBatchSites;
+  int rc = 0;
+  if (have_all && field_alloc(c, all, 60, CVCHIP_PREC_F64)) have_all = false;
+  if (have_all) {
+    rc = source(all, 0, 5);
+    if (!rc) rc = solve(out, all, 5);
+  }
+  if (!have_all || rc == CVCHIP_ERR_OOM) {
+    rc = field_alloc(c, b, 12, CVCHIP_PREC_F64);
+    if (!rc) rc = field_alloc(c, x, 12, CVCHIP_PREC_F64);
+    for (int s = 0; s < 5 && !rc; s++) {
+      rc = have_all ? copy_columns(c, b, 0, all, 12 * s, 12) : source(b, s, 1);
+      if (!rc) rc = solve(x, b, 1);
+      if (!rc) rc = copy_columns(c, out, 12 * s, x, 0, 12);
+    }
+  }
+  field_free(all);
+  field_free(b);
+  field_free(x);
+  return rc;
+}
+
 // 5 x 12 up (mu) and 5 x 12 down (-mu) propagators from point sources at y + s^
 // (s = 0..3) and y (s = 4) into the 60-column sets up / dn (column 12 s + k),
 // with the gamma5-hermitian BiCGStab; statistics summed into tot.
 int solve_source_props(cvchip_ctx *c, const int src[4], double sp, int niter_max, int prec, double delta,
                        Field &up, Field &dn, cvchip_stats *tot) {
-  const uint32_t V = (uint32_t)c->lat.V;
-  Field b, x;
-  int rc = field_alloc(c, b, 12, CVCHIP_PREC_F64);
-  if (!rc) rc = field_alloc(c, x, 12, CVCHIP_PREC_F64);
-  const double mu0 = c->mu;
-  for (int s = 0; s < 5 && !rc; s++) {
-    const int d[4] = {s == 0, s == 1, s == 2, s == 3};
-    const uint32_t ys = site_of(c, src[0] + d[0], src[1] + d[1], src[2] + d[2], src[3] + d[3]);
-    for (int fl = 0; fl < 2 && !rc; fl++) {
-      hipLaunchKernelGGL(k_point_sources, dim3((144u * V + 255) / 256), dim3(256), 0, c->stream,
-                         (double2 *)b.data, V, ys);
-      if (hipMemsetAsync(x.data, 0, x.bytes, c->stream) != hipSuccess) rc = CVCHIP_ERR_HIP;
-      c->mu = fl == 0 ? mu0 : -mu0;              // down flavour: mu -> -mu (record 1)
-      cvchip_stats st;
-      memset(&st, 0, sizeof(st));
-      if (!rc) rc = invert_her_fields(c, x, b, sp, niter_max, prec, delta, 0, &st);
-      c->mu = mu0;
-      if (rc > 0) rc = 0;
-      if (rc) break;
-      if (tot) {
-        tot->iterations += st.iterations;
-        tot->converged += st.converged;
-        tot->reliable_updates += st.reliable_updates;
-        tot->dslash_calls += st.dslash_calls;
-        tot->seconds += st.seconds;
-        if (st.true_res2_max > tot->true_res2_max) tot->true_res2_max = st.true_res2_max;
-      }
-      Field &dst = fl == 0 ? up : dn;
-      hipLaunchKernelGGL(k_put_columns, dim3((144u * V + 255) / 256), dim3(256), 0, c->stream, (double2 *)dst.data,
-                         (const double2 *)x.data, V, 60, 12 * s);
-      if (hipGetLastError() != hipSuccess) rc = CVCHIP_ERR_HIP;
-    }
-  }
-  field_free(b);
-  field_free(x);
-  return rc;
+  uint32_t sites[5];
+  for (int s = 0; s < 5; s++)
+    sites[s] = site_of(c, src[0] + (s == 0), src[1] + (s == 1), src[2] + (s == 2), src[3] + (s == 3));
+  auto points = [&](Field &b, int s0, int ns) { return point_sources_at(c, b, ns, sites + s0); };
+  CVC_TRY(solve_five_sources(c, up, c->mu, points, sp, niter_max, prec, delta, tot));
+  return solve_five_sources(c, dn, -c->mu, points, sp, niter_max, prec, delta, tot);   // down flavour: mu -> -mu (record 1)
 }
 
 }  // namespace cvchip

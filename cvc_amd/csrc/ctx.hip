@@ -338,6 +338,16 @@ __global__ void k_point_sources_n(double2 *__restrict__ b, uint32_t V, uint32_t 
   b[i] = make_double2((site == ps.site[r / 12] && c == r % 12) ? 1.0 : 0.0, 0.0);
 }
 
+int point_sources_at(cvchip_ctx *c, Field &f, int nsrc, const uint32_t *sites) {
+  PointSites ps{};
+  for (int k = 0; k < nsrc; k++) ps.site[k] = sites[k];
+  const uint64_t n = (uint64_t)12 * f.V * f.nrhs;
+  hipLaunchKernelGGL(k_point_sources_n, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, (double2 *)f.data,
+                     (uint32_t)f.V, (uint32_t)f.nrhs, ps);
+  CVC_HIP(hipGetLastError());
+  return 0;
+}
+
 __global__ void k_zero16(uint4 *__restrict__ p, uint64_t n) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -351,6 +361,15 @@ __global__ void k_copy_columns(double2 *__restrict__ dst, const double2 *__restr
   const uint32_t r = (uint32_t)(i % n);
   const uint64_t cs = i / n;   // c V + site
   dst[cs * ND + d0 + r] = src[cs * NS + s0 + r];
+}
+
+int copy_columns(cvchip_ctx *c, Field &dst, int d0, const Field &src, int s0, int n) {
+  const uint64_t tot = (uint64_t)12 * dst.V * n;
+  hipLaunchKernelGGL(k_copy_columns, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->stream, (double2 *)dst.data,
+                     (const double2 *)src.data, (uint32_t)dst.V, (uint32_t)dst.nrhs, (uint32_t)src.nrhs, (uint32_t)d0,
+                     (uint32_t)s0, (uint32_t)n);
+  CVC_HIP(hipGetLastError());
+  return 0;
 }
 
 }  // namespace cvchip
@@ -392,7 +411,7 @@ extern "C" int cvchip_field_point_sources(cvchip_ctx *c, cvchip_field *fh, int n
       return CVCHIP_ERR_ARG;
     }
     const int L[4] = {c->lat.T, c->lat.LX, c->lat.LY, c->lat.LZ};
-    PointSites ps{};
+    uint32_t sites[kMaxPointSources];
     for (int k = 0; k < nsrc; k++) {
       const int *x = coords + 4 * k;
       for (int m = 0; m < 4; m++)
@@ -400,12 +419,9 @@ extern "C" int cvchip_field_point_sources(cvchip_ctx *c, cvchip_field *fh, int n
           set_error("source %d coordinate %d = %d outside 0..%d", k, m, x[m], L[m] - 1);
           return CVCHIP_ERR_ARG;
         }
-      ps.site[k] = (uint32_t)((((int64_t)x[0] * L[1] + x[1]) * L[2] + x[2]) * L[3] + x[3]);
+      sites[k] = (uint32_t)((((int64_t)x[0] * L[1] + x[1]) * L[2] + x[2]) * L[3] + x[3]);
     }
-    const uint64_t n = (uint64_t)12 * f.V * f.nrhs;
-    hipLaunchKernelGGL(k_point_sources_n, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream,
-                       (double2 *)f.data, (uint32_t)f.V, (uint32_t)f.nrhs, ps);
-    CVC_HIP(hipGetLastError());
+    CVC_TRY(point_sources_at(c, f, nsrc, sites));
     CVC_HIP(hipStreamSynchronize(c->stream));
     return CVCHIP_OK;
   });
@@ -430,11 +446,7 @@ extern "C" int cvchip_field_copy_columns(cvchip_ctx *c, cvchip_field *dst, int d
       return CVCHIP_ERR_ARG;
     }
     if (n == 0) return CVCHIP_OK;
-    const uint64_t tot = (uint64_t)12 * d.V * n;
-    hipLaunchKernelGGL(k_copy_columns, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->stream, (double2 *)d.data,
-                       (const double2 *)s.data, (uint32_t)d.V, (uint32_t)d.nrhs, (uint32_t)s.nrhs, (uint32_t)dst_col0,
-                       (uint32_t)src_col0, (uint32_t)n);
-    CVC_HIP(hipGetLastError());
+    CVC_TRY(copy_columns(c, dst->f, dst_col0, s, src_col0, n));
     CVC_HIP(hipStreamSynchronize(c->stream));
     return CVCHIP_OK;
   });

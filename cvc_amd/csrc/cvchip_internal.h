@@ -16,6 +16,7 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 #include <stddef.h>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -144,6 +145,8 @@ struct cvchip_ctx {
   // right-hand side r has converged); the operator skips those rhs
   const int *op_mask = nullptr;
   int op_mask_stride = 0;
+  // iterations of each right-hand side of the last solve (0: an exact start vector)
+  std::vector<int> col_iters;
   // staging for host <-> device transfers (AoS reference layout)
   double *stage = nullptr;
   size_t stage_bytes = 0;
@@ -194,6 +197,17 @@ void pool_release(cvchip_ctx *c);
 // host AoS [V][24] (nrhs contiguous fields) <-> device field rhs range
 int upload_aos(cvchip_ctx *c, Field &f, const double *host, int rhs0, int n);
 int download_aos(cvchip_ctx *c, const Field &f, double *host, int rhs0, int n);
+
+// f = unit point sources of the 12 spin-colour components at nsrc sites (column 12 k + a)
+int point_sources_at(cvchip_ctx *c, Field &f, int nsrc, const uint32_t *sites);
+// out (60 columns) = the solutions of the five 12-column sources that source(b, s0, ns) writes
+// into b (columns 12 k + a = source s0 + k), with the twisted mass mu; statistics added to tot
+int solve_five_sources(cvchip_ctx *c, Field &out, double mu, const std::function<int(Field &, int, int)> &source,
+                       double sp, int niter_max, int prec, double delta, cvchip_stats *tot);
+// dst[.., d0 + r] = src[.., s0 + r] for r < n (FP64 sets of one volume, ranges checked by the caller)
+int copy_columns(cvchip_ctx *c, Field &dst, int d0, const Field &src, int s0, int n);
+// f = gamma5 f (FP64 set)
+int gamma5_inplace(cvchip_ctx *c, Field &f);
 
 // Dslash launcher: out = D(mutm) in (gamma5_out: out = gamma5 D in).
 // Optional fused reductions, written as per-block partials into c->red:

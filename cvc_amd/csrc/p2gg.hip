@@ -22,9 +22,6 @@ int solve_source_props(cvchip_ctx *c, const int src[4], double sp, int niter_max
                        Field &up, Field &dn, cvchip_stats *tot);
 int contract_fields(cvchip_ctx *c, double *conn, double contact[8], const Field &up, const Field &dn,
                     const int src[4]);
-int invert_her_fields(cvchip_ctx *c, Field &x, const Field &b, double sp, int niter_max, int prec,
-                      double delta, unsigned flags, cvchip_stats *stats);
-int put_columns(cvchip_ctx *c, Field &dst, const Field &src, int col0);
 
 struct SeqParams {
   int col[4];
@@ -125,7 +122,7 @@ extern "C" int cvchip_field_sequential_sources(cvchip_ctx *c, cvchip_field *out,
 }
 
 // The whole P -> gamma gamma source point: 120 point propagators, 60
-// sequential sources and solves (12 at a time), the contraction.
+// sequential sources and solves, the contraction.
 extern "C" int cvchip_p2gg_source(cvchip_ctx *c, double *conn, double contact[8], const int src[4], int seq_timeslice,
                                   int seq_gamma_id, const int seq_mom[3], int propagator_position, double sp,
                                   int niter_max, int prec, double delta, cvchip_stats *stats) {
@@ -145,44 +142,26 @@ extern "C" int cvchip_p2gg_source(cvchip_ctx *c, double *conn, double contact[8]
     const int T = c->lat.T;
     const int tseq = (((src[0] + seq_timeslice) % T) + T) % T;   // p2gg_xspace.c:446
     const double sgn = 1. - 2. * propagator_position;
-    Field up, dn, seq, b, x;
+    Field up, dn, seq;
     int rc = field_alloc(c, up, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, dn, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, seq, 60, CVCHIP_PREC_F64);
-    if (!rc) rc = field_alloc(c, b, 12, CVCHIP_PREC_F64);
-    if (!rc) rc = field_alloc(c, x, 12, CVCHIP_PREC_F64);
     cvchip_stats tot;
     memset(&tot, 0, sizeof(tot));
     if (!rc) rc = solve_source_props(c, src, sp, niter_max, prec, delta, up, dn, &tot);
     Field &P = propagator_position == 0 ? up : dn;
     Field &Q = propagator_position == 0 ? dn : up;
-    const double mu0 = c->mu;
-    for (int s = 0; s < 5 && !rc; s++) {
-      rc = seq_sources(c, b, P, 12 * s, tseq, seq_gamma_id, seq_mom, sgn);
-      if (!rc && hipMemsetAsync(x.data, 0, x.bytes, c->stream) != hipSuccess) rc = CVCHIP_ERR_HIP;
-      if (rc) break;
-      c->mu = propagator_position == 0 ? mu0 : -mu0;
-      cvchip_stats st;
-      memset(&st, 0, sizeof(st));
-      rc = invert_her_fields(c, x, b, sp, niter_max, prec, delta, 0, &st);
-      c->mu = mu0;
-      if (rc > 0) rc = 0;
-      if (rc) break;
-      tot.iterations += st.iterations;
-      tot.converged += st.converged;
-      tot.reliable_updates += st.reliable_updates;
-      tot.dslash_calls += st.dslash_calls;
-      tot.seconds += st.seconds;
-      if (st.true_res2_max > tot.true_res2_max) tot.true_res2_max = st.true_res2_max;
-      rc = put_columns(c, seq, x, 12 * s);
-    }
+    if (!rc)
+      rc = solve_five_sources(c, seq, propagator_position == 0 ? c->mu : -c->mu,
+                              [&](Field &b, int s0, int) {
+                                return seq_sources(c, b, P, 12 * s0, tseq, seq_gamma_id, seq_mom, sgn);
+                              },
+                              sp, niter_max, prec, delta, &tot);
     if (!rc) rc = contract_fields(c, conn, contact, seq, Q, src);
     if (stats) *stats = tot;
     field_free(up);
     field_free(dn);
     field_free(seq);
-    field_free(b);
-    field_free(x);
     return rc;
   });
 }

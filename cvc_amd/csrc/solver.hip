@@ -714,6 +714,22 @@ __global__ void k_g5(double2 *__restrict__ f, uint32_t VN) {
   }
 }
 
+int gamma5_inplace(cvchip_ctx *c, Field &f) {
+  const uint32_t VN = (uint32_t)(f.V * f.nrhs);
+  hipLaunchKernelGGL(k_g5, dim3((VN + 255) / 256), dim3(256), 0, c->stream, (double2 *)f.data, VN);
+  CVC_HIP(hipGetLastError());
+  return 0;
+}
+
+// per right-hand side, as stats->iterations counts them
+static void record_iterations(Solve &S, int iters) {
+  S.c->col_iters.resize(S.N);
+  for (int r = 0; r < S.N; r++) {
+    const RhsState &h = S.hst[r];
+    S.c->col_iters[r] = iters == 0 ? 0 : (h.done || h.final_upd) ? h.iter + 1 : iters;
+  }
+}
+
 // FP64 BiCGStab (on the gamma5-hermitian system when her != 0; then b is
 // expected as gamma5 b and x receives y of A y = gamma5 b)
 static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int niter_max, unsigned flags,
@@ -794,6 +810,7 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
   }
   // final state (final_upd counts as converged)
   TRY(pull_state(S));
+  record_iterations(S, iters);
   int nconv = 0, maxit = 0;
   for (int r = 0; r < N; r++) {
     if (S.hst[r].done || S.hst[r].final_upd) {
@@ -979,6 +996,7 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
     }
   }
   TRY(pull_state(S));
+  record_iterations(S, iters);
   int nconv = 0, maxit = 0, nstall = 0;
   for (int r = 0; r < N; r++)
     if (S.hst[r].done && !S.hst[r].stalled) {
