@@ -17,6 +17,7 @@
 #include <stdint.h>
 #include <stddef.h>
 #include <functional>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -113,6 +114,18 @@ struct Field {
   cvchip_ctx *pool = nullptr;  // context whose idle-buffer pool takes the memory back (temporaries)
 };
 
+// Block-to-site mapping of an operator launch (see dslash.hip)
+struct Traversal {
+  uint32_t csz, bpc, nblk;
+  int mode;
+  uint32_t yb, runlen, bpr, nrun;
+  uint32_t bx, ncx, bpp, npx, npair, bpcol;
+  uint32_t zb, ncy, ncz, lzb, lyz, lA, colsz;
+  uint32_t mS, mM, mXP, mYP, mCP, mNR, mNPX;
+  int mXcd;
+  unsigned threads;   // workgroup size
+};
+
 struct Scratch {
   void *ptr = nullptr;
   size_t bytes = 0;
@@ -147,6 +160,8 @@ struct cvchip_ctx {
   int op_mask_stride = 0;
   // iterations of each right-hand side of the last solve (0: an exact start vector)
   std::vector<int> col_iters;
+  // traversals already planned, by policy, rhs count, lattice half and precision
+  mutable std::map<uint64_t, cvchip::Traversal> plans;
   // staging for host <-> device transfers (AoS reference layout)
   double *stage = nullptr;
   size_t stage_bytes = 0;

@@ -12,6 +12,8 @@
 // the link, and rebuilds the lower spin components from the upper ones.
 // Periodic wrap and the boundary phase are resolved in the kernel: there is no
 // halo.  Optional epilogues fuse the solver's per-rhs dot products.
+#include <math.h>
+
 #include <algorithm>
 
 #include <type_traits>
@@ -20,15 +22,32 @@
 
 namespace cvchip {
 
+// n / d for a divisor fixed for the launch and n < 2^31: a shift for d = 2^l
+// (m = 0, a branch uniform across the grid); else, with l = ceil(log2 d) and
+// m = ceil(2^(31 + l) / d), m d exceeds 2^(31 + l) by less than 2^l, so the
+// quotient of n m by 2^(31 + l) is exact: one high product and a shift, on the
+// scalar unit where n is uniform (a 32-bit division is about 20 instructions).
+struct FDiv {
+  uint32_t m;
+  int sh;
+};
+static FDiv make_fdiv(uint32_t d) {
+  int l = 0;
+  while (((uint64_t)1 << l) < d) l++;
+  if (((uint64_t)1 << l) == d) return FDiv{0u, l};
+  const uint64_t p = (uint64_t)1 << (31 + l);
+  return FDiv{(uint32_t)((p + d - 1) / d), l - 1};
+}
+__device__ __forceinline__ uint32_t fdiv(uint32_t n, FDiv f) { return f.m ? __umulhi(n, f.m) >> f.sh : n >> f.sh; }
+
 template <typename R>
 struct DParams {
   uint32_t V, VN, sX, sT;
   int N, T, LX, LY, LZ;
-  // log2 of LZ, LY, LX, sX, sT and of the traversal's LZt when a power of two,
-  // else -1 (coordinates then come from shifts and masks instead of divisions);
-  // 1/N, 1/S and 1/(S KL) for the small quotients of thread and staging indices
-  int shLZ, shLY, shLX, shSX, shST, shLZt;
-  float invN, invS, invKS;
+  // coordinates of a traversal index, and the quotients of the block index
+  FDiv fLZt, fLY, fLX, fT, fbpc, fbpcol, fbpp, fbpr, fncx, fslice, fncy, fncz;
+  // 1/N and 1/S for the small quotients of thread and staging indices
+  float invN, invS;
   int partner;   // DOT_TS: dot with the separate field r2 instead of the input
   // traversal (mode 1): the lattice is cut into chunks of csz consecutive
   // sites (one eighth of a time slice when possible), bpc blocks per chunk;
@@ -39,9 +58,11 @@ struct DParams {
   // sites), x within y block: the x and y neighbours of a run were touched a
   // few runs earlier and are still in the XCD's L2, and the t neighbours are
   // the slices the adjacent XCDs are working on at the same time.
-  // Mode 4: bricks of bt time slices x bx x-planes x yb y-rows (all z); the
-  // bricks of one (x, y) column follow each other in t on one XCD, so the
-  // sites in flight on an XCD form a compact 4D region.
+  // Mode 4: columns of bx x-planes x yb y-rows (all z) swept in t, slice by
+  // slice.  The (column, slice) pairs, slices fastest, are cut into eight runs
+  // of npx, one per XCD: the sites in flight on an XCD form a compact 4D region
+  // and its t neighbours are one cross-section away, whether or not the columns
+  // divide by eight.
   // Mode 5: columns of bx x-planes x yb y-rows x zb z-sites (powers of two)
   // swept along the whole t extent, one column at a time per XCD, with the
   // column's sites ordered z, y, x within a time slice: the t neighbour of a
@@ -50,7 +71,7 @@ struct DParams {
   uint32_t csz, bpc;
   int mode;
   uint32_t yb, runlen, bpr, nrun;
-  uint32_t bt, bx, ncx, bpb, bpcol;
+  uint32_t bx, ncx, bpp, npx, npair, bpcol;   // mode 4: bpp blocks per pair, npair pairs
   uint32_t zb, ncy, ncz, lzb, lyz, lA, colsz, sTt, sXt;
   // Mode 6 (k_dslash_march): mS columns per workgroup marched through mM
   // slices; patches of mXP x mYP x LZ columns (mNPX along x), mCP chunks of mS
@@ -76,10 +97,6 @@ struct DParams {
   int dstride;
 };
 
-// n / d and n % d for a divisor fixed for the launch: a shift and a mask when
-// d = 2^sh (sh >= 0, a branch uniform across the grid)
-__device__ __forceinline__ uint32_t qdiv(uint32_t n, uint32_t d, int sh) { return sh >= 0 ? n >> sh : n / d; }
-__device__ __forceinline__ uint32_t qmod(uint32_t n, uint32_t d, int sh) { return sh >= 0 ? n & (d - 1u) : n % d; }
 // floor(n / d) for n < 2^21 from inv, the float nearest 1/d (or within two
 // roundings of it): (n + 1/2) / d stays at least 1/(2d) away from an integer,
 // and the float product errs by less than (n + 1/2) 2^-22 / d
@@ -101,9 +118,11 @@ __device__ __forceinline__ void project(C h[2][3], Get get) {
   for (int c = 0; c < 3; c++) h[1][c] = cadd(get(3 + c), cunit<g1>(get(3 * p1 + c)));
 }
 
-// FP16 storage: the projection straight from the stored halves with the site's
-// scale n, each output real one pair of mixed-precision FMAs (half operand,
-// FP32 scale and accumulator): h = n A + u n B for the unit u of cunit.
+// FP16 storage: the projection of the stored halves, each output real one
+// mixed-precision FMA of half operands (exact sums of two halves, rounded once
+// to FP32; `one` is 1.0f, opaque to the compiler, which otherwise converts both
+// halves and adds).  The site's scale multiplies the link product where it is
+// added to the accumulator.
 __device__ __forceinline__ float half_lo(uint32_t w) {
   return (float)__builtin_bit_cast(_Float16, (unsigned short)(w & 0xffffu));
 }
@@ -111,22 +130,21 @@ __device__ __forceinline__ float half_hi(uint32_t w) {
   return (float)__builtin_bit_cast(_Float16, (unsigned short)(w >> 16));
 }
 template <int U>
-__device__ __forceinline__ float2 half_pair(uint32_t A, uint32_t B, float n) {
-  const float ax = __builtin_fmaf(half_lo(A), n, 0.0f), ay = __builtin_fmaf(half_hi(A), n, 0.0f);
-  if constexpr (U == 0) return make_float2(__builtin_fmaf(half_lo(B), n, ax), __builtin_fmaf(half_hi(B), n, ay));
-  else if constexpr (U == 1) return make_float2(__builtin_fmaf(half_lo(B), -n, ax), __builtin_fmaf(half_hi(B), -n, ay));
-  else if constexpr (U == 2) return make_float2(__builtin_fmaf(half_hi(B), -n, ax), __builtin_fmaf(half_lo(B), n, ay));
-  else return make_float2(__builtin_fmaf(half_hi(B), n, ax), __builtin_fmaf(half_lo(B), -n, ay));
+__device__ __forceinline__ float2 half_pair(uint32_t A, uint32_t B, float one) {
+  if constexpr (U == 0) return make_float2(__builtin_fmaf(half_lo(B), one, half_lo(A)), __builtin_fmaf(half_hi(B), one, half_hi(A)));
+  else if constexpr (U == 1) return make_float2(__builtin_fmaf(half_lo(B), -one, half_lo(A)), __builtin_fmaf(half_hi(B), -one, half_hi(A)));
+  else if constexpr (U == 2) return make_float2(__builtin_fmaf(half_hi(B), -one, half_lo(A)), __builtin_fmaf(half_lo(B), one, half_hi(A)));
+  else return make_float2(__builtin_fmaf(half_hi(B), one, half_lo(A)), __builtin_fmaf(half_lo(B), -one, half_hi(A)));
 }
 template <int MU, bool FWD>
-__device__ __forceinline__ void project_half(float2 h[2][3], const uint32_t w[12], float n) {
+__device__ __forceinline__ void project_half(float2 h[2][3], const uint32_t w[12], float one) {
   constexpr int p0 = GCOL[MU][0], p1 = GCOL[MU][1];
   constexpr int g0 = FWD ? uneg(GVAL[MU][0]) : GVAL[MU][0];
   constexpr int g1 = FWD ? uneg(GVAL[MU][1]) : GVAL[MU][1];
 #pragma unroll
-  for (int c = 0; c < 3; c++) h[0][c] = half_pair<g0>(w[c], w[3 * p0 + c], n);
+  for (int c = 0; c < 3; c++) h[0][c] = half_pair<g0>(w[c], w[3 * p0 + c], one);
 #pragma unroll
-  for (int c = 0; c < 3; c++) h[1][c] = half_pair<g1>(w[3 + c], w[3 * p1 + c], n);
+  for (int c = 0; c < 3; c++) h[1][c] = half_pair<g1>(w[3 + c], w[3 * p1 + c], one);
 }
 
 // acc += (1 - gamma_MU) U ph psi (FWD) or (1 + gamma_MU) U^dagger conj(ph) psi
@@ -145,10 +163,21 @@ __device__ __forceinline__ void rebuild_row3(C u[9]) {
   u[8] = mk<decltype(a.x)>(d.x, -d.y);
 }
 
-// PHASE false: the entries at base already carry the boundary phase
-template <typename R, int RECON, int MU, bool FWD, bool PHASE = true>
+// a + u n b for the unit code U of cunit (SCALED), or a + u b
+template <int U, bool SCALED, typename C, typename R>
+__device__ __forceinline__ C add_unit(C a, C b, R n) {
+  if constexpr (!SCALED) return cadd(a, cunit<U>(b));
+  else if constexpr (U == 0) return mk<R>(fmar(n, b.x, a.x), fmar(n, b.y, a.y));
+  else if constexpr (U == 1) return mk<R>(fmar(-n, b.x, a.x), fmar(-n, b.y, a.y));
+  else if constexpr (U == 2) return mk<R>(fmar(-n, b.y, a.x), fmar(n, b.x, a.y));
+  else return mk<R>(fmar(n, b.y, a.x), fmar(-n, b.x, a.y));
+}
+
+// PHASE false: the entries at base already carry the boundary phase; SCALED:
+// the spinor's scale n multiplies the product (FP16 storage)
+template <typename R, int RECON, int MU, bool FWD, bool PHASE = true, bool SCALED = false>
 __device__ __forceinline__ void link_apply(cplx<R> acc[12], const cplx<R> h[2][3],
-                                           const cplx<R> *__restrict__ base, uint32_t stride, cplx<R> ph) {
+                                           const cplx<R> *__restrict__ base, uint32_t stride, cplx<R> ph, R n = 1) {
   using C = cplx<R>;
   constexpr int q2 = GCOL[MU][2], q3 = GCOL[MU][3];
   constexpr int l2 = FWD ? uneg(GVAL[MU][2]) : GVAL[MU][2];
@@ -182,10 +211,10 @@ __device__ __forceinline__ void link_apply(cplx<R> acc[12], const cplx<R> h[2][3
       w0 = cmulc(ph, w0);
       w1 = cmulc(ph, w1);
     }
-    acc[i] = cadd(acc[i], w0);
-    acc[3 + i] = cadd(acc[3 + i], w1);
-    acc[6 + i] = cadd(acc[6 + i], cunit<l2>(q2 == 0 ? w0 : w1));
-    acc[9 + i] = cadd(acc[9 + i], cunit<l3>(q3 == 0 ? w0 : w1));
+    acc[i] = add_unit<0, SCALED>(acc[i], w0, n);
+    acc[3 + i] = add_unit<0, SCALED>(acc[3 + i], w1, n);
+    acc[6 + i] = add_unit<l2, SCALED>(acc[6 + i], q2 == 0 ? w0 : w1, n);
+    acc[9 + i] = add_unit<l3, SCALED>(acc[9 + i], q3 == 0 ? w0 : w1, n);
   }
 }
 
@@ -193,10 +222,64 @@ __device__ __forceinline__ void link_apply(cplx<R> acc[12], const cplx<R> h[2][3
 // U_mu(x - mu) (backward), 2*mu + 1 is U_mu(x) (forward).
 constexpr int LDS_SITES = 32;
 
-// Projected neighbour spinors.  With LDSS the block's own sites and the two
-// sites before and after them are staged in LDS, so the z neighbours
-// (adjacent sites) and the own spinor come from LDS instead of the texture
-// path.
+// A neighbour spinor as it is stored: loaded whole, projected later, so that
+// the loads of the next hop can be in flight during the products of this one.
+template <typename IO> struct Raw;
+template <> struct Raw<IOPlain<double>> {
+  double2 v[12];
+  __device__ __forceinline__ void load(const IOPlain<double> &in, uint32_t idx) { in.load(v, idx); }
+  __device__ __forceinline__ void full(double2 o[12]) const {
+#pragma unroll
+    for (int c = 0; c < 12; c++) o[c] = v[c];
+  }
+  template <int MU, bool FWD> __device__ __forceinline__ double project(double2 h[2][3], double) const {
+    cvchip::project<MU, FWD>(h, [&](int c) { return v[c]; });
+    return 1.;
+  }
+};
+template <> struct Raw<IOPlain<float>> {
+  float2 v[12];
+  __device__ __forceinline__ void load(const IOPlain<float> &in, uint32_t idx) { in.load(v, idx); }
+  __device__ __forceinline__ void full(float2 o[12]) const {
+#pragma unroll
+    for (int c = 0; c < 12; c++) o[c] = v[c];
+  }
+  template <int MU, bool FWD> __device__ __forceinline__ float project(float2 h[2][3], float) const {
+    cvchip::project<MU, FWD>(h, [&](int c) { return v[c]; });
+    return 1.f;
+  }
+};
+template <> struct Raw<IOHalf> {
+  uint32_t w[12];
+  float n;
+  __device__ __forceinline__ void load(const IOHalf &in, uint32_t idx) {
+    const uint4 *q = reinterpret_cast<const uint4 *>(in.p);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const uint4 v = q[(size_t)k * in.VN + idx];
+      w[4 * k] = v.x;
+      w[4 * k + 1] = v.y;
+      w[4 * k + 2] = v.z;
+      w[4 * k + 3] = v.w;
+    }
+    n = in.nrm[idx];
+  }
+  __device__ __forceinline__ void full(float2 o[12]) const {
+#pragma unroll
+    for (int c = 0; c < 12; c++) o[c] = make_float2(half_lo(w[c]) * n, half_hi(w[c]) * n);
+  }
+  template <int MU, bool FWD> __device__ __forceinline__ float project(float2 h[2][3], float one) const {
+    project_half<MU, FWD>(h, w, one);
+    return n;
+  }
+};
+template <typename IO> struct IsHalf { static constexpr bool value = false; };
+template <> struct IsHalf<IOHalf> { static constexpr bool value = true; };
+
+// Projected neighbour spinors, returning the scale that their link product
+// takes.  With LDSS the block's own sites and the two sites before and after
+// them are staged in LDS (scales applied), so the z neighbours (adjacent sites)
+// and the own spinor come from LDS instead of the texture path.
 template <typename IO, bool LDSS>
 struct NbLoader {
   using R = typename IO::real;
@@ -204,6 +287,7 @@ struct NbLoader {
   const IO &in;
   const C *Sp;
   uint32_t N, r, s0, S;
+  R one;
   // the staged slot of site, or -1
   __device__ __forceinline__ int slot(uint32_t site, bool from_lds) const {
     if constexpr (LDSS) {
@@ -215,32 +299,21 @@ struct NbLoader {
     return -1;
   }
   template <int MU, bool FWD>
-  __device__ __forceinline__ void proj(C h[2][3], uint32_t site, bool from_lds) const {
+  __device__ __forceinline__ R proj(C h[2][3], uint32_t site, bool from_lds) const {
     const int d = slot(site, from_lds);
     if (d >= 0) {
       const C *q = Sp + (uint32_t)d * 12 * N + r;
       project<MU, FWD>(h, [&](int c) { return q[c * N]; });
-      return;
+      return (R)1;
     }
     const uint32_t idx = site * N + r;
-    if constexpr (IO::K == 1) {
+    if constexpr (IO::K == 1) {   // each component loaded where it is used
       project<MU, FWD>(h, [&](int c) { return in.load_c(c, idx); });
-    } else if constexpr (IO::K == 4) {
-      const uint4 *q = reinterpret_cast<const uint4 *>(in.p);
-      uint32_t w[12];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const uint4 v = q[(size_t)k * in.VN + idx];
-        w[4 * k] = v.x;
-        w[4 * k + 1] = v.y;
-        w[4 * k + 2] = v.z;
-        w[4 * k + 3] = v.w;
-      }
-      project_half<MU, FWD>(h, w, in.nrm[idx]);
+      return (R)1;
     } else {
-      C v[12];
-      in.load(v, idx);
-      project<MU, FWD>(h, [&](int c) { return v[c]; });
+      Raw<IO> raw;
+      raw.load(in, idx);
+      return raw.template project<MU, FWD>(h, one);
     }
   }
   __device__ __forceinline__ void full(C v[12], uint32_t site, bool from_lds) const {
@@ -254,51 +327,112 @@ struct NbLoader {
   }
 };
 
-// Multi-rhs operator (links from LDS): the compiler would otherwise issue the
-// loads of all eight hops up front and defer the arithmetic to the epilogue
-// (the accumulator is not needed before), keeping every loaded value live,
-// spilling, and running one wave per SIMD.  An empty asm that reads and writes
-// the accumulator (and, at PIN 2, the projected half spinor) and clobbers
-// memory bounds each hop: its arithmetic is done before, and the next hop's
-// loads cannot move above it, so three to four waves fit per SIMD and cover
-// each other's latency.  The single-rhs operator keeps the compiler's
-// schedule (all loads in flight, one wave per SIMD): it is faster there.
-#ifndef CVC_HOP_PIN
-#define CVC_HOP_PIN 2
-#endif
+// Bounds a hop: an empty asm that reads and writes the accumulator (and the
+// projected half spinor) and clobbers memory, so that its arithmetic is done
+// before and the loads that follow cannot move above it (the compiler otherwise
+// issues the loads of all eight hops first, keeps every loaded value live and
+// runs one wave per SIMD).
 template <typename C>
 __device__ __forceinline__ void pin_regs(C *v, int n) {
 #pragma unroll
   for (int k = 0; k < n; k++) asm volatile("" : "+v"(v[k].x), "+v"(v[k].y) : : "memory");
 }
 
-template <typename IO, int RECON, int MU, bool LDSL, bool LDSS, bool EO>
-__device__ __forceinline__ void hop_pair(cplx<typename IO::real> acc[12], const NbLoader<IO, LDSS> &ld,
-                                         const cplx<typename IO::real> *__restrict__ U,
-                                         const cplx<typename IO::real> *__restrict__ Ul,
-                                         const DParams<typename IO::real> &P, uint32_t s, uint32_t sl,
-                                         int coord, int L, uint32_t stride) {
+// A thread's output site: traversal coordinates (zt counts half-sites on the
+// even/odd lattice), traversal index v, lexicographic site s, and there the
+// offset s - 2 v of an even/odd half-site.
+struct SitePos {
+  uint32_t t, x, y, zt, v, s, off;
+};
+
+// Hop h = 2 mu (backward) or 2 mu + 1 (forward): traversal index of the
+// neighbour.  A t, x or y neighbour on the even/odd lattice has the same zt
+// (its parity and the coordinate change together); the z neighbours of offset
+// off are zt - 1 + off and zt + off.
+template <int H, bool EO, typename R>
+__device__ __forceinline__ uint32_t neighbour(const SitePos &q, const DParams<R> &P) {
+  constexpr int MU = H >> 1;
+  constexpr bool FWD = (H & 1) != 0;
+  const uint32_t crd = MU == 0 ? q.t : MU == 1 ? q.x : MU == 2 ? q.y : q.zt;
+  const uint32_t L = (uint32_t)(MU == 0 ? P.T : MU == 1 ? P.LX : MU == 2 ? P.LY : (int)P.LZt);
+  const uint32_t str = MU == 0 ? P.sTt : MU == 1 ? P.sXt : MU == 2 ? P.LZt : 1u;
+  const uint32_t nb = FWD ? (crd == L - 1 ? q.v - (L - 1) * str : q.v + str)
+                          : (crd == 0 ? q.v + (L - 1) * str : q.v - str);
+  if constexpr (EO && MU == 3) return (q.off != 0) == FWD ? nb : q.v;
+  return nb;
+}
+
+// the site whose link the hop takes: s (forward), s - mu (backward)
+template <bool EO, typename R>
+__device__ __forceinline__ uint32_t link_site(const SitePos &q, const DParams<R> &P, int mu, bool fwd) {
+  if (fwd) return q.s;
+  const uint32_t crd = mu == 0 ? q.t : mu == 1 ? q.x : mu == 2 ? q.y : (EO ? 2u * q.zt + q.off : q.zt);
+  const uint32_t L = (uint32_t)(mu == 0 ? P.T : mu == 1 ? P.LX : mu == 2 ? P.LY : P.LZ);
+  const uint32_t str = mu == 0 ? P.sT : mu == 1 ? P.sX : mu == 2 ? (uint32_t)P.LZ : 1u;
+  return crd == 0 ? q.s + (L - 1) * str : q.s - str;
+}
+
+// one hop from the projected spinor h of scale n; links from LDS (Ul, slot sl) or memory
+template <typename IO, int RECON, int H, bool LDSL, bool EO>
+__device__ __forceinline__ void hop_links(cplx<typename IO::real> acc[12], const cplx<typename IO::real> h[2][3],
+                                          typename IO::real n, const cplx<typename IO::real> *__restrict__ U,
+                                          const cplx<typename IO::real> *__restrict__ Ul,
+                                          const DParams<typename IO::real> &P, const SitePos &q, uint32_t sl) {
   using R = typename IO::real;
+  constexpr int MU = H >> 1;
+  constexpr bool FWD = (H & 1) != 0;
   constexpr int KL = RECON == 18 ? 9 : 6;
   // staged whole with the phase applied (see k_dslash): read as full links, no phase multiply
   constexpr bool FOLD = LDSL && RECON == 12 && sizeof(R) == 4;
   constexpr int KS = FOLD ? 9 : KL;
   constexpr int RL = FOLD ? 18 : RECON;
+  constexpr bool SC = IsHalf<IO>::value;
+  if constexpr (LDSL) link_apply<R, RL, MU, FWD, !FOLD, SC>(acc, h, Ul + H * KS * LDS_SITES + sl, LDS_SITES, P.ph[MU], n);
+  else link_apply<R, RECON, MU, FWD, true, SC>(acc, h, U + (size_t)MU * KL * P.V + link_site<EO>(q, P, MU, FWD), P.V,
+                                               P.ph[MU], n);
+}
+
+// Hop H of the multi-rhs operator with its neighbour in raw, and the loads of
+// hop H + 1 (after the last, the own spinor's) in flight during the products of
+// this one: each wave has up to two neighbours' loads outstanding.  What bounds
+// the kernel: a wave's 108 (FP64) 1 KB loads mostly miss the 32 KB L1, and about
+// 40 % of them the XCD's L2; the FP64 kernel needs 182 VGPRs with the second
+// spinor in flight, so two waves per SIMD instead of four, which read 15.6
+// instead of 19.4 GB from beyond L2 at 64x32^3 with 12 rhs.  Together with the
+// batched link staging, the columns and the scalar index arithmetic, 12 rhs
+// (before -> now): FP64 64x32^3 3.90 -> 3.45 ms, 40x20^3 649 -> 500 us, 32x16^3
+// 246 -> 200 us; even/odd at 40x20^3 FP64 375 -> 288 us, FP32 188 -> 156 us,
+// FP16 108 -> 92 us.
+template <typename IO, int RECON, int H, bool EO>
+__device__ __forceinline__ void hop_pipelined(cplx<typename IO::real> acc[12], Raw<IO> &raw, const IO &in,
+                                              const IO &own, typename IO::real one, const cplx<typename IO::real> *__restrict__ Ul,
+                                              const DParams<typename IO::real> &P, const SitePos &q, uint32_t r,
+                                              uint32_t sl) {
+  using R = typename IO::real;
   cplx<R> h[2][3];
-  const uint32_t sm = coord == 0 ? s + (uint32_t)(L - 1) * stride : s - stride;
-  const uint32_t sp = coord == L - 1 ? s - (uint32_t)(L - 1) * stride : s + stride;
-  // backward: (1 + gamma_mu) U_mu(x-mu)^dagger phi(x-mu)
-  ld.template proj<MU, false>(h, EO ? sm >> 1 : sm, MU == 3);
-  if constexpr (LDSL && CVC_HOP_PIN == 2) pin_regs(&h[0][0], 6);
-  if constexpr (LDSL) link_apply<R, RL, MU, false, !FOLD>(acc, h, Ul + (2 * MU) * KS * LDS_SITES + sl, LDS_SITES, P.ph[MU]);
-  else link_apply<R, RECON, MU, false>(acc, h, U + (size_t)MU * KL * P.V + sm, P.V, P.ph[MU]);
-  if constexpr (LDSL && (CVC_HOP_PIN == 1 || CVC_HOP_PIN == 2)) pin_regs(acc, 12);
-  // forward: (1 - gamma_mu) U_mu(x) phi(x+mu)
-  ld.template proj<MU, true>(h, EO ? sp >> 1 : sp, MU == 3);
-  if constexpr (LDSL && CVC_HOP_PIN == 2) pin_regs(&h[0][0], 6);
-  if constexpr (LDSL) link_apply<R, RL, MU, true, !FOLD>(acc, h, Ul + (2 * MU + 1) * KS * LDS_SITES + sl, LDS_SITES, P.ph[MU]);
-  else link_apply<R, RECON, MU, true>(acc, h, U + (size_t)MU * KL * P.V + s, P.V, P.ph[MU]);
-  if constexpr (LDSL && CVC_HOP_PIN > 0) pin_regs(acc, 12);
+  Raw<IO> next;
+  if constexpr (H < 7) next.load(in, neighbour<H + 1, EO>(q, P) * (uint32_t)P.N + r);
+  else if constexpr (!EO) next.load(in, q.v * (uint32_t)P.N + r);
+  else if (P.dmode != 1) next.load(own, q.v * (uint32_t)P.N + r);
+  asm volatile("" : : : "memory");
+  const R n = raw.template project<(H >> 1), (H & 1) != 0>(h, one);
+  hop_links<IO, RECON, H, true, EO>(acc, h, n, nullptr, Ul, P, q, sl);
+  pin_regs(acc, 12);
+  raw = next;
+}
+
+// the same without LDS links or with staged spinors: load, project, multiply
+template <typename IO, int RECON, int H, bool LDSL, bool LDSS, bool EO>
+__device__ __forceinline__ void hop_plain(cplx<typename IO::real> acc[12], const NbLoader<IO, LDSS> &ld,
+                                          const cplx<typename IO::real> *__restrict__ U,
+                                          const cplx<typename IO::real> *__restrict__ Ul,
+                                          const DParams<typename IO::real> &P, const SitePos &q, uint32_t sl) {
+  using R = typename IO::real;
+  cplx<R> h[2][3];
+  const R n = ld.template proj<(H >> 1), (H & 1) != 0>(h, neighbour<H, EO>(q, P), (H >> 1) == 3);
+  if constexpr (LDSL) pin_regs(&h[0][0], 6);
+  hop_links<IO, RECON, H, LDSL, EO>(acc, h, n, U, Ul, P, q, sl);
+  if constexpr (LDSL) pin_regs(acc, 12);
 }
 
 // Minimum resident waves per SIMD the register allocation must allow (the
@@ -326,84 +460,89 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
   using C = cplx<R>;
   constexpr int KL = RECON == 18 ? 9 : 6;
   static_assert(!(EO && LDSS), "the even/odd operator stages no spinors");
-  // lexicographic site of traversal index v
-  auto lex_of = [&](uint32_t v) -> uint32_t {
-    if constexpr (!EO) {
-      return v;
-    } else {
-      const uint32_t zl = qmod(v, P.LZt, P.shLZt);
-      uint32_t q = qdiv(v, P.LZt, P.shLZt);
-      const uint32_t y = qmod(q, (uint32_t)P.LY, P.shLY);
-      q = qdiv(q, (uint32_t)P.LY, P.shLY);
-      const uint32_t x = qmod(q, (uint32_t)P.LX, P.shLX), t = qdiv(q, (uint32_t)P.LX, P.shLX);
-      return ((q * (uint32_t)P.LY + y) * (uint32_t)P.LZ) + 2u * zl + (((uint32_t)P.par + t + x + y) & 1u);
-    }
-  };
   const uint32_t S = blockDim.x / (uint32_t)P.N;
-  uint32_t s0 = 0, s_end = 0;   // modes 0-4: the block's contiguous traversal range
-  uint32_t jb = 0, cbase = 0;   // mode 5: first column-local index, column origin
-  if (P.mode == 5) {
-    const uint32_t k = blockIdx.x / kXcds;
-    const uint32_t col = (k / P.bpcol) * kXcds + blockIdx.x % kXcds;
-    jb = (k - (k / P.bpcol) * P.bpcol) * S;
-    const uint32_t cz = col % P.ncz, q = col / P.ncz;
-    const uint32_t cy = q % P.ncy, cx = q / P.ncy;
-    cbase = ((cx * P.bx) * (uint32_t)P.LY + cy * P.yb) * P.LZt + cz * P.zb;
-  } else if (P.mode == 4) {
-    const uint32_t k = blockIdx.x / kXcds;
-    const uint32_t col = k / P.bpcol, rem = k - col * P.bpcol;
-    const uint32_t brick = rem / P.bpb, rem2 = rem - brick * P.bpb;
-    const uint32_t run = rem2 / P.bpr, blk = rem2 - run * P.bpr;
-    const uint32_t c = col * kXcds + blockIdx.x % kXcds;
-    const uint32_t cy = c / P.ncx, cx = c - cy * P.ncx;
-    const uint32_t tin = run / P.bx, xin = run - tin * P.bx;
-    const uint32_t t = brick * P.bt + tin, x = cx * P.bx + xin;
-    const uint32_t start = ((t * (uint32_t)P.LX + x) * (uint32_t)P.LY + cy * P.yb) * P.LZt;
-    s0 = start + blk * S;
-    s_end = min(s0 + S, start + P.runlen);
+  // The block's range of slots, from the block index by scalar quotients.
+  // Rows (modes 2, 4): slots j0 .. of a run of yb rows at (t0, x0, y0).
+  // Chunks (modes 0, 1): consecutive traversal indices j0 .. jend.  Mode 5: slots
+  // j0 .. of a column at (x0, y0, zt0).
+  const uint32_t bx8 = blockIdx.x / kXcds, b8 = blockIdx.x % kXcds;
+  uint32_t t0 = 0, x0 = 0, y0 = 0, z0 = 0, j0, jend;
+  if (P.mode == 4) {
+    const uint32_t k = fdiv(bx8, P.fbpp), rem = bx8 - k * P.bpp;
+    const uint32_t xin = fdiv(rem, P.fbpr), blk = rem - xin * P.bpr;
+    const uint32_t pair = b8 * P.npx + k;
+    const uint32_t col = fdiv(pair, P.fT), cy = fdiv(col, P.fncx);
+    t0 = pair - col * (uint32_t)P.T;
+    x0 = (col - cy * P.ncx) * P.bx + xin;
+    y0 = cy * P.yb;
+    j0 = blk * S;
+    jend = pair < P.npair ? P.runlen : 0u;   // the last XCD's run may be shorter
   } else if (P.mode == 2) {
-    const uint32_t k = blockIdx.x / kXcds;
-    const uint32_t per_slice = P.nrun * P.bpr;
-    const uint32_t tl = k / per_slice, rem = k - tl * per_slice;
-    const uint32_t run = rem / P.bpr, blk = rem - run * P.bpr;
-    const uint32_t t = tl * kXcds + blockIdx.x % kXcds;
-    const uint32_t ybl = run / (uint32_t)P.LX, x = run - ybl * (uint32_t)P.LX;
-    const uint32_t start = ((t * (uint32_t)P.LX + x) * (uint32_t)P.LY + ybl * P.yb) * P.LZt;
-    s0 = start + blk * S;
-    s_end = min(s0 + S, start + P.runlen);
+    const uint32_t tl = fdiv(bx8, P.fslice), rem = bx8 - tl * (P.nrun * P.bpr);
+    const uint32_t run = fdiv(rem, P.fbpr), blk = rem - run * P.bpr;
+    const uint32_t ybl = fdiv(run, P.fLX);
+    t0 = tl * kXcds + b8;
+    x0 = run - ybl * (uint32_t)P.LX;
+    y0 = ybl * P.yb;
+    j0 = blk * S;
+    jend = P.runlen;
+  } else if (P.mode == 5) {
+    const uint32_t cl = fdiv(bx8, P.fbpcol), col = cl * kXcds + b8;
+    const uint32_t q = fdiv(col, P.fncz), cx = fdiv(q, P.fncy);
+    z0 = (col - q * P.ncz) * P.zb;
+    y0 = (q - cx * P.ncy) * P.yb;
+    x0 = cx * P.bx;
+    j0 = (bx8 - cl * P.bpcol) * S;
+    jend = P.colsz;
   } else {
     uint32_t chunk, blk;
     if (P.mode == 1) {
-      const uint32_t j = blockIdx.x / kXcds;
-      chunk = (j / P.bpc) * kXcds + blockIdx.x % kXcds;
-      blk = j % P.bpc;
+      const uint32_t k = fdiv(bx8, P.fbpc);
+      chunk = k * kXcds + b8;
+      blk = bx8 - k * P.bpc;
     } else {
-      chunk = blockIdx.x / P.bpc;
-      blk = blockIdx.x % P.bpc;
+      chunk = fdiv(blockIdx.x, P.fbpc);
+      blk = blockIdx.x - chunk * P.bpc;
     }
-    s0 = chunk * P.csz + blk * S;
-    s_end = min(s0 + S, (chunk + 1) * P.csz);
+    j0 = chunk * P.csz + blk * S;
+    jend = (chunk + 1) * P.csz;
   }
-  // traversal index (site, or half-site for EO) of block slot sl; false past
-  // the end of the block's range
-  auto slot_v = [&](uint32_t sl, uint32_t &v) -> bool {
-    if (P.mode == 5) {
-      const uint32_t j = jb + sl;
-      v = 0;
-      if (j >= P.colsz) return false;
+  const uint32_t vrow = ((t0 * (uint32_t)P.LX + x0) * (uint32_t)P.LY + y0) * P.LZt;   // rows: traversal index of slot 0
+  // position of block slot sl; false past the end of the block's range
+  auto slot_pos = [&](uint32_t sl, SitePos &q) -> bool {
+    const uint32_t j = j0 + sl;
+    if (j >= jend) return false;
+    if (P.mode == 2 || P.mode == 4) {
+      const uint32_t dy = fdiv(j, P.fLZt);
+      q.t = t0;
+      q.x = x0;
+      q.y = y0 + dy;
+      q.zt = j - dy * P.LZt;
+      q.v = vrow + j;
+    } else if (P.mode == 5) {
       const uint32_t rem = j & ((1u << P.lA) - 1u);
-      v = cbase + (j >> P.lA) * P.sTt + (rem >> P.lyz) * P.sXt + ((rem >> P.lzb) & (P.yb - 1u)) * P.LZt +
-          (rem & (P.zb - 1u));
-      return true;
+      q.t = j >> P.lA;
+      q.x = x0 + (rem >> P.lyz);
+      q.y = y0 + ((rem >> P.lzb) & (P.yb - 1u));
+      q.zt = z0 + (rem & (P.zb - 1u));
+      q.v = ((q.t * (uint32_t)P.LX + q.x) * (uint32_t)P.LY + q.y) * P.LZt + q.zt;
+    } else {
+      uint32_t k = fdiv(j, P.fLZt);
+      q.zt = j - k * P.LZt;
+      const uint32_t k2 = fdiv(k, P.fLY);
+      q.y = k - k2 * (uint32_t)P.LY;
+      q.t = fdiv(k2, P.fLX);
+      q.x = k2 - q.t * (uint32_t)P.LX;
+      q.v = j;
     }
-    v = s0 + sl;
-    return v < s_end;
+    q.off = EO ? ((uint32_t)P.par + q.t + q.x + q.y) & 1u : 0u;
+    q.s = EO ? 2u * q.v + q.off : q.v;
+    return true;
   };
   const uint32_t sl = sdiv(threadIdx.x, P.invN);
   const uint32_t r = threadIdx.x - sl * (uint32_t)P.N;
-  uint32_t vs;
-  const bool active = slot_v(sl, vs) && !(P.done && P.done[(size_t)r * P.dstride]);
-  const uint32_t i = vs * (uint32_t)P.N + r;
+  SitePos q;
+  const bool active = slot_pos(sl, q) && !(P.done && P.done[(size_t)r * P.dstride]);
   double dv[3] = {0., 0., 0.};
   // FP32 / FP16 with 2-row links: the staged links are whole (third row rebuilt)
   // and carry the boundary phase, both done once per site here instead of once
@@ -412,24 +551,20 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
   constexpr bool FOLD = LDSL && RECON == 12 && sizeof(R) == 4;
   constexpr int KS = FOLD ? 9 : KL;
   __shared__ C Ul[LDSL ? 8 * KS * LDS_SITES : 1];
-  // the link of hop hopi (2 mu: backward, U_mu(x - mu); 2 mu + 1: forward) of lexicographic site
-  auto link_site = [&](uint32_t hopi, uint32_t site) -> uint32_t {
-    if (hopi & 1u) return site;
-    const int mu = (int)(hopi >> 1);
-    const uint32_t str = mu == 0 ? P.sT : mu == 1 ? P.sX : mu == 2 ? (uint32_t)P.LZ : 1u;
-    const int shs = mu == 0 ? P.shST : mu == 1 ? P.shSX : mu == 2 ? P.shLZ : 0;
-    const uint32_t L = (uint32_t)(mu == 0 ? P.T : mu == 1 ? P.LX : mu == 2 ? P.LY : P.LZ);
-    const int shl = mu == 0 ? -1 : mu == 1 ? P.shLX : mu == 2 ? P.shLY : P.shLZ;
-    const uint32_t crd = qmod(qdiv(site, str, shs), L, shl);
-    return crd == 0 ? site + (L - 1) * str : site - str;
-  };
+  // the first neighbour's loads are in flight while the links are staged
+  constexpr bool PIPE = LDSL && !LDSS;
+  Raw<IOI> raw;
+  if constexpr (PIPE) {
+    if (active) raw.load(in, neighbour<0, EO>(q, P) * (uint32_t)P.N + r);
+    asm volatile("" : : : "memory");
+  }
   if constexpr (FOLD) {
     for (uint32_t e = threadIdx.x; e < 8u * S; e += blockDim.x) {
       const uint32_t hopi = sdiv(e, P.invS), sle = e - hopi * S;
-      uint32_t ve;
-      if (!slot_v(sle, ve)) continue;
-      const uint32_t ls = link_site(hopi, lex_of(ve));
+      SitePos qe;
+      if (!slot_pos(sle, qe)) continue;
       const int mu = (int)(hopi >> 1);
+      const uint32_t ls = link_site<EO>(qe, P, mu, (hopi & 1u) != 0);
       C u[9];
 #pragma unroll
       for (int k = 0; k < 6; k++) u[k] = U[((size_t)mu * 6 + k) * P.V + ls];
@@ -439,30 +574,26 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
     }
     __syncthreads();
   } else if constexpr (LDSL) {
-    const uint32_t tot = 8u * KL * S;
-    for (uint32_t e = threadIdx.x; e < tot; e += blockDim.x) {
-      const uint32_t hopi = sdiv(e, P.invKS), rem = e - hopi * (KL * S);
-      const uint32_t k = sdiv(rem, P.invS), sle = rem - k * S;
-      uint32_t ve;
-      if (!slot_v(sle, ve)) continue;
-      const uint32_t site = lex_of(ve);
+    // all entries of a link in flight together: one memory latency per block
+    for (uint32_t e = threadIdx.x; e < 8u * S; e += blockDim.x) {
+      const uint32_t hopi = sdiv(e, P.invS), sle = e - hopi * S;
+      SitePos qe;
+      if (!slot_pos(sle, qe)) continue;
       const int mu = (int)(hopi >> 1);
-      uint32_t ls = site;
-      if ((hopi & 1u) == 0) {          // backward hop: link at site - mu
-        const uint32_t str = mu == 0 ? P.sT : mu == 1 ? P.sX : mu == 2 ? (uint32_t)P.LZ : 1u;
-        const int shs = mu == 0 ? P.shST : mu == 1 ? P.shSX : mu == 2 ? P.shLZ : 0;
-        const uint32_t L = (uint32_t)(mu == 0 ? P.T : mu == 1 ? P.LX : mu == 2 ? P.LY : P.LZ);
-        const int shl = mu == 0 ? -1 : mu == 1 ? P.shLX : mu == 2 ? P.shLY : P.shLZ;
-        const uint32_t crd = qmod(qdiv(site, str, shs), L, shl);
-        ls = crd == 0 ? site + (L - 1) * str : site - str;
-      }
-      Ul[(hopi * KL + k) * LDS_SITES + sle] = U[((size_t)mu * KL + k) * P.V + ls];
+      const uint32_t ls = link_site<EO>(qe, P, mu, (hopi & 1u) != 0);
+      C u[KL];
+#pragma unroll
+      for (int k = 0; k < KL; k++) u[k] = U[((size_t)mu * KL + k) * P.V + ls];
+#pragma unroll
+      for (int k = 0; k < KL; k++) Ul[(hopi * KL + k) * LDS_SITES + sle] = u[k];
     }
     __syncthreads();
   }
   extern __shared__ unsigned char dyn_lds[];
   C *Sp = reinterpret_cast<C *>(dyn_lds);
+  uint32_t s0 = 0;   // first traversal index of the block's (contiguous) range
   if constexpr (LDSS) {
+    s0 = P.mode == 2 || P.mode == 4 ? vrow + j0 : j0;
     // stage sites s0-1 .. s0+S (all rhs); (s0 - 1 + k) mod V, every index is a valid site
     const uint32_t nst = (S + 2) * (uint32_t)P.N;
     for (uint32_t u = threadIdx.x; u < nst; u += blockDim.x) {
@@ -475,33 +606,26 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
     }
     __syncthreads();
   }
-  const NbLoader<IOI, LDSS> ld{in, Sp, (uint32_t)P.N, r, s0, S};
+  // 1.0f that the compiler does not know (see project_half)
+  R one = (R)1;
+  if constexpr (IsHalf<IOI>::value) asm volatile("" : "+v"(one));
+  const NbLoader<IOI, LDSS> ld{in, Sp, (uint32_t)P.N, r, s0, S, one};
   if (active) {
-    const uint32_t s = lex_of(vs);
-    const uint32_t t = qdiv(s, P.sT, P.shST);
-    uint32_t rem = s - t * P.sT;
-    const uint32_t x = qdiv(rem, P.sX, P.shSX);
-    rem -= x * P.sX;
-    const uint32_t y = qdiv(rem, (uint32_t)P.LZ, P.shLZ);
-    const uint32_t z = rem - y * (uint32_t)P.LZ;
-
+    const uint32_t i = q.v * (uint32_t)P.N + r;
     C acc[12];
 #pragma unroll
     for (int c = 0; c < 12; c++) acc[c] = mk<R>(0, 0);
-#ifndef CVC_HOP_ORDER
-#define CVC_HOP_ORDER 0
-#endif
-#define CVC_HOP(MU, CRD, L, STR) hop_pair<IOI, RECON, MU, LDSL, LDSS, EO>(acc, ld, U, Ul, P, s, sl, (int)(CRD), L, STR)
-#if CVC_HOP_ORDER == 0
-    CVC_HOP(0, t, P.T, P.sT); CVC_HOP(1, x, P.LX, P.sX); CVC_HOP(2, y, P.LY, (uint32_t)P.LZ); CVC_HOP(3, z, P.LZ, 1u);
-#elif CVC_HOP_ORDER == 1
-    CVC_HOP(1, x, P.LX, P.sX); CVC_HOP(2, y, P.LY, (uint32_t)P.LZ); CVC_HOP(3, z, P.LZ, 1u); CVC_HOP(0, t, P.T, P.sT);
-#elif CVC_HOP_ORDER == 2
-    CVC_HOP(0, t, P.T, P.sT); CVC_HOP(3, z, P.LZ, 1u); CVC_HOP(2, y, P.LY, (uint32_t)P.LZ); CVC_HOP(1, x, P.LX, P.sX);
-#else
-    CVC_HOP(0, t, P.T, P.sT); CVC_HOP(1, x, P.LX, P.sX); CVC_HOP(3, z, P.LZ, 1u); CVC_HOP(2, y, P.LY, (uint32_t)P.LZ);
-#endif
+    // t first: its neighbours are the farthest apart, and this order hits L2
+    // most often (9.4 M KiB fetched against 12.4 M with t last, 12 rhs FP64)
+    if constexpr (PIPE) {
+#define CVC_HOP(H) hop_pipelined<IOI, RECON, H, EO>(acc, raw, in, own_f, one, Ul, P, q, r, sl)
+      CVC_HOP(0); CVC_HOP(1); CVC_HOP(2); CVC_HOP(3); CVC_HOP(4); CVC_HOP(5); CVC_HOP(6); CVC_HOP(7);
 #undef CVC_HOP
+    } else {
+#define CVC_HOP(H) hop_plain<IOI, RECON, H, LDSL, LDSS, EO>(acc, ld, U, Ul, P, q, sl)
+      CVC_HOP(0); CVC_HOP(1); CVC_HOP(2); CVC_HOP(3); CVC_HOP(4); CVC_HOP(5); CVC_HOP(6); CVC_HOP(7);
+#undef CVC_HOP
+    }
 
     // the shadow residual of the <r2, out> epilogue is read once per launch:
     // streaming loads, issued beside the own spinor's (the latencies overlap)
@@ -509,7 +633,8 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
     if constexpr (DM == DOT_R2) r2.load_nt(w2, i);
     C own[12];
     if constexpr (!EO) {
-      ld.full(own, s, true);
+      if constexpr (PIPE) raw.full(own);
+      else ld.full(own, q.v, true);
       const R mh = (R)-0.5;
 #pragma unroll
       for (int c = 0; c < 12; c++) {
@@ -522,7 +647,10 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
         acc[c] = o;
       }
     } else {
-      if (P.dmode != 1) own_f.load(own, i);
+      if (P.dmode != 1) {
+        if constexpr (PIPE) raw.full(own);
+        else own_f.load(own, i);
+      }
 #pragma unroll
       for (int c = 0; c < 12; c++) {
         const R m = c < 6 ? P.mutm : -P.mutm;
@@ -644,6 +772,18 @@ __device__ __forceinline__ void link_mul(cplx<R> w[2][3], const cplx<R> h[2][3],
   }
 }
 
+// the scale of an FP16 spinor, on its link product
+template <typename IO, typename C, typename R>
+__device__ __forceinline__ void scale_w(C w[2][3], R n) {
+  if constexpr (IsHalf<IO>::value) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      w[0][i] = cscale(w[0][i], n);
+      w[1][i] = cscale(w[1][i], n);
+    }
+  }
+}
+
 template <typename C, int MU, bool FWD>
 __device__ __forceinline__ void expand_w(C acc[12], const C w[2][3]) {
   constexpr int q2 = GCOL[MU][2], q3 = GCOL[MU][3];
@@ -715,7 +855,9 @@ k_dslash_march(IOO out, IOI in, const cplx<typename IOI::real> *__restrict__ U, 
   const uint32_t t0 = rng * P.mM;
   extern __shared__ unsigned char dyn_lds[];
   C *Ul = reinterpret_cast<C *>(dyn_lds);   // [kMarchSlots][KS][S]
-  const NbLoader<IOI, false> ld{in, nullptr, (uint32_t)P.N, r, 0, 0};
+  R one = (R)1;   // opaque to the compiler (see project_half)
+  if constexpr (IsHalf<IOI>::value) asm volatile("" : "+v"(one));
+  const NbLoader<IOI, false> ld{in, nullptr, (uint32_t)P.N, r, 0, 0, one};
   double dv[3] = {0., 0., 0.};
 
   // carry: (U_0^dagger (1 + gamma_0) phi)(t - 1) as the six complex numbers w
@@ -724,8 +866,9 @@ k_dslash_march(IOO out, IOI in, const cplx<typename IOI::real> *__restrict__ U, 
     const uint32_t tm = t0 == 0 ? (uint32_t)P.T - 1 : t0 - 1;
     const uint32_t sm = tm * P.sT + sxyz;
     C h[2][3];
-    ld.template proj<0, false>(h, sm, false);
+    const R n = ld.template proj<0, false>(h, sm, false);
     link_mul<R, RECON, false, true>(carry, h, U + sm, P.V, P.ph[0]);
+    scale_w<IOI>(carry, n);
   }
 
   for (uint32_t step = 0; step < P.mM; step++) {
@@ -788,14 +931,16 @@ k_dslash_march(IOO out, IOI in, const cplx<typename IOI::real> *__restrict__ U, 
       const uint32_t sm_ = (CRD) == 0 ? s + (uint32_t)((L) - 1) * (STR) : s - (STR);                          \
       const uint32_t sp_ = (CRD) == (uint32_t)(L) - 1 ? s - (uint32_t)((L) - 1) * (STR) : s + (STR);           \
       C h[2][3], w[2][3];                                                                                      \
-      ld.template proj<MU, false>(h, sm_, false);                                                              \
+      R n = ld.template proj<MU, false>(h, sm_, false);                                                        \
       pin_regs(&h[0][0], 6);                                                                                   \
       link_mul<R, RL, false, !FOLD>(w, h, Ul + (3 + MU) * KS * S + cl, S, P.ph[MU]);                           \
+      scale_w<IOI>(w, n);                                                                                      \
       expand_w<C, MU, false>(acc, w);                                                                          \
       pin_regs(acc, 12);                                                                                       \
-      ld.template proj<MU, true>(h, sp_, false);                                                               \
+      n = ld.template proj<MU, true>(h, sp_, false);                                                           \
       pin_regs(&h[0][0], 6);                                                                                   \
       link_mul<R, RL, true, !FOLD>(w, h, Ul + (MU)*KS * S + cl, S, P.ph[MU]);                                  \
+      scale_w<IOI>(w, n);                                                                                      \
       expand_w<C, MU, true>(acc, w);                                                                           \
       pin_regs(acc, 12);                                                                                       \
     }
@@ -808,9 +953,10 @@ k_dslash_march(IOO out, IOI in, const cplx<typename IOI::real> *__restrict__ U, 
     {
       const uint32_t sp = t == (uint32_t)P.T - 1 ? sxyz : s + P.sT;
       C h[2][3], w[2][3];
-      ld.template proj<0, true>(h, sp, false);
+      const R n = ld.template proj<0, true>(h, sp, false);
       pin_regs(&h[0][0], 6);
       link_mul<R, RL, true, !FOLD>(w, h, Ul + cl, S, P.ph[0]);
+      scale_w<IOI>(w, n);
       expand_w<C, 0, true>(acc, w);
     }
     const R mh = (R)-0.5;
@@ -877,14 +1023,8 @@ static DParams<R> make_params(const cvchip_ctx *c, int N, double mutm) {
   P.LZ = c->lat.LZ;
   P.sX = (uint32_t)(c->lat.LY * c->lat.LZ);
   P.sT = (uint32_t)(c->lat.LX * c->lat.LY * c->lat.LZ);
-  P.shLZ = log2_exact((uint32_t)c->lat.LZ);
-  P.shLY = log2_exact((uint32_t)c->lat.LY);
-  P.shLX = log2_exact((uint32_t)c->lat.LX);
-  P.shSX = log2_exact(P.sX);
-  P.shST = log2_exact(P.sT);
-  P.shLZt = P.shLZ;
   P.invN = 1.0f / (float)N;
-  P.invS = P.invKS = 0.f;
+  P.invS = 0.f;
   P.k2 = (R)(0.5 / c->kappa);
   P.mutm = (R)mutm;
   for (int m = 0; m < 4; m++) P.ph[m] = mk<R>((R)c->ph.re[m], (R)c->ph.im[m]);
@@ -901,17 +1041,6 @@ template <> IOPlain<float> make_io<IOPlain<float>>(const Field &f) {
 template <> IOHalf make_io<IOHalf>(const Field &f) {
   return IOHalf{(__half2 *)f.data, f.norm, (uint32_t)(f.V * f.nrhs)};
 }
-
-struct Traversal {
-  uint32_t csz, bpc, nblk;
-  int mode;
-  uint32_t yb, runlen, bpr, nrun;
-  uint32_t bt, bx, ncx, bpb, bpcol;
-  uint32_t zb, ncy, ncz, lzb, lyz, lA, colsz;
-  uint32_t mS, mM, mXP, mYP, mCP, mNR, mNPX;
-  int mXcd;
-  unsigned threads;   // workgroup size
-};
 
 // t-march geometry (mode 6) for N rhs on the whole lattice L; bits 8-15 of the
 // policy give the march length M (0: 16; the largest divisor of T not above
@@ -947,65 +1076,114 @@ static bool march_geometry(const cvchip_ctx *c, int N, Traversal &t, bool explic
 }
 
 
+// Sites per operator block for runs of len sites: at most what fits 256
+// threads, the count that pads the run least, and among equals the largest whose
+// S N is a multiple of 8, so that a block's stores begin and end on 128-byte
+// lines (a line shared by two blocks is written twice, in halves).
+static uint32_t op_sites(int N, uint32_t len) {
+  const uint32_t S0 = (uint32_t)(block_for(N) / N);
+  if (N < 8) return S0;   // links from memory: blocks of 256 threads win although their last one is padded more
+  auto cost = [&](uint32_t S) {   // padded sites, and the halved lines as sites
+    const uint64_t nb = (len + S - 1) / S;
+    return 16 * nb * S + (S * (uint32_t)N % 8 ? nb * S / 2 + 16 : 0);
+  };
+  uint32_t best = S0;
+  for (uint32_t S = S0; S > 0 && 2 * S >= S0; S--)
+    if (cost(S) < cost(best)) best = S;
+  return best;
+}
+
+// The columns of the automatic traversal (mode 4): bx planes x yb rows of the
+// lattice L (its half for the even/odd operator) for N rhs.  A step in t should still find the last
+// slice's cross-section in the XCD's 4 MB L2 beside what streams through (the
+// outputs, the links, the neighbours of the columns' sides), so of the divisors
+// of LX and LY those are taken that read the fewest sides again (weight hw per
+// unit of 2/bx + 2/yb) while the cross-section's spinors stay below `budget`
+// bytes, corrected for padded blocks and for XCDs that get a pair less.  Sweep
+// of 0.6-9 MB and hw 0.1-0.7 over 24 operators (FP64, FP64 / FP32 / FP16
+// even/odd on six lattices): geometric mean 1.5 % above the best of each at
+// 1.5 MB and 0.3, 4-6 % at 1.2 and 2.4 MB.
+static void best_columns(const Lattice &L, int N, int K, uint32_t &bx, uint32_t &yb) {
+  const double site = 12. * 16 / K * N;   // bytes of a site's spinors
+  const double budget = 1.5e6, hw = 0.3;
+  double best = 0.;
+  bx = yb = 1;
+  for (int cx = 1; cx <= L.LX; cx++) {
+    if (L.LX % cx) continue;
+    for (int cy = 1; cy <= L.LY; cy++) {
+      if (L.LY % cy) continue;
+      const uint32_t len = (uint32_t)(cy * L.LZ), S = op_sites(N, len);
+      const double pad = (double)((len + S - 1) / S * S) / len;
+      const double npair = (double)(L.LX / cx) * (L.LY / cy) * L.T, npx = ceil(npair / kXcds);
+      const double halo = (cx < L.LX ? 2. / cx : 0.) + (cy < L.LY ? 2. / cy : 0.);
+      const double over = site * cx * len / budget;
+      const double cost = (1. + hw * halo + (over > 1. ? hw * 2 * (1. - 1. / over) : 0.)) * pad * (npx * kXcds / npair);
+      if (best == 0. || cost < best) {
+        best = cost;
+        bx = (uint32_t)cx;
+        yb = (uint32_t)cy;
+      }
+    }
+  }
+}
+
 // Block-to-site mapping; the policy's bits 4-7 pick the mode (0: automatic),
-// bits 8-15 the y-block height of modes 2, 4 and 5 (0: automatic), bits 16-19
-// and 20-23 the brick's t and x extents of mode 4 (0: 4); for mode 5, bits
-// 16-19 are log2 of the column's z extent (0: 8) and bits 20-23 its x extent
-// (0: 4).
+// bits 8-15 the y-block height of modes 2, 4 and 5 (0: automatic), bits 20-23
+// the columns' x extent of mode 4 (0: 4 or 1; its t extent in bits 16-19 does not
+// change the order); for mode 5, bits 16-19 are log2 of the column's z extent
+// (0: 8) and bits 20-23 its x extent (0: 4).
+// Automatic: N >= 8 the columns of best_columns; below, XCD chunks of a slice
+// (one rhs at 64x32^3: 0.46 ms against 0.51-0.57 ms for the other traversals).
 // K: complexes per 16 bytes of the operator's spinors (1 FP64, 2 FP32, 4
-// FP16+norm).  The FP32 operator's automatic traversal is the t march with
-// marches of 4 slices for 8 <= N <= 20 (at 64x32^3, per 12 rhs: 1.72-1.80 ms
-// against 1.92-2.06 ms for the best bricks with 12 rhs, 1.74 against 1.91 ms
-// with 16) and bricks beyond (24 rhs: 1.83 ms against 1.93 ms for the march);
-// the FP64 and FP16 operators keep the bricks
-static Traversal traversal(const cvchip_ctx *c, int N, bool eo = false, int K = 1) {
+// FP16+norm).  The FP32 operator on the whole lattice marches in t (mode 6,
+// marches of 4 slices) where a set of up to 16 rhs is 2 GiB or more: 1.73 ms
+// against 1.87 ms for the columns at 64x32^3 with 12 rhs; on smaller lattices the
+// columns win (40x20^3 268 against 431 us, 32x16^3 110 against 139 us, 32^4 with
+// 20 rhs 1.54 against 1.56 ms).
+static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
   Lattice L = c->lat;
   if (eo) {   // the half lattice of one parity: LZ/2 half-sites per z line
     L.LZ /= 2;
     L.V /= 2;
   }
   const uint32_t V = (uint32_t)L.V, slice = (uint32_t)(L.LX * L.LY * L.LZ);
-  const uint32_t S = (uint32_t)(block_for(N) / N);
   int want = (c->dslash_policy >> 4) & 15;
   if (want == 6) {
     Traversal t{};
     if (!eo && march_geometry(c, N, t, true, 16)) return t;
     want = 4;   // the even/odd operator does not march
   }
-  if (want == 0 && K == 2 && !eo && N >= 8 && N <= 20) {
+  if (want == 0 && K == 2 && !eo && N >= 8 && N <= 16 && (uint64_t)V * N * 96 >= ((uint64_t)1 << 31) &&
+      L.LX % 8 == 0 && L.LY % 8 == 0) {
     Traversal t{};
     if (march_geometry(c, N, t, false, 4)) return t;
   }
   uint32_t yb = (uint32_t)((c->dslash_policy >> 8) & 255);
-  // automatic: bricks of 4 slices x 4 x-planes x yb y-rows for the multi-rhs
-  // operator, else one slice per XCD in y blocks (both measured at 64x32^3
-  // with 12 rhs: 3.98 and 4.19 ms against 4.75 ms for XCD chunks of a
-  // slice); XCD chunks of a slice for a single rhs (0.48 ms against 0.54).
-  // The brick's y extent shrinks as N grows so that the spinor bytes of a
-  // brick's x-y cross-section stay about constant, yb * N <= 96 K: measured at
-  // 64x32^3, FP64 12 rhs best at yb 8, 24 rhs at 4, 48 rhs at 2; FP32 24 rhs
-  // at 8, 48 rhs at 4 (1.86 ms per 12 rhs against 1.96-1.99 ms at yb 2); FP16
-  // 12 rhs at 16 (1.18 ms against 1.20 ms at yb 8).
-  const bool autom = want == 0;
-  if (autom) want = N >= 8 ? 4 : 1;
+  uint32_t bx = (uint32_t)((c->dslash_policy >> 20) & 15);
+  if (want == 0 && N >= 8) {
+    best_columns(L, N, K, bx, yb);
+    want = 4;
+  }
+  if (want == 0) want = 1;
   if (yb == 0) {
     yb = 1;
-    if (autom && want == 4) {
-      const uint32_t budget = 96u * (uint32_t)K;
-      for (uint32_t y : {16u, 8u, 4u, 2u})
-        if (y * (uint32_t)N <= budget && L.LY % (int)y == 0) { yb = y; break; }
-    } else {
-      for (uint32_t y : {16u, 8u, 4u, 2u})
-        if (L.LY % (int)y == 0) { yb = y; break; }
-    }
+    for (uint32_t y : {16u, 8u, 4u, 2u})
+      if (L.LY % (int)y == 0) { yb = y; break; }
   }
+  if (bx == 0) bx = L.LX % 4 == 0 ? 4 : 1;
   Traversal t{};
-  t.threads = (unsigned)block_for(N);
+  uint32_t S = 1;
+  // blocks of S sites over runs of len sites
+  auto runs = [&](uint32_t len) {
+    S = op_sites(N, len);
+    t.threads = S * (unsigned)N;
+    return (len + S - 1) / S;
+  };
   if (want == 5) {
     const uint32_t cyb = (c->dslash_policy >> 8) & 255 ? yb : 4u;
     const uint32_t lz = (c->dslash_policy >> 16) & 15;
     const uint32_t czb = lz ? (1u << lz) : 8u;
-    const uint32_t cbx = (c->dslash_policy >> 20) & 15 ? (c->dslash_policy >> 20) & 15 : 4u;
+    const uint32_t cbx = (c->dslash_policy >> 20) & 15 ? bx : 4u;
     const int l1 = log2_exact(cbx), l2 = log2_exact(cyb), l3 = log2_exact(czb);
     if (l1 >= 0 && l2 >= 0 && l3 >= 0 && L.LX % (int)cbx == 0 && L.LY % (int)cyb == 0 && L.LZ % (int)czb == 0) {
       const uint32_t ncol = (uint32_t)(L.LX / (int)cbx) * (uint32_t)(L.LY / (int)cyb) * (uint32_t)(L.LZ / (int)czb);
@@ -1020,29 +1198,24 @@ static Traversal traversal(const cvchip_ctx *c, int N, bool eo = false, int K = 
         t.lyz = (uint32_t)(l2 + l3);
         t.lA = (uint32_t)(l1 + l2 + l3);
         t.colsz = (uint32_t)L.T << t.lA;
-        t.bpcol = (t.colsz + S - 1) / S;
+        t.bpcol = runs(t.colsz);
         t.nblk = ncol * t.bpcol;
         return t;
       }
     }
     want = 4;   // a column request that does not tile the lattice falls back to bricks
   }
-  uint32_t bt = (uint32_t)((c->dslash_policy >> 16) & 15), bx = (uint32_t)((c->dslash_policy >> 20) & 15);
-  if (bt == 0) bt = 4;
-  if (bx == 0) bx = 4;
-  if (want == 4 && L.T % (int)bt == 0 && L.LX % (int)bx == 0 && L.LY % (int)yb == 0 &&
-      ((uint32_t)(L.LX / (int)bx) * (uint32_t)(L.LY / (int)yb)) % kXcds == 0) {
+  if (want == 4 && L.LX % (int)bx == 0 && L.LY % (int)yb == 0) {
     t.mode = 4;
     t.yb = yb;
-    t.bt = bt;
     t.bx = bx;
     t.ncx = (uint32_t)L.LX / bx;
     t.runlen = yb * (uint32_t)L.LZ;
-    t.bpr = (t.runlen + S - 1) / S;
-    t.bpb = bt * bx * t.bpr;
-    t.bpcol = (uint32_t)L.T / bt * t.bpb;
-    const uint32_t ncol = t.ncx * ((uint32_t)L.LY / yb);
-    t.nblk = ncol * t.bpcol;
+    t.bpr = runs(t.runlen);
+    t.bpp = bx * t.bpr;
+    t.npair = t.ncx * ((uint32_t)L.LY / yb) * (uint32_t)L.T;
+    t.npx = (t.npair + kXcds - 1) / kXcds;
+    t.nblk = kXcds * t.npx * t.bpp;
     return t;
   }
   // (a brick request that does not tile the lattice falls back to mode 2)
@@ -1050,7 +1223,7 @@ static Traversal traversal(const cvchip_ctx *c, int N, bool eo = false, int K = 
     t.mode = 2;
     t.yb = yb;
     t.runlen = yb * (uint32_t)L.LZ;
-    t.bpr = (t.runlen + S - 1) / S;
+    t.bpr = runs(t.runlen);
     t.nrun = (uint32_t)(L.LY / (int)yb) * (uint32_t)L.LX;
     t.nblk = (uint32_t)L.T * t.nrun * t.bpr;
     return t;
@@ -1059,9 +1232,67 @@ static Traversal traversal(const cvchip_ctx *c, int N, bool eo = false, int K = 
   else if (V % kXcds == 0) { t.csz = V / kXcds; t.mode = 1; }
   else { t.csz = V; t.mode = 0; }
   if (want == 3) t.mode = 0;
-  t.bpc = (t.csz + S - 1) / S;
+  t.bpc = runs(t.csz);
   t.nblk = (V / t.csz) * t.bpc;
   return t;
+}
+
+// planned once per context, policy, rhs count and precision (a launch on a small
+// lattice is shorter than the plan)
+static const Traversal &traversal(const cvchip_ctx *c, int N, bool eo, int K) {
+  const uint64_t key = ((uint64_t)c->dslash_policy << 16) | ((uint64_t)N << 4) | ((uint64_t)eo << 3) | (uint64_t)K;
+  const auto it = c->plans.find(key);
+  if (it != c->plans.end()) return it->second;
+  return c->plans.emplace(key, plan_traversal(c, N, eo, K)).first->second;
+}
+
+template <typename R>
+static void set_traversal(DParams<R> &P, const Traversal &tr, uint32_t LZt) {
+  P.LZt = LZt;
+  P.invS = 1.0f / (float)(tr.threads / (unsigned)P.N);   // sites per block
+  P.csz = tr.csz;
+  P.bpc = tr.bpc;
+  P.mode = tr.mode;
+  P.yb = tr.yb;
+  P.runlen = tr.runlen;
+  P.bpr = tr.bpr;
+  P.nrun = tr.nrun;
+  P.bx = tr.bx;
+  P.ncx = tr.ncx;
+  P.bpp = tr.bpp;
+  P.npx = tr.npx;
+  P.npair = tr.npair;
+  P.bpcol = tr.bpcol;
+  P.zb = tr.zb;
+  P.ncy = tr.ncy;
+  P.ncz = tr.ncz;
+  P.lzb = tr.lzb;
+  P.lyz = tr.lyz;
+  P.lA = tr.lA;
+  P.colsz = tr.colsz;
+  P.sXt = (uint32_t)P.LY * LZt;
+  P.sTt = (uint32_t)P.LX * P.sXt;
+  P.mS = tr.mS;
+  P.mM = tr.mM;
+  P.mXP = tr.mXP;
+  P.mYP = tr.mYP;
+  P.mCP = tr.mCP;
+  P.mNR = tr.mNR;
+  P.mNPX = tr.mNPX;
+  P.mXcd = tr.mXcd;
+  auto div = [](uint32_t d) { return make_fdiv(d ? d : 1); };   // 0: a quotient of another mode
+  P.fLZt = div(LZt);
+  P.fLY = div((uint32_t)P.LY);
+  P.fLX = div((uint32_t)P.LX);
+  P.fbpc = div(tr.bpc);
+  P.fbpcol = div(tr.bpcol);
+  P.fT = div((uint32_t)P.T);
+  P.fbpp = div(tr.bpp);
+  P.fbpr = div(tr.bpr);
+  P.fncx = div(tr.ncx);
+  P.fslice = div(tr.nrun * tr.bpr);
+  P.fncy = div(tr.ncy);
+  P.fncz = div(tr.ncz);
 }
 
 unsigned dslash_blocks(const cvchip_ctx *c, int N) {
@@ -1092,48 +1323,13 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
   const int N = in.nrhs;
   DParams<R> P = make_params<R>(c, N, mutm);
   P.partner = (dm == DOT_TS && r2 != nullptr) ? 1 : 0;
-  P.LZt = EO ? (uint32_t)c->lat.LZ / 2 : (uint32_t)c->lat.LZ;
-  P.shLZt = log2_exact(P.LZt);
   P.par = eo ? eo->par : 0;
   P.dmode = eo ? eo->dmode : 0;
   P.hopc = (R)(eo ? eo->hopc : -0.5);
   P.dinv = (R)(1.0 / (0.25 / (c->kappa * c->kappa) + mutm * mutm));
-  const int B = block_for(N);
-  {
-    const int S = B / N, KLs = RECON == 18 ? 9 : 6;   // sites per block, link entries per hop
-    P.invS = 1.0f / (float)S;
-    P.invKS = 1.0f / (float)(KLs * S);
-  }
-  const Traversal tr = traversal(c, N, EO, IOI::K);
-  P.csz = tr.csz;
-  P.bpc = tr.bpc;
-  P.mode = tr.mode;
-  P.yb = tr.yb;
-  P.runlen = tr.runlen;
-  P.bpr = tr.bpr;
-  P.nrun = tr.nrun;
-  P.bt = tr.bt;
-  P.bx = tr.bx;
-  P.ncx = tr.ncx;
-  P.bpb = tr.bpb;
-  P.bpcol = tr.bpcol;
-  P.zb = tr.zb;
-  P.ncy = tr.ncy;
-  P.ncz = tr.ncz;
-  P.lzb = tr.lzb;
-  P.lyz = tr.lyz;
-  P.lA = tr.lA;
-  P.colsz = tr.colsz;
-  P.sXt = (uint32_t)c->lat.LY * P.LZt;
-  P.sTt = (uint32_t)c->lat.LX * P.sXt;
-  P.mS = tr.mS;
-  P.mM = tr.mM;
-  P.mXP = tr.mXP;
-  P.mYP = tr.mYP;
-  P.mCP = tr.mCP;
-  P.mNR = tr.mNR;
-  P.mNPX = tr.mNPX;
-  P.mXcd = tr.mXcd;
+  const Traversal &tr = traversal(c, N, EO, IOI::K);
+  set_traversal(P, tr, EO ? (uint32_t)c->lat.LZ / 2 : (uint32_t)c->lat.LZ);
+  const int B = (int)tr.threads;
   P.done = c->op_mask;
   P.dstride = c->op_mask_stride;
   // streaming stores only for outputs that cannot stay in the 256 MB MALL
