@@ -540,6 +540,9 @@ extern "C" int cvchip_ctx_destroy(cvchip_ctx *c) {
       if (c->pin[k]) (void)hipHostFree(c->pin[k]);
       if (c->pin_ev[k]) (void)hipEventDestroy(c->pin_ev[k]);
     }
+    if (c->solve_bufs.st) (void)hipFree(c->solve_bufs.st);
+    if (c->solve_bufs.res) (void)hipFree(c->solve_bufs.res);
+    if (c->solve_bufs.hst) (void)hipHostFree(c->solve_bufs.hst);
     if (c->red.ptr) (void)hipFree(c->red.ptr);
     if (c->red2.ptr) (void)hipFree(c->red2.ptr);
     if (c->ev0) (void)hipEventDestroy(c->ev0);

@@ -126,6 +126,13 @@ struct Traversal {
   unsigned threads;   // workgroup size
 };
 
+// A solve's per-rhs state on the device and its pinned host side (solver.hip),
+// kept by the context between solves
+struct SolveBuffers {
+  void *st = nullptr, *res = nullptr, *hst = nullptr;
+  bool in_use = false;
+};
+
 struct Scratch {
   void *ptr = nullptr;
   size_t bytes = 0;
@@ -160,6 +167,7 @@ struct cvchip_ctx {
   int op_mask_stride = 0;
   // iterations of each right-hand side of the last solve (0: an exact start vector)
   std::vector<int> col_iters;
+  cvchip::SolveBuffers solve_bufs;
   // traversals already planned, by policy, rhs count, lattice half and precision
   mutable std::map<uint64_t, cvchip::Traversal> plans;
   // staging for host <-> device transfers (AoS reference layout)
@@ -249,6 +257,17 @@ inline int block_for(int nrhs) {
   int s = 256 / nrhs;
   if (s < 1) s = 1;
   return s * nrhs;
+}
+
+// ... and smaller blocks, down to one wave, where the V x nrhs pairs would not
+// make kFillBlocks blocks: with 16 blocks of 256 threads (8^4, one rhs) 240 of the
+// 256 compute units idle while each of the 16 serves four waves' loads in turn
+// (the solver's x/p update 5.7 -> 4.2 us, its r update 6.0 -> 4.4 us there).
+constexpr int64_t kFillBlocks = 512;
+inline int launch_block(int64_t V, int nrhs) {
+  const int full = block_for(nrhs) / nrhs, wave = 64 / nrhs > 0 ? 64 / nrhs : 1;
+  const int64_t fill = V / kFillBlocks;
+  return (int)(fill >= full ? full : fill > wave ? fill : wave < full ? wave : full) * nrhs;
 }
 
 }  // namespace cvchip

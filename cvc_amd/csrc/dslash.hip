@@ -1076,12 +1076,12 @@ static bool march_geometry(const cvchip_ctx *c, int N, Traversal &t, bool explic
 }
 
 
-// Sites per operator block for runs of len sites: at most what fits 256
-// threads, the count that pads the run least, and among equals the largest whose
+// Sites per operator block for runs of len of a lattice's V sites: at most
+// launch_block's, the count that pads the run least, and among equals the largest whose
 // S N is a multiple of 8, so that a block's stores begin and end on 128-byte
 // lines (a line shared by two blocks is written twice, in halves).
-static uint32_t op_sites(int N, uint32_t len) {
-  const uint32_t S0 = (uint32_t)(block_for(N) / N);
+static uint32_t op_sites(int N, uint32_t len, int64_t V) {
+  const uint32_t S0 = (uint32_t)(launch_block(V, N) / N);
   if (N < 8) return S0;   // links from memory: blocks of 256 threads win although their last one is padded more
   auto cost = [&](uint32_t S) {   // padded sites, and the halved lines as sites
     const uint64_t nb = (len + S - 1) / S;
@@ -1112,7 +1112,7 @@ static void best_columns(const Lattice &L, int N, int K, uint32_t &bx, uint32_t 
     if (L.LX % cx) continue;
     for (int cy = 1; cy <= L.LY; cy++) {
       if (L.LY % cy) continue;
-      const uint32_t len = (uint32_t)(cy * L.LZ), S = op_sites(N, len);
+      const uint32_t len = (uint32_t)(cy * L.LZ), S = op_sites(N, len, L.V);
       const double pad = (double)((len + S - 1) / S * S) / len;
       const double npair = (double)(L.LX / cx) * (L.LY / cy) * L.T, npx = ceil(npair / kXcds);
       const double halo = (cx < L.LX ? 2. / cx : 0.) + (cy < L.LY ? 2. / cy : 0.);
@@ -1175,7 +1175,7 @@ static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
   uint32_t S = 1;
   // blocks of S sites over runs of len sites
   auto runs = [&](uint32_t len) {
-    S = op_sites(N, len);
+    S = op_sites(N, len, L.V);
     t.threads = S * (unsigned)N;
     return (len + S - 1) / S;
   };
@@ -1378,7 +1378,7 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
     if (nblk_out) *nblk_out = (int)nblk;
     return 0;
   }
-  const bool multi = B / N <= LDS_SITES;
+  const bool multi = block_for(N) / N <= LDS_SITES;
   const bool ldsl = multi && (c->dslash_policy & 1);
   const bool ldss = !EO && multi && (c->dslash_policy & 2) && tr.mode != 5;
   // bits 24-27: extra LDS per block in 8 KiB units (caps the blocks per CU)

@@ -42,6 +42,16 @@ struct RhsState {
   int done, final_upd, iter, upd, last_upd;
   int stall;          // mixed: own reliable updates in a row that did not halve best
   int stalled;        // mixed: stopped at the floor of the true residual, not converged
+  int hold;           // operator applications skip this rhs: done, or (between its own
+                      // reliable-update trigger and that update) p2 is still needed
+};
+
+// What the host needs of a rhs after each iteration, written by the scalar
+// kernel straight into pinned host memory; seq last, so that a host that sees
+// the iteration's seq sees the rest.
+struct RhsMirror {
+  double norm, normb;
+  int done, final_upd, upd, seq;
 };
 
 // ------------------------------------------------------------ vector kernels
@@ -282,6 +292,7 @@ __global__ void k_sc_init(RhsState *st, const double *res, int N, double sp, int
   S.last_upd = 0;
   S.iter = -1;
   S.done = (S.norm <= S.tol2) ? 1 : 0;       // invert_Qtm.c:142-147: return 0
+  S.hold = S.done;
   if (S.done) S.iter = 0;
   S.alpha[0] = S.alpha[1] = S.omega[0] = S.omega[1] = S.beta[0] = S.beta[1] = 0.;
   (void)mixed;
@@ -356,10 +367,10 @@ __global__ void __launch_bounds__(kScThreads) k_sc_alpha(RhsState *st, const dou
   if (threadIdx.x) return;
   RhsState &S = st[r];
   if (S.final_upd) {
-    S.done = 1;
+    S.done = S.hold = 1;
     S.final_upd = 0;
   }
-  if (S.done) return;
+  if (S.hold) return;
   cdiv(S.alpha, S.r0rn, w);
 }
 
@@ -391,19 +402,15 @@ __global__ void __launch_bounds__(kScThreads) k_sc_omega_her(RhsState *st, const
 }
 
 // after r1: convergence test (or reliable-update trigger), beta, r0rn
-__global__ void __launch_bounds__(kScThreads) k_sc_beta(RhsState *st, const double *__restrict__ part, int n, int N,
-                                                        int it, int lagged, int mixed, double delta2) {
-  const int r = blockIdx.x;
-  double res[3];
-  sum_rows<3>(part + (size_t)r * n, (size_t)N * n, n, res);
-  RhsState &S = st[r];
-  if (threadIdx.x || S.done) return;
+__device__ __forceinline__ void beta_step(RhsState &S, const double res[3], int it, int lagged, int mixed,
+                                          double delta2) {
+  if (S.done) return;
   S.norm = res[0];
   const double w[2] = {res[1], res[2]};
   if (!mixed) {
     if (S.norm <= S.tol2) {
       S.iter = it;
-      if (lagged) S.done = 1;
+      if (lagged) S.done = S.hold = 1;
       else S.final_upd = 1;
       if (S.done) return;
     }
@@ -414,6 +421,7 @@ __global__ void __launch_bounds__(kScThreads) k_sc_beta(RhsState *st, const doub
     // (the tolerance trigger waits for a factor 10 margin in |r|: the iterated
     // low-precision residual runs slightly ahead of the true one)
     S.upd = (S.norm <= delta2 * S.rmax || S.norm <= 0.01 * S.tol2 || it - S.last_upd >= kMaxGap) ? 1 : 0;
+    S.hold = S.upd;
   }
   double w2[2], w3[2];
   cdiv(w2, w, S.r0rn);
@@ -424,6 +432,23 @@ __global__ void __launch_bounds__(kScThreads) k_sc_beta(RhsState *st, const doub
   S.r0rn_prev[1] = S.r0rn[1];
   S.r0rn[0] = w[0];
   S.r0rn[1] = w[1];
+}
+
+__global__ void __launch_bounds__(kScThreads) k_sc_beta(RhsState *st, RhsMirror *host, const double *__restrict__ part,
+                                                        int n, int N, int it, int lagged, int mixed, double delta2) {
+  const int r = blockIdx.x;
+  double res[3];
+  sum_rows<3>(part + (size_t)r * n, (size_t)N * n, n, res);
+  if (threadIdx.x) return;
+  RhsState &S = st[r];
+  beta_step(S, res, it, lagged, mixed, delta2);
+  RhsMirror &m = host[r];
+  m.norm = S.norm;
+  m.normb = S.normb;
+  m.done = S.done;
+  m.final_upd = S.final_upd;
+  m.upd = S.upd;
+  __hip_atomic_store(&m.seq, it + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // A column whose own reliable-update trigger fired kMaxStall times in a row
@@ -444,7 +469,7 @@ __global__ void k_sc_reliable(RhsState *st, const double *res, int N, int it) {
   S.rmax = S.norm;
   S.last_upd = it;
   if (S.norm <= S.tol2) {
-    S.done = 1;
+    S.done = S.hold = 1;
     S.iter = it;
     return;
   }
@@ -452,7 +477,7 @@ __global__ void k_sc_reliable(RhsState *st, const double *res, int N, int it) {
     S.best = S.norm;
     S.stall = 0;
   } else if (S.upd == 1 && ++S.stall >= kMaxStall) {
-    S.done = 1;
+    S.done = S.hold = 1;
     S.stalled = 1;
     S.iter = it;
   }
@@ -506,7 +531,9 @@ __global__ void k_sc_restart(RhsState *st, int N) {
 // replaced).
 __global__ void k_sc_upd_all(RhsState *st, int N) {
   const int r = threadIdx.x;
-  if (r < N && !st[r].done && !st[r].upd) st[r].upd = 2;
+  if (r >= N || st[r].done) return;
+  if (!st[r].upd) st[r].upd = 2;
+  st[r].hold = 0;
 }
 
 __global__ void k_sc_clear_upd(RhsState *st, int N) {
@@ -544,7 +571,10 @@ struct Solve {
   unsigned nblk;
   RhsState *st = nullptr;     // device
   double *res = nullptr;      // device [4][N]
-  RhsState *hst = nullptr;    // pinned host mirror
+  RhsState *hst = nullptr;    // pinned host copy
+  RhsMirror *mir = nullptr;   // pinned, written by the device each iteration
+  bool kept = false;          // st .. mir are the context's kept buffers
+  int ahead = 0;              // the next iteration's first operator is enqueued before this one's test
   int nt = 0;                 // streaming stores in the vector kernels
 };
 
@@ -554,7 +584,7 @@ struct Solve {
 struct OpMask {
   cvchip_ctx *c;
   OpMask(cvchip_ctx *cc, const RhsState *st) : c(cc) {
-    c->op_mask = &st->done;
+    c->op_mask = &st->hold;
     c->op_mask_stride = (int)(sizeof(RhsState) / sizeof(int));
   }
   void clear() {
@@ -569,7 +599,7 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   S.c = c;
   S.N = N;
   S.VN = (uint32_t)((V > 0 ? V : c->lat.V) * N);
-  S.B = block_for(N);
+  S.B = launch_block(V > 0 ? V : c->lat.V, N);
   S.nblk = (S.VN + S.B - 1) / S.B;
   // an FP64 set of this size is 192 B per site and rhs
   S.nt = (size_t)S.VN * 192 >= ((size_t)256 << 20) ? 1 : 0;
@@ -577,14 +607,46 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   const size_t nb_max = std::max<size_t>(S.nblk, dslash_blocks(c, N));
   // (two launches' norms side by side in Op::apply_omega)
   CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 4 * N + 64 * 256)));
-  CVC_HIP(hipMalloc(&S.st, sizeof(RhsState) * N));
-  CVC_HIP(hipMalloc(&S.res, sizeof(double) * 4 * N));
-  CVC_HIP(hipHostMalloc(&S.hst, sizeof(RhsState) * N, hipHostMallocDefault));
+  // The small buffers are made once per context, for the largest N; a second
+  // solve running at the same time on the context gets its own.
+  constexpr int kMaxN = 256;
+  cvchip::SolveBuffers &B = c->solve_bufs;
+  S.kept = !B.in_use;
+  if (S.kept && !B.st) {
+    CVC_HIP(hipMalloc(&B.st, sizeof(RhsState) * kMaxN));
+    CVC_HIP(hipMalloc(&B.res, sizeof(double) * 4 * kMaxN));
+    CVC_HIP(hipHostMalloc(&B.hst, (sizeof(RhsState) + sizeof(RhsMirror)) * kMaxN, hipHostMallocCoherent | hipHostMallocMapped));
+  }
+  if (S.kept) {
+    B.in_use = true;
+    S.st = (RhsState *)B.st;
+    S.res = (double *)B.res;
+    S.hst = (RhsState *)B.hst;
+  } else {
+    CVC_HIP(hipMalloc(&S.st, sizeof(RhsState) * N));
+    CVC_HIP(hipMalloc(&S.res, sizeof(double) * 4 * N));
+    CVC_HIP(hipHostMalloc(&S.hst, (sizeof(RhsState) + sizeof(RhsMirror)) * kMaxN, hipHostMallocCoherent | hipHostMallocMapped));
+  }
+  S.mir = (RhsMirror *)(S.hst + kMaxN);
+  for (int r = 0; r < N; r++) S.mir[r].seq = 0;
+  // The next iteration's first operator goes out before the host has seen this
+  // iteration's residual while that operator is short: it hides the host's wait and
+  // launches (8^4, one rhs: 58 -> 41 us an iteration; the gradient at 8^4 65.3 ->
+  // 62.8 ms) and is done in vain once per solve, which at 32x16^3 with 12 rhs
+  // (0.9 ms) would cost what it saves.
+  S.ahead = (uint64_t)S.VN <= ((uint64_t)1 << 20);
   CVC_HIP(hipMemsetAsync(S.st, 0, sizeof(RhsState) * N, c->stream));
   return 0;
 }
 
 static void solve_free(Solve &S) {
+  if (S.kept) {
+    // nothing of this solve may still write to the buffers when the next takes them
+    (void)hipStreamSynchronize(S.c->stream);
+    S.c->solve_bufs.in_use = false;
+    S.kept = false;
+    return;
+  }
   if (S.st) (void)hipFree(S.st);
   if (S.res) (void)hipFree(S.res);
   if (S.hst) (void)hipHostFree(S.hst);
@@ -608,6 +670,25 @@ template <typename F> static int scalar_rows(Solve &S, int nblk, int Q, F f) {
 static int pull_state(Solve &S) {
   CVC_HIP(hipMemcpyAsync(S.hst, S.st, sizeof(RhsState) * S.N, hipMemcpyDeviceToHost, S.c->stream));
   CVC_HIP(hipStreamSynchronize(S.c->stream));
+  return 0;
+}
+
+// Waits until every rhs' state after iteration it is in the mirror: reads pinned
+// memory instead of draining the stream, so work enqueued behind it keeps running.
+static int wait_state(Solve &S, int it) {
+  for (int r = 0; r < S.N; r++) {
+    int spins = 0;
+    while (__atomic_load_n(&S.mir[r].seq, __ATOMIC_ACQUIRE) != it + 1) {
+      if (++spins % 4096) continue;
+      // a finished (or failed) stream writes no more
+      const hipError_t e = hipStreamQuery(S.c->stream);
+      if (e == hipErrorNotReady) continue;
+      if (e != hipSuccess) return hip_fail(e, "solver iteration", __FILE__, __LINE__);
+      if (__atomic_load_n(&S.mir[r].seq, __ATOMIC_ACQUIRE) == it + 1) break;
+      set_error("solver state of iteration %d missing after its kernels ended", it);
+      return CVCHIP_ERR_STATE;
+    }
+  }
   return 0;
 }
 
@@ -778,33 +859,39 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
   TRY(pull_state(S));
   all_done = 1;
   for (int r = 0; r < N; r++) all_done &= S.hst[r].done;
+  // p2 = A p and alpha
+  auto advance = [&]() -> int {
+    CVC_TRY(op.apply(p2, p, DOT_R2, &r2, &nb));
+    return scalar_rows(S, nb, 2, [&](const double *q, int n) {
+      hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
+    });
+  };
   if (!all_done) {
-    TRY(op.apply(p2, p, DOT_R2, &r2, &nb));
+    TRY(advance());
     dcalls++;
     for (int it = 0; it <= niter_max; it++) {
-      TRY(scalar_rows(S, nb, 2, [&](const double *q, int n) {
-        hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
-      }));
       hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt);
       TRY(op.apply_omega(t, s, c, N, S.st));
       dcalls++;
       hipLaunchKernelGGL((k_r1_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
                          S.VN, N, (double *)c->red.ptr, S.nt);
       TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
-        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N, it, lagged, 0, 0.0);
+        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, lagged, 0, 0.0);
       }));
       hipLaunchKernelGGL((k_xp_update<IO, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ix, ip, is, ir1, ip2,
                          S.st, S.VN, N, S.nt);
       CVC_HIP(hipGetLastError());
       iters = it + 1;
-      TRY(pull_state(S));
+      const bool ahead = S.ahead && it < niter_max;
+      if (ahead) TRY(advance());
+      TRY(wait_state(S, it));
       all_done = 1;
-      for (int r = 0; r < N; r++) all_done &= (S.hst[r].done | S.hst[r].final_upd);
+      for (int r = 0; r < N; r++) all_done &= (S.mir[r].done | S.mir[r].final_upd);
       if (verbose)
         for (int r = 0; r < N; r++)
-          printf("# [%d] residuum after iteration %d: %25.16e\n", r, it, S.hst[r].norm);
+          printf("# [%d] residuum after iteration %d: %25.16e\n", r, it, S.mir[r].norm);
       if (all_done) break;
-      TRY(op.apply(p2, p, DOT_R2, &r2, &nb));
+      if (!ahead) TRY(advance());
       dcalls++;
     }
   }
@@ -920,34 +1007,46 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
   TRY(pull_state(S));
   all_done = 1;
   for (int r = 0; r < N; r++) all_done &= S.hst[r].done;
+  // p2 = A p and alpha (of the rhs that do not hold their p2)
+  auto advance = [&]() -> int {
+    CVC_TRY(opl.apply(p2, p, DOT_R2, &r2, &nb));
+    return scalar_rows(S, nb, 2, [&](const double *q, int n) {
+      hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
+    });
+  };
   if (!all_done) {
-    TRY(opl.apply(p2, p, DOT_R2, &r2, &nb));
+    TRY(advance());
     dcalls++;
     for (int it = 0; it <= niter_max; it++) {
-      TRY(scalar_rows(S, nb, 2, [&](const double *q, int n) {
-        hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
-      }));
       hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt);
       TRY(opl.apply_omega(t, s, c, N, S.st));
       dcalls++;
       hipLaunchKernelGGL((k_r1_update<IO, IOR>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
                          S.VN, N, (double *)c->red.ptr, S.nt);
       TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
-        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N, it, 0, 1, delta2);
+        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, 0, 1, delta2);
       }));
       // xl += omega s + alpha p ; p = r1 + beta (p - omega p2)
       hipLaunchKernelGGL((k_xp_update<IOPlain<float>, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ixl, ip, is, ir1, ip2,
                          S.st, S.VN, N, S.nt);
       CVC_HIP(hipGetLastError());
       iters = it + 1;
-      TRY(pull_state(S));
+      // ahead of the test: a rhs whose own update was triggered holds its p2 and
+      // alpha, which that update needs; after an update this is done again
+      const bool ahead = S.ahead && it < niter_max;
+      if (ahead) TRY(advance());
+      TRY(wait_state(S, it));
       int any_upd = 0;
-      for (int r = 0; r < N; r++) any_upd |= (!S.hst[r].done && S.hst[r].upd);
+      all_done = 1;
+      for (int r = 0; r < N; r++) {
+        any_upd |= (!S.mir[r].done && S.mir[r].upd);
+        all_done &= S.mir[r].done;
+      }
       if (verbose && (any_upd || it % 16 == 0)) {
         double mx = 0.;
         for (int r = 0; r < N; r++) {
-          if (S.hst[r].done) continue;
-          const double q = S.hst[r].norm / S.hst[r].normb;
+          if (S.mir[r].done) continue;
+          const double q = S.mir[r].norm / S.mir[r].normb;
           if (!(q <= mx)) mx = q;   // a NaN propagates
         }
         printf("# [mixed] iteration %d: max iterated |r|^2/|b|^2 = %e\n", it, mx);
@@ -987,11 +1086,11 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
         }
         CVC_HIP(hipGetLastError());
         TRY(pull_state(S));
+        all_done = 1;
+        for (int r = 0; r < N; r++) all_done &= S.hst[r].done;
       }
-      all_done = 1;
-      for (int r = 0; r < N; r++) all_done &= S.hst[r].done;
       if (all_done) break;
-      TRY(opl.apply(p2, p, DOT_R2, &r2, &nb));
+      if (!ahead || any_upd) TRY(advance());
       dcalls++;
     }
   }
