@@ -48,7 +48,7 @@ constexpr size_t kPinMin = (size_t)16 << 20;
 static void par_memcpy(void *dst, const void *src, size_t bytes) {
   unsigned nt = std::thread::hardware_concurrency();
   nt = std::max(1u, std::min(8u, nt));
-  nt = (unsigned)std::min<size_t>(nt, std::max<size_t>(1, bytes / ((size_t)4 << 20)));
+  nt = (unsigned)std::min<size_t>(nt, std::max<size_t>(1, bytes / ((size_t)1 << 20)));
   const size_t per = (bytes + nt - 1) / nt;
   std::vector<std::thread> th;
   for (unsigned t = 1; t < nt; t++) {
@@ -96,6 +96,50 @@ int copy_to_host(cvchip_ctx *c, void *host, const void *dev, size_t bytes) {
     if (i + 2 < n) CVC_TRY(issue(i + 2));   // this buffer is free again
   }
   return 0;
+}
+
+// A slot is a quarter of a pinned buffer; larger pieces take the plain copy.
+constexpr size_t kSlotBytes = kPinChunk / 4;
+
+int HostStream::push(void *host, const void *dev, size_t bytes) {
+  static_assert(kSlots == 8, "two pinned buffers of four slots");
+  if (bytes > kSlotBytes) {
+    CVC_TRY(finish());   // the plain copy uses the same pinned buffers
+    return copy_to_host(c_, host, dev, bytes);
+  }
+  if (!c_->copy_stream) {
+    CVC_TRY(ensure_pinned(c_));
+    CVC_HIP(hipEventCreateWithFlags(&c_->copy_after, hipEventDisableTiming));
+    for (auto &e : c_->slot_ev) CVC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    CVC_HIP(hipStreamCreateWithFlags(&c_->copy_stream, hipStreamNonBlocking));
+  }
+  if (head_ - tail_ == kSlots) CVC_TRY(drain());
+  const size_t k = head_ % kSlots;
+  CVC_HIP(hipEventRecord(c_->copy_after, c_->stream));
+  CVC_HIP(hipStreamWaitEvent(c_->copy_stream, c_->copy_after, 0));
+  CVC_HIP(hipMemcpyAsync((char *)c_->pin[k / 4] + (k % 4) * kSlotBytes, dev, bytes, hipMemcpyDeviceToHost,
+                         c_->copy_stream));
+  CVC_HIP(hipEventRecord(c_->slot_ev[k], c_->copy_stream));
+  piece_[k] = Piece{host, bytes};
+  head_++;
+  return 0;
+}
+
+int HostStream::drain() {
+  const size_t k = tail_ % kSlots;
+  tail_++;
+  CVC_HIP(hipEventSynchronize(c_->slot_ev[k]));
+  par_memcpy(piece_[k].host, (char *)c_->pin[k / 4] + (k % 4) * kSlotBytes, piece_[k].bytes);
+  return 0;
+}
+
+int HostStream::finish() {
+  int rc = 0;
+  while (tail_ < head_) {
+    const int r = drain();
+    if (r && !rc) rc = r;
+  }
+  return rc;
 }
 
 // Host-to-device copies of 16 MB and more: each chunk is copied into a pinned
@@ -536,6 +580,13 @@ extern "C" int cvchip_ctx_destroy(cvchip_ctx *c) {
     if (c->gauge64r12) (void)hipFree(c->gauge64r12);
     if (c->gauge32r12) (void)hipFree(c->gauge32r12);
     if (c->stage) (void)hipFree(c->stage);
+    if (c->copy_stream) {
+      (void)hipStreamSynchronize(c->copy_stream);
+      (void)hipStreamDestroy(c->copy_stream);
+    }
+    if (c->copy_after) (void)hipEventDestroy(c->copy_after);
+    for (auto &e : c->slot_ev)
+      if (e) (void)hipEventDestroy(e);
     for (int k = 0; k < 2; k++) {
       if (c->pin[k]) (void)hipHostFree(c->pin[k]);
       if (c->pin_ev[k]) (void)hipEventDestroy(c->pin_ev[k]);

@@ -176,6 +176,9 @@ struct cvchip_ctx {
   // pinned host buffers (used in turn) and their events for device-to-host copies
   void *pin[2] = {nullptr, nullptr};
   hipEvent_t pin_ev[2] = {nullptr, nullptr};
+  // HostStream: its stream, "kernels done" event and one event per slot
+  hipStream_t copy_stream = nullptr;
+  hipEvent_t copy_after = nullptr, slot_ev[8] = {};
   // reduction scratch
   cvchip::Scratch red;
   size_t red_off = 0;     // where the operator's next partials start in red (doubles)
@@ -196,6 +199,30 @@ int copy_to_host(cvchip_ctx *c, void *host, const void *dev, size_t bytes);
 // host -> device copy enqueued on the context's stream; the caller
 // synchronizes the stream before the host buffer may change
 int copy_to_device(cvchip_ctx *c, void *dev, const void *host, size_t bytes);
+// Device -> host copies of pieces as they are computed: push() enqueues the copy of
+// a piece into a pinned slot behind the work enqueued on the context's stream so
+// far, on a second stream, so that later kernels run beside it; the host copies
+// finished pieces to their place while it waits for slots.  finish() (and the
+// destructor, on a failed path) waits for everything.
+class HostStream {
+ public:
+  static constexpr size_t kMinTotal = (size_t)16 << 20;   // less goes by one plain copy (no pinned buffers)
+  explicit HostStream(cvchip_ctx *c) : c_(c) {}
+  ~HostStream() { (void)finish(); }
+  int push(void *host, const void *dev, size_t bytes);
+  int finish();
+
+ private:
+  struct Piece {
+    void *host;
+    size_t bytes;
+  };
+  static constexpr int kSlots = 8;
+  int drain();   // the oldest piece in flight to its place
+  cvchip_ctx *c_;
+  Piece piece_[kSlots];
+  size_t head_ = 0, tail_ = 0;   // pieces pushed and placed
+};
 // device address of the allocation-free two-point entry point's scratch on
 // `device` (the current device), taken once per device
 int twopoint_scratch_init(int device);
