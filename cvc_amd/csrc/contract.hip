@@ -97,11 +97,6 @@ __global__ void __launch_bounds__(240) k_psi(double2 *__restrict__ psi, const do
   for (int c = 0; c < 12; c++) psi[(size_t)c * VP + (size_t)x * 24u + j24] = p[c];
 }
 
-// u v for a unit code u known at compile time after unrolling
-__device__ __forceinline__ double2 times_unit(int u, double2 v) {
-  return u == 0 ? v : u == 1 ? make_double2(-v.x, -v.y) : u == 2 ? make_double2(-v.y, v.x) : make_double2(v.y, -v.x);
-}
-
 // Combined columns of one slab: [2 (D, U)][4 nu][12 comps][sites of ns slices][12 columns].
 struct Slab {
   double2 *p;

@@ -16,6 +16,10 @@ __device__ __forceinline__ double2 unit_val(int code) {
   return code == 0 ? make_double2(1, 0) : code == 1 ? make_double2(-1, 0)
          : code == 2 ? make_double2(0, 1) : make_double2(0, -1);
 }
+// u v for a unit code u known at compile time after unrolling
+__device__ __forceinline__ double2 times_unit(int u, double2 v) {
+  return u == 0 ? v : u == 1 ? make_double2(-v.x, -v.y) : u == 2 ? make_double2(-v.y, v.x) : make_double2(v.y, -v.x);
+}
 __device__ __forceinline__ int g5sign(int spin) { return spin < 2 ? 1 : -1; }
 
 // v = gamma5 (gamma_mu -+ 1) w  (sgn = -1: Gm, +1: Gp), for runtime mu
