@@ -78,7 +78,8 @@ struct DParams {
   // columns per patch, mNR = T / mM slice ranges; mXcd: patch p on XCD p mod 8.
   uint32_t mS, mM, mXP, mYP, mCP, mNR, mNPX;
   int mXcd;
-  int nt;   // streaming output stores
+  int nt;       // streaming output stores
+  int nt_own;   // even/odd: streaming loads of the own spinors
   // Even/odd operator (EO kernels): the traversal runs over the half lattice
   // (T, LX, LY, LZ/2); half-site h of parity par is the lexicographic site
   // with z = 2 (h mod LZ/2) + ((par + t + x + y) mod 2), i.e. lex = 2h or 2h+1.
@@ -228,6 +229,7 @@ template <typename IO> struct Raw;
 template <> struct Raw<IOPlain<double>> {
   double2 v[12];
   __device__ __forceinline__ void load(const IOPlain<double> &in, uint32_t idx) { in.load(v, idx); }
+  __device__ __forceinline__ void load_nt(const IOPlain<double> &in, uint32_t idx) { in.load_nt(v, idx); }
   __device__ __forceinline__ void full(double2 o[12]) const {
 #pragma unroll
     for (int c = 0; c < 12; c++) o[c] = v[c];
@@ -240,6 +242,7 @@ template <> struct Raw<IOPlain<double>> {
 template <> struct Raw<IOPlain<float>> {
   float2 v[12];
   __device__ __forceinline__ void load(const IOPlain<float> &in, uint32_t idx) { in.load(v, idx); }
+  __device__ __forceinline__ void load_nt(const IOPlain<float> &in, uint32_t idx) { in.load_nt(v, idx); }
   __device__ __forceinline__ void full(float2 o[12]) const {
 #pragma unroll
     for (int c = 0; c < 12; c++) o[c] = v[c];
@@ -263,6 +266,19 @@ template <> struct Raw<IOHalf> {
       w[4 * k + 3] = v.w;
     }
     n = in.nrm[idx];
+  }
+  __device__ __forceinline__ void load_nt(const IOHalf &in, uint32_t idx) {
+    typedef unsigned u4v __attribute__((ext_vector_type(4)));
+    const u4v *q = reinterpret_cast<const u4v *>(in.p);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const u4v v = __builtin_nontemporal_load(q + (size_t)k * in.VN + idx);
+      w[4 * k] = v.x;
+      w[4 * k + 1] = v.y;
+      w[4 * k + 2] = v.z;
+      w[4 * k + 3] = v.w;
+    }
+    n = __builtin_nontemporal_load(in.nrm + idx);
   }
   __device__ __forceinline__ void full(float2 o[12]) const {
 #pragma unroll
@@ -413,7 +429,10 @@ __device__ __forceinline__ void hop_pipelined(cplx<typename IO::real> acc[12], R
   Raw<IO> next;
   if constexpr (H < 7) next.load(in, neighbour<H + 1, EO>(q, P) * (uint32_t)P.N + r);
   else if constexpr (!EO) next.load(in, q.v * (uint32_t)P.N + r);
-  else if (P.dmode != 1) next.load(own, q.v * (uint32_t)P.N + r);
+  else if (P.dmode != 1) {
+    if (P.nt_own) next.load_nt(own, q.v * (uint32_t)P.N + r);
+    else next.load(own, q.v * (uint32_t)P.N + r);
+  }
   asm volatile("" : : : "memory");
   const R n = raw.template project<(H >> 1), (H & 1) != 0>(h, one);
   hop_links<IO, RECON, H, true, EO>(acc, h, n, nullptr, Ul, P, q, sl);
@@ -1332,9 +1351,15 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
   const int B = (int)tr.threads;
   P.done = c->op_mask;
   P.dstride = c->op_mask_stride;
-  // streaming stores only for outputs that cannot stay in the 256 MB MALL
-  // (bit 3: for every output)
-  P.nt = (((c->dslash_policy >> 2) & 1) && out.bytes >= ((size_t)256 << 20)) || ((c->dslash_policy >> 3) & 1);
+  // Streaming stores only for outputs that would not stay in the 256 MB MALL
+  // beside the other fields (bit 3: for every output), and streaming loads for
+  // own spinors, which the even/odd forms read once, that do not stay in the caches
+  // anyway: both leave the L2 to the neighbours.  Per iteration (FP32 28x18x14x20,
+  // FP16 40x20^3, FP32 24x14x14x16 with 48 rhs): 908 / 1460 / 1881 us with stores
+  // from 256 MB and cached loads, 875 / 1410 / 1775 us with these; stores from 64
+  // MB 890 / 1409 / 1780; own loads of 40 MB sets slow the operator by 10 %.
+  P.nt = (((c->dslash_policy >> 2) & 1) && out.bytes >= ((size_t)128 << 20)) || ((c->dslash_policy >> 3) & 1);
+  P.nt_own = eo && eo->own && eo->own->bytes >= ((size_t)64 << 20);
   const unsigned nblk = tr.nblk;
   double *part = nullptr;
   if (dm != DOT_NONE) {

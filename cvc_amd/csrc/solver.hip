@@ -57,13 +57,23 @@ struct RhsMirror {
 // ------------------------------------------------------------ vector kernels
 
 // Streaming (non-temporal) stores for the vector kernels' outputs when a
-// vector set is 256 MB or more: it does not stay in the caches between kernels
-// anyway, and the stores then leave them to the inputs (measured at 64x32^3,
-// 12 rhs: FP64 solve 4.01 -> 3.67 s)
+// vector set of FP64 size is 128 MB or more: it does not stay in the caches between
+// kernels anyway, and the stores then leave them to the inputs (64x32^3, 12 rhs:
+// FP64 solve 4.01 -> 3.67 s; threshold 256 MB: 908 -> 897 us an iteration at
+// 28x18x14x20 with FP32 inside), and streaming loads of the fields that no later
+// kernel of the iteration reads (860 -> 838 us there, 1410 -> 1385 us at 40x20^3 with
+// FP16 inside)
 template <typename IO>
 __device__ __forceinline__ void vstore(const IO &io, const typename IO::C v[12], uint32_t i, int nt) {
   if (nt) io.store_nt(v, i);
   else io.store(v, i);
+}
+
+// and streaming loads of the fields whose values are not needed again
+template <typename IO>
+__device__ __forceinline__ void vload(const IO &io, typename IO::C v[12], uint32_t i, int nt) {
+  if (nt) io.load_nt(v, i);
+  else io.load(v, i);
 }
 
 template <typename IO> static IO mkio(const Field &f);
@@ -112,8 +122,8 @@ __global__ void __launch_bounds__(256) k_r1_update(IO r1, IO s, IO t, IOR r2, co
     const C w = mk<R>((R)st[rhs].omega[0], (R)st[rhs].omega[1]);
     C vs[12], vt[12], v2[12];
     s.load(vs, i);
-    t.load(vt, i);
-    r2.load(v2, i);
+    vload(t, vt, i, nt);
+    vload(r2, v2, i, nt);
     // products in FP64: squares of a small-scale rhs underflow FP32
     double n = 0, a = 0, b = 0;
 #pragma unroll
@@ -151,8 +161,8 @@ __global__ void __launch_bounds__(256) k_xp_update(IOX x, IO p, IO s, IO r1, IO 
   C vp[12], vs[12], vr[12], v2[12];
   CX vx[12];
   p.load(vp, i);
-  s.load(vs, i);
-  x.load(vx, i);
+  vload(s, vs, i, nt);
+  vload(x, vx, i, nt);
   // FP16 fields are a quarter of the FP64 bytes per lane: the loads of all
   // five fields go out together (the FP16-inner kernel 1140 -> 1047 us at
   // 32^3x64 even/odd; the FP32 one was 2 % slower, the FP64 one would halve
@@ -160,7 +170,7 @@ __global__ void __launch_bounds__(256) k_xp_update(IOX x, IO p, IO s, IO r1, IO 
   constexpr bool kAll = IO::K == 4;
   if (kAll && upp) {
     r1.load(vr, i);
-    p2.load(v2, i);
+    vload(p2, v2, i, nt);
   }
 #pragma unroll
   for (int c = 0; c < 12; c++) {
@@ -173,7 +183,7 @@ __global__ void __launch_bounds__(256) k_xp_update(IOX x, IO p, IO s, IO r1, IO 
     const C be = mk<R>((R)S.beta[0], (R)S.beta[1]);
     if (!kAll) {
       r1.load(vr, i);
-      p2.load(v2, i);
+      vload(p2, v2, i, nt);
     }
 #pragma unroll
     for (int c = 0; c < 12; c++) vp[c] = cadd(vr[c], cmul(be, csub(vp[c], cmul(w, v2[c]))));
@@ -602,7 +612,7 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   S.B = launch_block(V > 0 ? V : c->lat.V, N);
   S.nblk = (S.VN + S.B - 1) / S.B;
   // an FP64 set of this size is 192 B per site and rhs
-  S.nt = (size_t)S.VN * 192 >= ((size_t)256 << 20) ? 1 : 0;
+  S.nt = (size_t)S.VN * 192 >= ((size_t)128 << 20) ? 1 : 0;
   // room for the operator's partials too (its traversal has its own block count)
   const size_t nb_max = std::max<size_t>(S.nblk, dslash_blocks(c, N));
   // (two launches' norms side by side in Op::apply_omega)
