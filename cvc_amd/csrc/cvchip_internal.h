@@ -261,9 +261,15 @@ int gamma5_inplace(cvchip_ctx *c, Field &f);
 
 // Dslash launcher: out = D(mutm) in (gamma5_out: out = gamma5 D in).
 // Optional fused reductions, written as per-block partials into c->red:
-//   DOT_NONE, DOT_TS (<out,in> complex and <out,out>; <out,r2> when r2 is given),
-//   DOT_R2 (<r2,out> complex), DOT_NN (<out,out>)
-enum DotMode { DOT_NONE = 0, DOT_TS = 1, DOT_R2 = 2, DOT_NN = 3 };
+//   DOT_NONE, DOT_TS (<out,own> complex and <out,out>),
+//   DOT_R2 (<r2,out> complex), DOT_NN (<out,out>),
+//   DOT_TSR (<out,own> complex, <out,out>, <r2,out> complex), DOT_NNR (<out,out>, <r2,out> complex)
+// with own the spinor of the site in the operator's diagonal term.  gamma5 on the
+// output goes with NONE, R2, NN and NNR, none with NONE, R2, TS and TSR; TSR and
+// NNR are for FP64 fields.
+enum DotMode { DOT_NONE = 0, DOT_TS = 1, DOT_R2 = 2, DOT_NN = 3, DOT_TSR = 4, DOT_NNR = 5 };
+constexpr bool dot_shadow(int dm) { return dm == DOT_R2 || dm == DOT_TSR || dm == DOT_NNR; }   // r2 is the shadow residual
+constexpr int dot_rows(int dm) { return dm == DOT_TSR ? 5 : dm == DOT_TS || dm == DOT_NNR ? 3 : dm == DOT_R2 ? 2 : dm == DOT_NN ? 1 : 0; }
 int dslash(cvchip_ctx *c, Field &out, const Field &in, double mutm, int gamma5_out,
            DotMode dm = DOT_NONE, const Field *r2 = nullptr, int *nblocks_out = nullptr);
 

@@ -48,7 +48,6 @@ struct DParams {
   FDiv fLZt, fLY, fLX, fT, fbpc, fbpcol, fbpp, fbpr, fncx, fslice, fncy, fncz;
   // 1/N and 1/S for the small quotients of thread and staging indices
   float invN, invS;
-  int partner;   // DOT_TS: dot with the separate field r2 instead of the input
   // traversal (mode 1): the lattice is cut into chunks of csz consecutive
   // sites (one eighth of a time slice when possible), bpc blocks per chunk;
   // the 8 XCDs take the 8 chunks of a time slice side by side, so the whole
@@ -466,6 +465,33 @@ template <typename R> struct DslashWaves {
   static constexpr int value = sizeof(R) == 8 ? CVC_DSLASH_WAVES64 : CVC_DSLASH_WAVES32;
 };
 
+// A thread's terms of the fused dot products (DotMode): o the output, q the own
+// spinor, w the shadow residual; products in FP64: squares of a small-scale rhs
+// underflow FP32
+template <int DM, typename C>
+__device__ __forceinline__ void add_dots(double *dv, const C o[12], const C q[12], const C w[12]) {
+  double a = 0, b = 0, n = 0, ra = 0, rb = 0;
+#pragma unroll
+  for (int c = 0; c < 12; c++) {
+    const double ox = o[c].x, oy = o[c].y;
+    if constexpr (DM == DOT_TS || DM == DOT_TSR) {
+      const double qx = q[c].x, qy = q[c].y;
+      a += ox * qx + oy * qy;
+      b += ox * qy - oy * qx;
+    }
+    if constexpr (DM != DOT_R2) n += ox * ox + oy * oy;
+    if constexpr (dot_shadow(DM)) {
+      const double wx = w[c].x, wy = w[c].y;
+      ra += wx * ox + wy * oy;
+      rb += wx * oy - wy * ox;
+    }
+  }
+  int k = 0;
+  if constexpr (DM == DOT_TS || DM == DOT_TSR) { dv[k++] += a; dv[k++] += b; }
+  if constexpr (DM == DOT_TS || DM == DOT_TSR || DM == DOT_NN || DM == DOT_NNR) dv[k++] += n;
+  if constexpr (dot_shadow(DM)) { dv[k++] += ra; dv[k++] += rb; }
+}
+
 // LDSL: the block's sites share their links through LDS (N >= 8, at most
 // LDS_SITES sites per block): every link entry crosses the texture path once
 // per block instead of once per rhs lane.
@@ -562,7 +588,7 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
   const uint32_t r = threadIdx.x - sl * (uint32_t)P.N;
   SitePos q;
   const bool active = slot_pos(sl, q) && !(P.done && P.done[(size_t)r * P.dstride]);
-  double dv[3] = {0., 0., 0.};
+  double dv[dot_rows(DM) > 0 ? dot_rows(DM) : 1] = {};
   // FP32 / FP16 with 2-row links: the staged links are whole (third row rebuilt)
   // and carry the boundary phase, both done once per site here instead of once
   // per rhs lane in every hop (the multi-rhs kernels in these precisions are
@@ -649,7 +675,7 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
     // the shadow residual of the <r2, out> epilogue is read once per launch:
     // streaming loads, issued beside the own spinor's (the latencies overlap)
     C w2[12];
-    if constexpr (DM == DOT_R2) r2.load_nt(w2, i);
+    if constexpr (dot_shadow(DM)) r2.load_nt(w2, i);
     C own[12];
     if constexpr (!EO) {
       if constexpr (PIPE) raw.full(own);
@@ -694,38 +720,9 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
     }
     if (P.nt) out.store_nt(acc, i);
     else out.store(acc, i);
-    if constexpr (DM == DOT_TS) {
-      // <out, in> = sum conj(out) in ; <out, out>   (or <out, r2> when a partner is given)
-      if (P.partner) r2.load(own, i);
-      // products in FP64: squares of a small-scale rhs underflow FP32
-      double a = 0, b = 0, n = 0;
-#pragma unroll
-      for (int c = 0; c < 12; c++) {
-        const double ox = acc[c].x, oy = acc[c].y, qx = own[c].x, qy = own[c].y;
-        a += ox * qx + oy * qy;
-        b += ox * qy - oy * qx;
-        n += ox * ox + oy * oy;
-      }
-      dv[0] = a; dv[1] = b; dv[2] = n;
-    } else if constexpr (DM == DOT_R2) {
-      double a = 0, b = 0;
-#pragma unroll
-      for (int c = 0; c < 12; c++) {
-        const double ox = acc[c].x, oy = acc[c].y, qx = w2[c].x, qy = w2[c].y;
-        a += qx * ox + qy * oy;
-        b += qx * oy - qy * ox;
-      }
-      dv[0] = a; dv[1] = b;
-    } else if constexpr (DM == DOT_NN) {
-      double n = 0;
-#pragma unroll
-      for (int c = 0; c < 12; c++) n += (double)acc[c].x * acc[c].x + (double)acc[c].y * acc[c].y;
-      dv[0] = n;
-    }
+    add_dots<DM>(dv, acc, own, w2);
   }
-  if constexpr (DM == DOT_TS) block_reduce_store<3>(dv, part, P.N);
-  else if constexpr (DM == DOT_R2) block_reduce_store<2>(dv, part, P.N);
-  else if constexpr (DM == DOT_NN) block_reduce_store<1>(dv, part, P.N);
+  if constexpr (DM != DOT_NONE) block_reduce_store<dot_rows(DM)>(dv, part, P.N);
 }
 
 // ------------------------------------------------------- t-marching operator
@@ -877,7 +874,7 @@ k_dslash_march(IOO out, IOI in, const cplx<typename IOI::real> *__restrict__ U, 
   R one = (R)1;   // opaque to the compiler (see project_half)
   if constexpr (IsHalf<IOI>::value) asm volatile("" : "+v"(one));
   const NbLoader<IOI, false> ld{in, nullptr, (uint32_t)P.N, r, 0, 0, one};
-  double dv[3] = {0., 0., 0.};
+  double dv[dot_rows(DM) > 0 ? dot_rows(DM) : 1] = {};
 
   // carry: (U_0^dagger (1 + gamma_0) phi)(t - 1) as the six complex numbers w
   C carry[2][3];
@@ -924,7 +921,7 @@ k_dslash_march(IOO out, IOI in, const cplx<typename IOI::real> *__restrict__ U, 
     // the shadow residual of the <r2, out> epilogue is read once per launch:
     // streaming loads, issued with the own spinor's
     C w2[12];
-    if constexpr (DM == DOT_R2) r2.load_nt(w2, i);
+    if constexpr (dot_shadow(DM)) r2.load_nt(w2, i);
     C acc[12];
     {
       C own[12];
@@ -987,38 +984,11 @@ k_dslash_march(IOO out, IOI in, const cplx<typename IOI::real> *__restrict__ U, 
     }
     if (P.nt) out.store_nt(acc, i);
     else out.store(acc, i);
-    if constexpr (DM == DOT_TS) {
-      C own[12];
-      if (P.partner) r2.load(own, i);
-      else in.load(own, i);
-      double a = 0, b = 0, n = 0;
-#pragma unroll
-      for (int c = 0; c < 12; c++) {
-        const double ox = acc[c].x, oy = acc[c].y, qx = own[c].x, qy = own[c].y;
-        a += ox * qx + oy * qy;
-        b += ox * qy - oy * qx;
-        n += ox * ox + oy * oy;
-      }
-      dv[0] += a; dv[1] += b; dv[2] += n;
-    } else if constexpr (DM == DOT_R2) {
-      double a = 0, b = 0;
-#pragma unroll
-      for (int c = 0; c < 12; c++) {
-        const double ox = acc[c].x, oy = acc[c].y, qx = w2[c].x, qy = w2[c].y;
-        a += qx * ox + qy * oy;
-        b += qx * oy - qy * ox;
-      }
-      dv[0] += a; dv[1] += b;
-    } else if constexpr (DM == DOT_NN) {
-      double n = 0;
-#pragma unroll
-      for (int c = 0; c < 12; c++) n += (double)acc[c].x * acc[c].x + (double)acc[c].y * acc[c].y;
-      dv[0] += n;
-    }
+    C own[12];
+    if constexpr (DM == DOT_TS || DM == DOT_TSR) in.load(own, i);
+    add_dots<DM>(dv, acc, own, w2);
   }
-  if constexpr (DM == DOT_TS) block_reduce_store<3>(dv, part, P.N);
-  else if constexpr (DM == DOT_R2) block_reduce_store<2>(dv, part, P.N);
-  else if constexpr (DM == DOT_NN) block_reduce_store<1>(dv, part, P.N);
+  if constexpr (DM != DOT_NONE) block_reduce_store<dot_rows(DM)>(dv, part, P.N);
 }
 
 // ------------------------------------------------------------- launcher
@@ -1334,14 +1304,19 @@ template <typename IOI, typename IOO, int RECON, bool EO, typename IOR = IOI>
 static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g5, DotMode dm,
                   const Field *r2, int *nblk_out, const EOArgs *eo = nullptr) {
   constexpr bool kSameR = std::is_same<IOR, IOI>::value;
+  constexpr bool k64 = sizeof(typename IOI::real) == 8;
   if (!kSameR && (dm != DOT_R2 || !r2)) {
     set_error("operator: a shadow residual of another precision serves only the <r2, out> epilogue");
+    return CVCHIP_ERR_ARG;
+  }
+  if ((dot_shadow(dm) && !r2) || (g5 ? dm == DOT_TS || dm == DOT_TSR : dm == DOT_NN || dm == DOT_NNR) ||
+      (!k64 && (dm == DOT_TSR || dm == DOT_NNR))) {
+    set_error("operator: no such fused dot products (%d)", (int)dm);
     return CVCHIP_ERR_ARG;
   }
   using R = typename IOI::real;
   const int N = in.nrhs;
   DParams<R> P = make_params<R>(c, N, mutm);
-  P.partner = (dm == DOT_TS && r2 != nullptr) ? 1 : 0;
   P.par = eo ? eo->par : 0;
   P.dmode = eo ? eo->dmode : 0;
   P.hopc = (R)(eo ? eo->hopc : -0.5);
@@ -1363,7 +1338,7 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
   const unsigned nblk = tr.nblk;
   double *part = nullptr;
   if (dm != DOT_NONE) {
-    CVC_TRY(ensure_red(c, sizeof(double) * (c->red_off + (size_t)nblk * 3 * N + 64 * 256)));
+    CVC_TRY(ensure_red(c, sizeof(double) * (c->red_off + (size_t)nblk * dot_rows(dm) * N + 64 * 256)));
     part = (double *)c->red.ptr + c->red_off;
   }
   const cplx<R> *U;
@@ -1384,19 +1359,20 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
     dim3 bm(tr.threads);
 #define CVC_MLAUNCH(G5, DMV) \
     hipLaunchKernelGGL((k_dslash_march<IOI, IOO, RECON, G5, DMV, IOR>), g, bm, lds, c->stream, o, ii, U, P, rr, part)
-    if constexpr (!kSameR) {
-      if (g5) CVC_MLAUNCH(true, DOT_R2);
-      else CVC_MLAUNCH(false, DOT_R2);
-    } else if (g5) {
-      if (dm == DOT_NONE) CVC_MLAUNCH(true, DOT_NONE);
-      else if (dm == DOT_TS) CVC_MLAUNCH(true, DOT_TS);
-      else if (dm == DOT_NN) CVC_MLAUNCH(true, DOT_NN);
-      else CVC_MLAUNCH(true, DOT_R2);
+    if (g5) {
+      if (dm == DOT_R2) CVC_MLAUNCH(true, DOT_R2);
+      else if constexpr (kSameR) {
+        if (dm == DOT_NONE) CVC_MLAUNCH(true, DOT_NONE);
+        else if (dm == DOT_NN) CVC_MLAUNCH(true, DOT_NN);
+        else if constexpr (k64) CVC_MLAUNCH(true, DOT_NNR);
+      }
     } else {
-      if (dm == DOT_NONE) CVC_MLAUNCH(false, DOT_NONE);
-      else if (dm == DOT_TS) CVC_MLAUNCH(false, DOT_TS);
-      else if (dm == DOT_NN) CVC_MLAUNCH(false, DOT_NN);
-      else CVC_MLAUNCH(false, DOT_R2);
+      if (dm == DOT_R2) CVC_MLAUNCH(false, DOT_R2);
+      else if constexpr (kSameR) {
+        if (dm == DOT_NONE) CVC_MLAUNCH(false, DOT_NONE);
+        else if (dm == DOT_TS) CVC_MLAUNCH(false, DOT_TS);
+        else if constexpr (k64) CVC_MLAUNCH(false, DOT_TSR);
+      }
     }
 #undef CVC_MLAUNCH
     CVC_HIP(hipGetLastError());
@@ -1421,19 +1397,20 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
       else hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, false, false, false, IOR>), g, b, dyn, c->stream, o, ii, ii, U, P, rr, part); \
     }                                                                                                           \
   } while (0)
-  if constexpr (!kSameR) {
-    if (g5) CVC_LAUNCH(true, DOT_R2);
-    else CVC_LAUNCH(false, DOT_R2);
-  } else if (g5) {
-    if (dm == DOT_NONE) CVC_LAUNCH(true, DOT_NONE);
-    else if (dm == DOT_TS) CVC_LAUNCH(true, DOT_TS);
-    else if (dm == DOT_NN) CVC_LAUNCH(true, DOT_NN);
-    else CVC_LAUNCH(true, DOT_R2);
+  if (g5) {
+    if (dm == DOT_R2) CVC_LAUNCH(true, DOT_R2);
+    else if constexpr (kSameR) {
+      if (dm == DOT_NONE) CVC_LAUNCH(true, DOT_NONE);
+      else if (dm == DOT_NN) CVC_LAUNCH(true, DOT_NN);
+      else if constexpr (k64) CVC_LAUNCH(true, DOT_NNR);
+    }
   } else {
-    if (dm == DOT_NONE) CVC_LAUNCH(false, DOT_NONE);
-    else if (dm == DOT_TS) CVC_LAUNCH(false, DOT_TS);
-    else if (dm == DOT_NN) CVC_LAUNCH(false, DOT_NN);
-    else CVC_LAUNCH(false, DOT_R2);
+    if (dm == DOT_R2) CVC_LAUNCH(false, DOT_R2);
+    else if constexpr (kSameR) {
+      if (dm == DOT_NONE) CVC_LAUNCH(false, DOT_NONE);
+      else if (dm == DOT_TS) CVC_LAUNCH(false, DOT_TS);
+      else if constexpr (k64) CVC_LAUNCH(false, DOT_TSR);
+    }
   }
 #undef CVC_LAUNCH
   CVC_HIP(hipGetLastError());
@@ -1575,11 +1552,11 @@ int reduce_stage1(cvchip_ctx *c, const double *part, int nblk, int rows, int slo
     *n = nblk;
     return 0;
   }
-  // both halves at the size of a full set of rows, so that neither call grows
-  // the scratch under the other's result
-  const size_t half = (size_t)3 * 256 * kSegMax;
-  CVC_TRY(ensure_red2(c, sizeof(double) * 2 * half));
-  double *seg = (double *)c->red2.ptr + slot * half;
+  // every slot at the size of a full set of rows, so that no call grows the
+  // scratch under another's result
+  const size_t room = (size_t)5 * 256 * kSegMax;
+  CVC_TRY(ensure_red2(c, sizeof(double) * 3 * room));
+  double *seg = (double *)c->red2.ptr + slot * room;
   hipLaunchKernelGGL(k_reduce_seg, dim3(rows * G), dim3(256), 0, c->stream, part, nblk, G, seg);
   CVC_HIP(hipGetLastError());
   *out = seg;

@@ -9,6 +9,8 @@
 //   r1    = s - omega t,  <r1,r1>, <r2,r1>      (vector kernel with dots)
 //   test  |r1|^2 <= sp |b|^2; beta = (<r2,r1>/r0rn)(alpha/omega); r0rn = <r2,r1>
 //   x    += omega s + alpha p ;  p = r1 + beta (p - omega p2)   (one pass)
+// or, in FP64 and not lagged, the three in one pass: <r2,r1> = <r2,s> - omega <r2,t>,
+// summed where s and t are made, and the test follows the pass
 //   p2    = D p,  <r2,p2>                       (operator with fused dot epilogue)
 // Dot products are per-thread sums of a site's 12 components, block trees per
 // rhs and a fixed-order tree over blocks: results are reproducible run to run.
@@ -39,7 +41,7 @@ struct RhsState {
   double rmax;        // mixed: |r|^2 at the last reliable update
   double true_res2;
   double best;        // mixed: the smallest true |r|^2 at a reliable update so far
-  int done, final_upd, iter, upd, last_upd;
+  int done, iter, upd, last_upd;
   int stall;          // mixed: own reliable updates in a row that did not halve best
   int stalled;        // mixed: stopped at the floor of the true residual, not converged
   int hold;           // operator applications skip this rhs: done, or (between its own
@@ -51,7 +53,7 @@ struct RhsState {
 // the iteration's seq sees the rest.
 struct RhsMirror {
   double norm, normb;
-  int done, final_upd, upd, seq;
+  int done, upd, seq;
 };
 
 // ------------------------------------------------------------ vector kernels
@@ -93,21 +95,35 @@ template <> IOHalf mkio<IOHalf>(const Field &f) {
   const bool act = i < VN;                                     \
   (void)rhs;
 
-// s = r1 - alpha p2
-template <typename IO>
+// s = r1 - alpha p2; SHADOW: partial dots <r2,s>
+template <typename IO, int SHADOW = 0>
 __global__ void __launch_bounds__(256) k_s_update(IO s, IO r1, IO p2, const RhsState *__restrict__ st,
-                                                  uint32_t VN, int N, int nt) {
+                                                  uint32_t VN, int N, int nt, IO r2, double *__restrict__ part) {
   CVC_ELEMWISE_PROLOGUE
-  if (!act || st[rhs].done) return;
+  if constexpr (!SHADOW) {
+    if (!act || st[rhs].done) return;
+  }
   using R = typename IO::real;
   using C = cplx<R>;
-  const C a = mk<R>((R)st[rhs].alpha[0], (R)st[rhs].alpha[1]);
-  C vr[12], vp[12];
-  r1.load(vr, i);
-  p2.load(vp, i);
+  double dv[2] = {0., 0.};
+  if (!SHADOW || (act && !st[rhs].done)) {
+    const C a = mk<R>((R)st[rhs].alpha[0], (R)st[rhs].alpha[1]);
+    C vr[12], vp[12];
+    r1.load(vr, i);
+    p2.load(vp, i);
 #pragma unroll
-  for (int c = 0; c < 12; c++) vr[c] = csub(vr[c], cmul(a, vp[c]));
-  vstore(s, vr, i, nt);
+    for (int c = 0; c < 12; c++) vr[c] = csub(vr[c], cmul(a, vp[c]));
+    vstore(s, vr, i, nt);
+    if constexpr (SHADOW) {
+      vload(r2, vp, i, nt);
+#pragma unroll
+      for (int c = 0; c < 12; c++) {
+        dv[0] += vp[c].x * vr[c].x + vp[c].y * vr[c].y;
+        dv[1] += vp[c].x * vr[c].y - vp[c].y * vr[c].x;
+      }
+    }
+  }
+  if constexpr (SHADOW) block_reduce_store<2>(dv, part, N);
 }
 
 // r1 = s - omega t ; partial dots <r1,r1>, <r2,r1>  (r2 stored as IOR)
@@ -141,17 +157,16 @@ __global__ void __launch_bounds__(256) k_r1_update(IO r1, IO s, IO t, IOR r2, co
   block_reduce_store<3>(dv, part, N);
 }
 
-// x += omega s + alpha p  (while running, or once more on convergence when
-// not lagged); p = r1 + beta (p - omega p2) (while running)
+// x += omega s + alpha p; p = r1 + beta (p - omega p2) unless a reliable update
+// replaces r1 first
 template <typename IOX, typename IO>
 __global__ void __launch_bounds__(256) k_xp_update(IOX x, IO p, IO s, IO r1, IO p2,
                                                    const RhsState *__restrict__ st, uint32_t VN, int N, int nt) {
   CVC_ELEMWISE_PROLOGUE
   if (!act) return;
   const RhsState &S = st[rhs];
-  const bool upx = !S.done;               // includes the final (non-lagged) update
-  const bool upp = !S.done && !S.final_upd && !S.upd;
-  if (!upx) return;
+  if (S.done) return;
+  const bool upp = !S.upd;
   using R = typename IO::real;
   using C = cplx<R>;
   using RX = typename IOX::real;
@@ -189,6 +204,53 @@ __global__ void __launch_bounds__(256) k_xp_update(IOX x, IO p, IO s, IO r1, IO 
     for (int c = 0; c < 12; c++) vp[c] = cadd(vr[c], cmul(be, csub(vp[c], cmul(w, v2[c]))));
     vstore(p, vp, i, nt);
   }
+}
+
+// The end of an FP64 iteration in one pass, once omega and beta are known:
+//   r1 = s - omega t, <r1,r1>;  x += omega s + alpha p;  p = r1 + beta (p - omega p2)
+// Bound by memory: five fields in, three out, against four plus seven passes of the
+// two kernels above (r1 is not read back, s not read twice), for two more reads of r2
+// (in k_s_update and in the operator's epilogue): 1745 -> 1680 us an iteration at
+// 32x16^3 with 12 rhs, no change at 8^4.  Components are independent in FP64
+// storage; four at a time keep 20 loads in flight per lane.
+template <int NT>
+__global__ void __launch_bounds__(256) k_step(IOPlain<double> r1, IOPlain<double> x, IOPlain<double> p,
+                                              IOPlain<double> s, IOPlain<double> t, IOPlain<double> p2,
+                                              const RhsState *__restrict__ st, uint32_t VN, int N,
+                                              double *__restrict__ part) {
+  CVC_ELEMWISE_PROLOGUE
+  double dv[1] = {0.};
+  if (act && !st[rhs].done) {
+    const RhsState &S = st[rhs];
+    const double2 a = make_double2(S.alpha[0], S.alpha[1]), w = make_double2(S.omega[0], S.omega[1]),
+                  be = make_double2(S.beta[0], S.beta[1]);
+    auto in = [&](const IOPlain<double> &f, int c) { return NT ? f.load_c_nt(c, i) : f.load_c(c, i); };
+    auto out = [&](const IOPlain<double> &f, int c, double2 v) {
+      if constexpr (NT) f.store_c_nt(c, v, i);
+      else f.store_c(c, v, i);
+    };
+#pragma unroll 1
+    for (int g = 0; g < 12; g += 4) {
+      double2 vs[4], vt[4], vx[4], vp[4], v2[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        vs[k] = in(s, g + k);
+        vt[k] = in(t, g + k);
+        vx[k] = in(x, g + k);
+        vp[k] = p.load_c(g + k, i);
+        v2[k] = in(p2, g + k);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const double2 r = csub(vs[k], cmul(w, vt[k]));
+        dv[0] += r.x * r.x + r.y * r.y;
+        out(r1, g + k, r);
+        out(x, g + k, cadd(vx[k], cadd(cmul(w, vs[k]), cmul(a, vp[k]))));
+        out(p, g + k, cadd(r, cmul(be, csub(vp[k], cmul(w, v2[k])))));
+      }
+    }
+  }
+  block_reduce_store<1>(dv, part, N);
 }
 
 // r = b - t  (t = D x), optionally copied to r2 (stored as IOR) and p; partial dots <r,r>, <b,b>
@@ -297,7 +359,6 @@ __global__ void k_sc_init(RhsState *st, const double *res, int N, double sp, int
   S.best = S.norm;
   S.stall = 0;
   S.stalled = 0;
-  S.final_upd = 0;
   S.upd = 0;
   S.last_upd = 0;
   S.iter = -1;
@@ -376,53 +437,79 @@ __global__ void __launch_bounds__(kScThreads) k_sc_alpha(RhsState *st, const dou
   sum_rows<2>(part + (size_t)r * n, (size_t)N * n, n, w);
   if (threadIdx.x) return;
   RhsState &S = st[r];
-  if (S.final_upd) {
-    S.done = S.hold = 1;
-    S.final_upd = 0;
-  }
   if (S.hold) return;
   cdiv(S.alpha, S.r0rn, w);
 }
 
-// omega = <t,s>/<t,t> from one launch's three rows
-__global__ void __launch_bounds__(kScThreads) k_sc_omega(RhsState *st, const double *__restrict__ part, int n, int N) {
+// beta = (<r2,r1>/r0rn)(alpha/omega) and r0rn = <r2,r1> before r1 is formed, from
+// <r2,r1> = <r2,s> - omega <r2,t> (rs, rt).  <r2,s> would be zero but for
+// rounding; taken as zero, r0rn drifts and solves to 1e-26 |b|^2 do not converge.
+__device__ __forceinline__ void beta_from_t(RhsState &S, const double rs[2], const double rt[2]) {
+  const double w[2] = {rs[0] - (S.omega[0] * rt[0] - S.omega[1] * rt[1]),
+                       rs[1] - (S.omega[0] * rt[1] + S.omega[1] * rt[0])};
+  double w2[2], w3[2];
+  cdiv(w2, w, S.r0rn);
+  cdiv(w3, S.alpha, S.omega);
+  S.beta[0] = w2[0] * w3[0] - w2[1] * w3[1];
+  S.beta[1] = w2[0] * w3[1] + w2[1] * w3[0];
+  S.r0rn[0] = w[0];
+  S.r0rn[1] = w[1];
+}
+
+// omega = <t,s>/<t,t> from one launch's three rows; SHADOW: two more rows hold
+// <r2,t>, rs the partials of <r2,s>, and beta follows
+template <int SHADOW>
+__global__ void __launch_bounds__(kScThreads) k_sc_omega(RhsState *st, const double *__restrict__ part, int n, int N,
+                                                         const double *__restrict__ rs, int nrs) {
   const int r = blockIdx.x;
-  double w[3];
-  sum_rows<3>(part + (size_t)r * n, (size_t)N * n, n, w);
+  double v[2];
+  if constexpr (SHADOW) {
+    sum_rows<2>(rs + (size_t)r * nrs, (size_t)N * nrs, nrs, v);
+    __syncthreads();
+  }
+  double w[SHADOW ? 5 : 3];
+  sum_rows<SHADOW ? 5 : 3>(part + (size_t)r * n, (size_t)N * n, n, w);
   RhsState &S = st[r];
   if (threadIdx.x || S.done) return;
   const double inv = 1. / w[2];
   S.omega[0] = w[0] * inv;
   S.omega[1] = w[1] * inv;
+  if constexpr (SHADOW) beta_from_t(S, v, w + 3);
 }
 
 // the same from the norms of the two halves of the gamma5-hermitian operator:
-// <t,s> = |B s|^2 (partials ts, real) and <t,t> (partials tt)
+// <t,s> = |B s|^2 (partials ts, real) and <t,t> (partials tt; SHADOW: with <r2,t>)
+template <int SHADOW>
 __global__ void __launch_bounds__(kScThreads) k_sc_omega_her(RhsState *st, const double *__restrict__ ts, int nts,
-                                                             const double *__restrict__ tt, int ntt) {
+                                                             const double *__restrict__ tt, int ntt, int N,
+                                                             const double *__restrict__ rs, int nrs) {
   const int r = blockIdx.x;
-  double a[1], b[1];
+  double a[1], b[SHADOW ? 3 : 1], v[2];
+  if constexpr (SHADOW) {
+    sum_rows<2>(rs + (size_t)r * nrs, (size_t)N * nrs, nrs, v);
+    __syncthreads();
+  }
   sum_rows<1>(ts + (size_t)r * nts, 0, nts, a);
   __syncthreads();
-  sum_rows<1>(tt + (size_t)r * ntt, 0, ntt, b);
+  sum_rows<SHADOW ? 3 : 1>(tt + (size_t)r * ntt, (size_t)N * ntt, ntt, b);
   RhsState &S = st[r];
   if (threadIdx.x || S.done) return;
   S.omega[0] = a[0] * (1. / b[0]);
   S.omega[1] = 0.;
+  if constexpr (SHADOW) beta_from_t(S, v, b + 1);
 }
 
-// after r1: convergence test (or reliable-update trigger), beta, r0rn
-__device__ __forceinline__ void beta_step(RhsState &S, const double res[3], int it, int lagged, int mixed,
-                                          double delta2) {
+// after r1: convergence test (lagged FP64: before x moves) or reliable-update
+// trigger (mixed), beta, r0rn
+__device__ __forceinline__ void beta_step(RhsState &S, const double res[3], int it, int mixed, double delta2) {
   if (S.done) return;
   S.norm = res[0];
   const double w[2] = {res[1], res[2]};
   if (!mixed) {
     if (S.norm <= S.tol2) {
       S.iter = it;
-      if (lagged) S.done = S.hold = 1;
-      else S.final_upd = 1;
-      if (S.done) return;
+      S.done = S.hold = 1;
+      return;
     }
   } else {
     // reliable update when the iterated residual fell by delta since the last
@@ -444,21 +531,42 @@ __device__ __forceinline__ void beta_step(RhsState &S, const double res[3], int 
   S.r0rn[1] = w[1];
 }
 
+// release order: a host that sees the iteration's seq sees the rest
+__device__ __forceinline__ void mirror_state(RhsMirror &m, const RhsState &S, int it) {
+  m.norm = S.norm;
+  m.normb = S.normb;
+  m.done = S.done;
+  m.upd = S.upd;
+  __hip_atomic_store(&m.seq, it + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// after k_step: |r1|^2 and the convergence test
+__global__ void __launch_bounds__(kScThreads) k_sc_test(RhsState *st, RhsMirror *host, const double *__restrict__ part,
+                                                        int n, int it) {
+  const int r = blockIdx.x;
+  double res[1];
+  sum_rows<1>(part + (size_t)r * n, 0, n, res);
+  if (threadIdx.x) return;
+  RhsState &S = st[r];
+  if (!S.done) {
+    S.norm = res[0];
+    if (S.norm <= S.tol2) {
+      S.iter = it;
+      S.done = S.hold = 1;
+    }
+  }
+  mirror_state(host[r], S, it);
+}
+
 __global__ void __launch_bounds__(kScThreads) k_sc_beta(RhsState *st, RhsMirror *host, const double *__restrict__ part,
-                                                        int n, int N, int it, int lagged, int mixed, double delta2) {
+                                                        int n, int N, int it, int mixed, double delta2) {
   const int r = blockIdx.x;
   double res[3];
   sum_rows<3>(part + (size_t)r * n, (size_t)N * n, n, res);
   if (threadIdx.x) return;
   RhsState &S = st[r];
-  beta_step(S, res, it, lagged, mixed, delta2);
-  RhsMirror &m = host[r];
-  m.norm = S.norm;
-  m.normb = S.normb;
-  m.done = S.done;
-  m.final_upd = S.final_upd;
-  m.upd = S.upd;
-  __hip_atomic_store(&m.seq, it + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  beta_step(S, res, it, mixed, delta2);
+  mirror_state(host[r], S, it);
 }
 
 // A column whose own reliable-update trigger fired kMaxStall times in a row
@@ -616,7 +724,7 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   // room for the operator's partials too (its traversal has its own block count)
   const size_t nb_max = std::max<size_t>(S.nblk, dslash_blocks(c, N));
   // (two launches' norms side by side in Op::apply_omega)
-  CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 4 * N + 64 * 256)));
+  CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 7 * N + 64 * 256)));
   // The small buffers are made once per context, for the largest N; a second
   // solve running at the same time on the context gets its own.
   constexpr int kMaxN = 256;
@@ -741,41 +849,61 @@ struct Op {
   int eo = 0;
   Field *tmp = nullptr;   // even/odd: the even-parity intermediate
   // Schur complement on the odd sites, M = A_oo - D_oe A_ee^-1 D_eo
-  //   = A_oo - H_oe A_ee^-1 H_eo / 4  (gamma5 on the output when g5); the fused
-  // <out,in> of DOT_TS pairs the output with `partner` (default: in)
-  int applyM(Field &out, const Field &in, double mutm, int g5, DotMode dm, const Field *partner, int *nb) {
+  //   = A_oo - H_oe A_ee^-1 H_eo / 4  (gamma5 on the output when g5)
+  int applyM(Field &out, const Field &in, double mutm, int g5, DotMode dm, const Field *r2, int *nb) {
     CVC_TRY(dslash_eo(c, *tmp, in, nullptr, mutm, 0, 1, 0.5, 0));
-    return dslash_eo(c, out, *tmp, &in, mutm, 1, 0, -0.5, g5, dm,
-                     dm == DOT_TS ? (partner ? partner : &in) : partner, nb);
+    return dslash_eo(c, out, *tmp, &in, mutm, 1, 0, -0.5, g5, dm, r2, nb);
   }
   // t = A in and omega = <t,in> / <t,t> into the state.  For the
   // gamma5-hermitian operator A = B^dagger B with B = gamma5 D(-mu) (gamma5
   // M(-mu) on the even/odd system), so <t,in> = <B in, B in> is the norm of the
   // first application's output: both applications fuse a norm, and neither
   // reads the input again.  The second one's partials follow the first one's in
-  // the reduction scratch (solve_setup makes room for both).
-  int apply_omega(Field &out, const Field &in, cvchip_ctx *cc, int N, RhsState *st) {
+  // the reduction scratch (solve_setup makes room for both).  With r2 the same
+  // launches also sum <r2,t>, and beta goes into the state too; <r2,s> is then in
+  // the scratch's first 2 N rows of nrs partials.
+  int apply_omega(Field &out, const Field &in, cvchip_ctx *cc, int N, RhsState *st, const Field *r2 = nullptr,
+                  int nrs = 0) {
     int nb1 = 0, nb2 = 0;
-    const double *p1 = nullptr, *p2 = nullptr;
+    const double *p1 = nullptr, *p2 = nullptr, *rs = nullptr;
     int n1 = 0, n2 = 0;
+    const size_t off = r2 ? (size_t)2 * N * nrs : 0;
+    int rc;
+    c->red_off = off;
     if (!her) {
-      CVC_TRY(apply(out, in, DOT_TS, nullptr, &nb1));
-      CVC_TRY(reduce_stage1(cc, (const double *)cc->red.ptr, nb1, 3 * N, 0, &p1, &n1));
-      hipLaunchKernelGGL(k_sc_omega, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, N);
+      rc = apply(out, in, r2 ? DOT_TSR : DOT_TS, r2, &nb1);
+      c->red_off = 0;
+      CVC_TRY(rc);
+      const double *red = (const double *)cc->red.ptr;
+      CVC_TRY(reduce_stage1(cc, red + off, nb1, (r2 ? 5 : 3) * N, 0, &p1, &n1));
+      if (r2) {
+        CVC_TRY(reduce_stage1(cc, red, nrs, 2 * N, 1, &rs, &nrs));
+        hipLaunchKernelGGL(k_sc_omega<1>, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, N, rs, nrs);
+      } else {
+        hipLaunchKernelGGL(k_sc_omega<0>, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, N, rs, nrs);
+      }
       CVC_HIP(hipGetLastError());
       return 0;
     }
-    if (eo) CVC_TRY(applyM(*aux, in, -c->mu, 1, DOT_NN, nullptr, &nb1));
-    else CVC_TRY(dslash(c, *aux, in, -c->mu, 1, DOT_NN, nullptr, &nb1));
-    c->red_off = (size_t)nb1 * N;
-    int rc;
-    if (eo) rc = applyM(out, *aux, c->mu, 1, DOT_NN, nullptr, &nb2);
-    else rc = dslash(c, out, *aux, c->mu, 1, DOT_NN, nullptr, &nb2);
+    if (eo) rc = applyM(*aux, in, -c->mu, 1, DOT_NN, nullptr, &nb1);
+    else rc = dslash(c, *aux, in, -c->mu, 1, DOT_NN, nullptr, &nb1);
+    if (!rc) {
+      c->red_off = off + (size_t)nb1 * N;
+      const DotMode dm = r2 ? DOT_NNR : DOT_NN;
+      if (eo) rc = applyM(out, *aux, c->mu, 1, dm, r2, &nb2);
+      else rc = dslash(c, out, *aux, c->mu, 1, dm, r2, &nb2);
+    }
     c->red_off = 0;
     CVC_TRY(rc);
-    CVC_TRY(reduce_stage1(cc, (const double *)cc->red.ptr, nb1, N, 0, &p1, &n1));
-    CVC_TRY(reduce_stage1(cc, (const double *)cc->red.ptr + (size_t)nb1 * N, nb2, N, 1, &p2, &n2));
-    hipLaunchKernelGGL(k_sc_omega_her, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, p2, n2);
+    const double *red = (const double *)cc->red.ptr;
+    CVC_TRY(reduce_stage1(cc, red + off, nb1, N, 0, &p1, &n1));
+    CVC_TRY(reduce_stage1(cc, red + off + (size_t)nb1 * N, nb2, (r2 ? 3 : 1) * N, 1, &p2, &n2));
+    if (r2) {
+      CVC_TRY(reduce_stage1(cc, red, nrs, 2 * N, 2, &rs, &nrs));
+      hipLaunchKernelGGL(k_sc_omega_her<1>, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, p2, n2, N, rs, nrs);
+    } else {
+      hipLaunchKernelGGL(k_sc_omega_her<0>, dim3(N), dim3(kScThreads), 0, cc->stream, st, p1, n1, p2, n2, N, rs, nrs);
+    }
     CVC_HIP(hipGetLastError());
     return 0;
   }
@@ -783,12 +911,11 @@ struct Op {
     if (eo) {
       if (!her) return applyM(out, in, c->mu, 0, dm, r2, nb);
       CVC_TRY(applyM(*aux, in, -c->mu, 1, DOT_NONE, nullptr, nullptr));
-      return applyM(out, *aux, c->mu, 1, dm, dm == DOT_TS ? &in : r2, nb);
+      return applyM(out, *aux, c->mu, 1, dm, r2, nb);
     }
     if (!her) return dslash(c, out, in, c->mu, 0, dm, r2, nb);
     CVC_TRY(dslash(c, *aux, in, -c->mu, 1));
-    // the fused <t,s> must pair the output with the operator's input, not with aux
-    return dslash(c, out, *aux, c->mu, 1, dm, dm == DOT_TS ? &in : r2, nb);
+    return dslash(c, out, *aux, c->mu, 1, dm, r2, nb);
   }
 };
 
@@ -817,7 +944,7 @@ static void record_iterations(Solve &S, int iters) {
   S.c->col_iters.resize(S.N);
   for (int r = 0; r < S.N; r++) {
     const RhsState &h = S.hst[r];
-    S.c->col_iters[r] = iters == 0 ? 0 : (h.done || h.final_upd) ? h.iter + 1 : iters;
+    S.c->col_iters[r] = iters == 0 ? 0 : h.done ? h.iter + 1 : iters;
   }
 }
 
@@ -880,23 +1007,41 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
     TRY(advance());
     dcalls++;
     for (int it = 0; it <= niter_max; it++) {
-      hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt);
-      TRY(op.apply_omega(t, s, c, N, S.st));
+      // a lagged solve needs |r1|^2 before x moves, so it keeps the separate passes
+      if (lagged)
+        hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt,
+                           ir2, nullptr);
+      else
+        hipLaunchKernelGGL((k_s_update<IO, 1>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N,
+                           S.nt, ir2, (double *)c->red.ptr);
+      TRY(op.apply_omega(t, s, c, N, S.st, lagged ? nullptr : &r2, (int)S.nblk));
       dcalls++;
-      hipLaunchKernelGGL((k_r1_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
-                         S.VN, N, (double *)c->red.ptr, S.nt);
-      TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
-        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, lagged, 0, 0.0);
-      }));
-      hipLaunchKernelGGL((k_xp_update<IO, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ix, ip, is, ir1, ip2,
-                         S.st, S.VN, N, S.nt);
-      CVC_HIP(hipGetLastError());
+      if (!lagged) {
+        if (S.nt)
+          hipLaunchKernelGGL(k_step<1>, dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, ix, ip, is, iT, ip2, S.st, S.VN, N,
+                             (double *)c->red.ptr);
+        else
+          hipLaunchKernelGGL(k_step<0>, dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, ix, ip, is, iT, ip2, S.st, S.VN, N,
+                             (double *)c->red.ptr);
+        TRY(scalar_rows(S, (int)S.nblk, 1, [&](const double *q, int n) {
+          hipLaunchKernelGGL(k_sc_test, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, it);
+        }));
+      } else {
+        hipLaunchKernelGGL((k_r1_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
+                           S.VN, N, (double *)c->red.ptr, S.nt);
+        TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
+          hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, 0, 0.0);
+        }));
+        hipLaunchKernelGGL((k_xp_update<IO, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ix, ip, is, ir1, ip2,
+                           S.st, S.VN, N, S.nt);
+        CVC_HIP(hipGetLastError());
+      }
       iters = it + 1;
       const bool ahead = S.ahead && it < niter_max;
       if (ahead) TRY(advance());
       TRY(wait_state(S, it));
       all_done = 1;
-      for (int r = 0; r < N; r++) all_done &= (S.mir[r].done | S.mir[r].final_upd);
+      for (int r = 0; r < N; r++) all_done &= S.mir[r].done;
       if (verbose)
         for (int r = 0; r < N; r++)
           printf("# [%d] residuum after iteration %d: %25.16e\n", r, it, S.mir[r].norm);
@@ -905,12 +1050,11 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
       dcalls++;
     }
   }
-  // final state (final_upd counts as converged)
   TRY(pull_state(S));
   record_iterations(S, iters);
   int nconv = 0, maxit = 0;
   for (int r = 0; r < N; r++) {
-    if (S.hst[r].done || S.hst[r].final_upd) {
+    if (S.hst[r].done) {
       nconv++;
       if (S.hst[r].iter > maxit) maxit = S.hst[r].iter;
     }
@@ -1028,13 +1172,14 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
     TRY(advance());
     dcalls++;
     for (int it = 0; it <= niter_max; it++) {
-      hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt);
+      hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt,
+                         ir1, nullptr);
       TRY(opl.apply_omega(t, s, c, N, S.st));
       dcalls++;
       hipLaunchKernelGGL((k_r1_update<IO, IOR>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
                          S.VN, N, (double *)c->red.ptr, S.nt);
       TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
-        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, 0, 1, delta2);
+        hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, 1, delta2);
       }));
       // xl += omega s + alpha p ; p = r1 + beta (p - omega p2)
       hipLaunchKernelGGL((k_xp_update<IOPlain<float>, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ixl, ip, is, ir1, ip2,

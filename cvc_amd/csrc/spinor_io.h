@@ -34,27 +34,29 @@ struct IOPlain<double> {
   }
   __device__ __forceinline__ C load_c(int c, uint32_t idx) const { return p[(size_t)c * VN + idx]; }
   // streaming load (no allocation in the caches): for a field read once per launch
-  __device__ __forceinline__ void load_nt(C v[12], uint32_t idx) const {
+  __device__ __forceinline__ C load_c_nt(int c, uint32_t idx) const {
     typedef double d2v __attribute__((ext_vector_type(2)));
-    const d2v *q = reinterpret_cast<const d2v *>(p);
-#pragma unroll
-    for (int c = 0; c < 12; c++) {
-      const d2v w = __builtin_nontemporal_load(q + (size_t)c * VN + idx);
-      v[c] = make_double2(w.x, w.y);
-    }
+    const d2v w = __builtin_nontemporal_load(reinterpret_cast<const d2v *>(p) + (size_t)c * VN + idx);
+    return make_double2(w.x, w.y);
   }
+  __device__ __forceinline__ void load_nt(C v[12], uint32_t idx) const {
+#pragma unroll
+    for (int c = 0; c < 12; c++) v[c] = load_c_nt(c, idx);
+  }
+  __device__ __forceinline__ void store_c(int c, C v, uint32_t idx) const { p[(size_t)c * VN + idx] = v; }
   __device__ __forceinline__ void store(const C v[12], uint32_t idx) const {
 #pragma unroll
     for (int c = 0; c < 12; c++) p[(size_t)c * VN + idx] = v[c];
   }
   // streaming store (no allocation in the caches)
-  __device__ __forceinline__ void store_nt(const C v[12], uint32_t idx) const {
+  __device__ __forceinline__ void store_c_nt(int c, C v, uint32_t idx) const {
     typedef double d2v __attribute__((ext_vector_type(2)));
+    const d2v w = {v.x, v.y};
+    __builtin_nontemporal_store(w, reinterpret_cast<d2v *>(p + (size_t)c * VN + idx));
+  }
+  __device__ __forceinline__ void store_nt(const C v[12], uint32_t idx) const {
 #pragma unroll
-    for (int c = 0; c < 12; c++) {
-      const d2v w = {v[c].x, v[c].y};
-      __builtin_nontemporal_store(w, reinterpret_cast<d2v *>(p + (size_t)c * VN + idx));
-    }
+    for (int c = 0; c < 12; c++) store_c_nt(c, v[c], idx);
   }
 };
 
