@@ -299,7 +299,8 @@ inline int block_for(int nrhs) {
 constexpr int64_t kFillBlocks = 512;
 inline int launch_block(int64_t V, int nrhs) {
   const int full = block_for(nrhs) / nrhs, wave = 64 / nrhs > 0 ? 64 / nrhs : 1;
-  const int64_t fill = V / kFillBlocks;
+  // (whole waves: 50 sites of 3 rhs would leave a third of a block's last wave idle)
+  const int64_t fill = (V / kFillBlocks * nrhs + 63) / 64 * 64 / nrhs;
   return (int)(fill >= full ? full : fill > wave ? fill : wave < full ? wave : full) * nrhs;
 }
 
