@@ -439,8 +439,15 @@ __device__ __forceinline__ void hop_pipelined(cplx<typename IO::real> acc[12], R
   raw = next;
 }
 
-// the same without LDS links or with staged spinors: load, project, multiply
-template <typename IO, int RECON, int H, bool LDSL, bool LDSS, bool EO>
+// the same without LDS links or with staged spinors: load, project, multiply.
+// Links from memory (N < 8): the compiler issues the loads of all hops that nothing
+// bounds at once.  One rhs gains by that (FEW: FP32 of one rhs unbounded, FP64 of
+// one and two bounded once, after four hops); more rhs re-read less and gain by a
+// second wave instead: FP32 bounded after three hops (48x24^3, 2 / 4 / 6 rhs: 136 /
+// 232 / 346 us against 142 / 243 / 363 us unbounded; one rhs 72 against 66 us), FP64
+// after three and six (48x24^3, 1 / 2 / 4 / 7 rhs: 185 / 265 / 444 / 752 us, after four
+// hops at one wave 166 / 262 / 473 / 892 us, unbounded 169 / 265 / 481 / 880 us).
+template <typename IO, int RECON, int H, bool LDSL, bool LDSS, bool EO, bool FEW>
 __device__ __forceinline__ void hop_plain(cplx<typename IO::real> acc[12], const NbLoader<IO, LDSS> &ld,
                                           const cplx<typename IO::real> *__restrict__ U,
                                           const cplx<typename IO::real> *__restrict__ Ul,
@@ -450,19 +457,22 @@ __device__ __forceinline__ void hop_plain(cplx<typename IO::real> acc[12], const
   const R n = ld.template proj<(H >> 1), (H & 1) != 0>(h, neighbour<H, EO>(q, P), (H >> 1) == 3);
   if constexpr (LDSL) pin_regs(&h[0][0], 6);
   hop_links<IO, RECON, H, LDSL, EO>(acc, h, n, U, Ul, P, q, sl);
-  if constexpr (LDSL) pin_regs(acc, 12);
+  constexpr bool bound = IO::K == 1 ? (FEW ? H == 3 : H == 2 || H == 5) : IO::K == 2 && !FEW && H == 2;
+  if constexpr (LDSL || bound) pin_regs(acc, 12);
 }
 
 // Minimum resident waves per SIMD the register allocation must allow (the
-// compiler otherwise hoists every neighbour load and ends at one wave).
+// compiler otherwise hoists every neighbour load and ends at one wave).  Links from
+// memory (few rhs) in FP32 and FP16: two, at three the FP32 kernel spills (48x24^3,
+// one / six rhs: 96 / 472 us against 66 / 346 us).
 #ifndef CVC_DSLASH_WAVES64
 #define CVC_DSLASH_WAVES64 1
 #endif
 #ifndef CVC_DSLASH_WAVES32
 #define CVC_DSLASH_WAVES32 3
 #endif
-template <typename R> struct DslashWaves {
-  static constexpr int value = sizeof(R) == 8 ? CVC_DSLASH_WAVES64 : CVC_DSLASH_WAVES32;
+template <typename R, bool LDSL, bool FEW> struct DslashWaves {
+  static constexpr int value = sizeof(R) == 8 ? (LDSL || FEW ? CVC_DSLASH_WAVES64 : 2) : LDSL ? CVC_DSLASH_WAVES32 : 2;
 };
 
 // A thread's terms of the fused dot products (DotMode): o the output, q the own
@@ -497,8 +507,10 @@ __device__ __forceinline__ void add_dots(double *dv, const C o[12], const C q[12
 // per block instead of once per rhs lane.
 // IOR: the storage of r2, the shadow residual of the <r2, out> epilogue (the
 // FP32 mixed solver keeps it in FP16 with a per-site scale)
-template <typename IOI, typename IOO, int RECON, bool G5OUT, int DM, bool LDSL, bool LDSS, bool EO, typename IOR = IOI>
-__global__ void __launch_bounds__(256, DslashWaves<typename IOI::real>::value)
+// FEW: one or two rhs (see hop_plain)
+template <typename IOI, typename IOO, int RECON, bool G5OUT, int DM, bool LDSL, bool LDSS, bool EO, typename IOR = IOI,
+          bool FEW = false>
+__global__ void __launch_bounds__(256, (DslashWaves<typename IOI::real, LDSL, FEW>::value))
 k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict__ U,
          DParams<typename IOI::real> P, IOR r2, double *__restrict__ part) {
   using R = typename IOI::real;
@@ -667,7 +679,7 @@ k_dslash(IOO out, IOI in, IOI own_f, const cplx<typename IOI::real> *__restrict_
       CVC_HOP(0); CVC_HOP(1); CVC_HOP(2); CVC_HOP(3); CVC_HOP(4); CVC_HOP(5); CVC_HOP(6); CVC_HOP(7);
 #undef CVC_HOP
     } else {
-#define CVC_HOP(H) hop_plain<IOI, RECON, H, LDSL, LDSS, EO>(acc, ld, U, Ul, P, q, sl)
+#define CVC_HOP(H) hop_plain<IOI, RECON, H, LDSL, LDSS, EO, FEW>(acc, ld, U, Ul, P, q, sl)
       CVC_HOP(0); CVC_HOP(1); CVC_HOP(2); CVC_HOP(3); CVC_HOP(4); CVC_HOP(5); CVC_HOP(6); CVC_HOP(7);
 #undef CVC_HOP
     }
@@ -1088,13 +1100,18 @@ static uint32_t op_sites(int N, uint32_t len, int64_t V) {
 // outputs, the links, the neighbours of the columns' sides), so of the divisors
 // of LX and LY those are taken that read the fewest sides again (weight hw per
 // unit of 2/bx + 2/yb) while the cross-section's spinors stay below `budget`
-// bytes, corrected for padded blocks and for XCDs that get a pair less.  Sweep
+// bytes, corrected for padded blocks and for XCDs that get a pair less; a plane of
+// the column above it reads the x neighbours inside the column again too (whole
+// slices, without that term, at 48 FP64 rhs: 64x32^3 20.8 ms against 16.0 ms for
+// the 2 x 2 columns).  Sweep
 // of 0.6-9 MB and hw 0.1-0.7 over 24 operators (FP64, FP64 / FP32 / FP16
 // even/odd on six lattices): geometric mean 1.5 % above the best of each at
-// 1.5 MB and 0.3, 4-6 % at 1.2 and 2.4 MB.
+// 1.5 MB and 0.3, 4-6 % at 1.2 and 2.4 MB.  1.8 MB against 1.5 MB, FP64: 48 rhs 64x32^3
+// 14.7 / 16.5 ms (2 x 4 columns), 24 rhs 7.06 / 7.27 ms, 24 rhs 40x20^3 1.02 / 1.09 ms,
+// even/odd 12 rhs at 40x20^3 3 % slower.
 static void best_columns(const Lattice &L, int N, int K, uint32_t &bx, uint32_t &yb) {
   const double site = 12. * 16 / K * N;   // bytes of a site's spinors
-  const double budget = 1.5e6, hw = 0.3;
+  const double budget = 1.8e6, hw = 0.3;
   double best = 0.;
   bx = yb = 1;
   for (int cx = 1; cx <= L.LX; cx++) {
@@ -1105,8 +1122,9 @@ static void best_columns(const Lattice &L, int N, int K, uint32_t &bx, uint32_t 
       const double pad = (double)((len + S - 1) / S * S) / len;
       const double npair = (double)(L.LX / cx) * (L.LY / cy) * L.T, npx = ceil(npair / kXcds);
       const double halo = (cx < L.LX ? 2. / cx : 0.) + (cy < L.LY ? 2. / cy : 0.);
-      const double over = site * cx * len / budget;
-      const double cost = (1. + hw * halo + (over > 1. ? hw * 2 * (1. - 1. / over) : 0.)) * pad * (npx * kXcds / npair);
+      auto missed = [&](double bytes) { return bytes > budget ? 2. * (1. - budget / bytes) : 0.; };
+      const double again = halo + missed(site * cx * len) + (1. - 1. / cx) * missed(site * len);
+      const double cost = (1. + hw * again) * pad * (npx * kXcds / npair);
       if (best == 0. || cost < best) {
         best = cost;
         bx = (uint32_t)cx;
@@ -1385,15 +1403,19 @@ static int launch(cvchip_ctx *c, Field &out, const Field &in, double mutm, int g
   // bits 24-27: extra LDS per block in 8 KiB units (caps the blocks per CU)
   const size_t pad = (size_t)((c->dslash_policy >> 24) & 15) * 8192;
   const size_t dyn = (ldss ? (size_t)(B / N + 2) * N * 12 * sizeof(cplx<R>) : 0) + pad;
+  constexpr bool kFew = IOI::K <= 2;   // kernels of their own for the fewest rhs (see hop_plain)
+  const bool few = kFew && N <= (k64 ? 2 : 1);
 #define CVC_LAUNCH(G5, DMV)                                                                                     \
   do {                                                                                                          \
     if constexpr (EO) {                                                                                         \
       if (ldsl) hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, true, false, true, IOR>), g, b, dyn, c->stream, o, ii, ow, U, P, rr, part); \
+      else if (few) hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, false, false, true, IOR, kFew>), g, b, dyn, c->stream, o, ii, ow, U, P, rr, part); \
       else hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, false, false, true, IOR>), g, b, dyn, c->stream, o, ii, ow, U, P, rr, part); \
     } else {                                                                                                    \
       if (ldsl && ldss) hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, true, true, false, IOR>), g, b, dyn, c->stream, o, ii, ii, U, P, rr, part); \
       else if (ldsl) hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, true, false, false, IOR>), g, b, dyn, c->stream, o, ii, ii, U, P, rr, part); \
       else if (ldss) hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, false, true, false, IOR>), g, b, dyn, c->stream, o, ii, ii, U, P, rr, part); \
+      else if (few) hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, false, false, false, IOR, kFew>), g, b, dyn, c->stream, o, ii, ii, U, P, rr, part); \
       else hipLaunchKernelGGL((k_dslash<IOI, IOO, RECON, G5, DMV, false, false, false, IOR>), g, b, dyn, c->stream, o, ii, ii, U, P, rr, part); \
     }                                                                                                           \
   } while (0)
