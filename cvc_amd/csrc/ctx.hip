@@ -652,8 +652,8 @@ extern "C" int cvchip_ctx_set_dslash_policy(cvchip_ctx *c, int policy) {
     const int bt = (policy >> 16) & 15, bx = (policy >> 20) & 15;
     if (policy < 0 || policy >= (1 << 28) || mode > 6) {
       set_error("operator policy 0x%x: bits 0-3 staging/streaming, 4-7 traversal 0..6, 8-15 y-block "
-                "(traversal 6: march length), 16-19 brick t (traversal 5: log2 of the column's z extent; 6: patch x), "
-                "20-23 brick x (traversal 6: patch y), 24-27 LDS padding",
+                "(traversal 6: march length), 16-19 log2 of the column's z extent (traversal 5; 6: patch x), "
+                "20-23 column x extent (traversal 6: patch y), 24-27 LDS padding",
                 policy);
       return CVCHIP_ERR_ARG;
     }

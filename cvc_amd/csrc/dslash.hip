@@ -1210,7 +1210,7 @@ static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
         return t;
       }
     }
-    want = 4;   // a column request that does not tile the lattice falls back to bricks
+    want = 4;   // a column request that does not tile the lattice falls back to mode 4
   }
   if (want == 4 && L.LX % (int)bx == 0 && L.LY % (int)yb == 0) {
     t.mode = 4;
@@ -1225,7 +1225,7 @@ static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
     t.nblk = kXcds * t.npx * t.bpp;
     return t;
   }
-  // (a brick request that does not tile the lattice falls back to mode 2)
+  // (a mode 4 request that does not tile the lattice falls back to mode 2)
   if ((want == 2 || want == 4) && L.T % (int)kXcds == 0 && L.LY % (int)yb == 0) {
     t.mode = 2;
     t.yb = yb;

@@ -77,25 +77,26 @@ int cvchip_ctx_set_link_recon(cvchip_ctx *ctx, int recon);
 int cvchip_ctx_set_solver_flags(cvchip_ctx *ctx, unsigned flags);
 /* operator tuning.  Bits 0-1, staging of the multi-rhs operator (N >= 8): bit 0
  * keeps a block's links in LDS, bit 1 its own and z-neighbour spinors; bit 2
- * writes outputs of 256 MB and more with streaming (non-temporal) stores, bit 3
+ * writes outputs of 128 MB and more with streaming (non-temporal) stores, bit 3
  * every output.  Bits 4-7,
  * block-to-site traversal: 0 automatic, 1 time slices cut into 8 XCD chunks,
- * 2 one time slice per XCD walked in y blocks, 3 linear, 4 bricks of bt x bx x
- * yb x LZ sites marched along t per XCD, 5 columns of bx x yb x zb sites
+ * 2 one time slice per XCD walked in y blocks, 3 linear, 4 columns of bx x yb x
+ * LZ sites swept in t, their (column, slice) pairs cut into eight runs, one per
+ * XCD, 5 columns of bx x yb x zb sites
  * (powers of two) swept along t per XCD, 6 t march (multi-rhs operator on the
  * whole lattice: each workgroup walks its columns through consecutive time
  * slices and carries the backward t hop in registers; bits 8-15 the march
  * length (0: 16), bits 16-19 and 20-23 the x and y extents of the patches of
  * columns that one XCD works on together (0: 8)).  Bits 8-15: the y-block height of
- * traversals 2, 4 and 5 (0: the largest of 16, 8, 4, 2 dividing LY; for the
- * automatic bricks the largest of 8, 4, 2 with yb * N <= 96; 4 for traversal
- * 5); bits 16-19 bt of traversal 4 (0: 4) or log2 zb of traversal 5 (0: zb 8)
+ * traversals 2, 4 and 5 (0: the largest of 16, 8, 4, 2 dividing LY; 4 for
+ * traversal 5); bits 16-19 log2 zb of traversal 5 (0: zb 8; traversal 4 takes
+ * no notice of them)
  * and 20-23 bx of traversals 4 and 5 (0: 4); bits 24-27 extra LDS per block in
  * 8 KiB units (caps the resident blocks).  Default 5: links in LDS,
- * streaming stores, automatic traversal (for N >= 8 bricks of 4 slices x 4
- * x-planes x yb y-rows, yb the largest of 16, 8, 4, 2 dividing LY with
- * yb * N <= 96 K, K = 1, 2, 4 for FP64, FP32, FP16+norm spinors; for the FP32
- * operator with 8 <= N <= 20 the t march over 4 slices in patches of 8x8
+ * streaming stores, automatic traversal (for N >= 8 traversal 4 with the divisors
+ * bx of LX and yb of LY whose cross-section's spinors fit an XCD's L2 beside what
+ * streams through; for the FP32 operator with 8 <= N <= 16 on sets of 2 GiB and more,
+ * LX and LY multiples of 8, the t march over 4 slices in patches of 8x8
  * columns).  The operator output
  * does not depend on the traversal up to rounding (the t march sums the
  * diagonal term first); the fused dot products of the solvers differ at
