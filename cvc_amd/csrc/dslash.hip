@@ -415,9 +415,9 @@ __device__ __forceinline__ void hop_links(cplx<typename IO::real> acc[12], const
 // spinor in flight, so two waves per SIMD instead of four, which read 15.6
 // instead of 19.4 GB from beyond L2 at 64x32^3 with 12 rhs.  Together with the
 // batched link staging, the columns and the scalar index arithmetic, 12 rhs
-// (before -> now): FP64 64x32^3 3.90 -> 3.45 ms, 40x20^3 649 -> 500 us, 32x16^3
-// 246 -> 200 us; even/odd at 40x20^3 FP64 375 -> 288 us, FP32 188 -> 156 us,
-// FP16 108 -> 92 us.
+// (before -> now): FP64 64x32^3 3.90 -> 3.51 ms, 40x20^3 649 -> 510 us, 32x16^3
+// 246 -> 200 us; even/odd at 40x20^3 FP64 375 -> 265 us, FP32 188 -> 150 us,
+// FP16 108 -> 85 us.
 template <typename IO, int RECON, int H, bool EO>
 __device__ __forceinline__ void hop_pipelined(cplx<typename IO::real> acc[12], Raw<IO> &raw, const IO &in,
                                               const IO &own, typename IO::real one, const cplx<typename IO::real> *__restrict__ Ul,
@@ -1106,12 +1106,12 @@ static uint32_t op_sites(int N, uint32_t len, int64_t V) {
 // the 2 x 2 columns).  Sweep
 // of 0.6-9 MB and hw 0.1-0.7 over 24 operators (FP64, FP64 / FP32 / FP16
 // even/odd on six lattices): geometric mean 1.5 % above the best of each at
-// 1.5 MB and 0.3, 4-6 % at 1.2 and 2.4 MB.  1.8 MB against 1.5 MB, FP64: 48 rhs 64x32^3
-// 14.7 / 16.5 ms (2 x 4 columns), 24 rhs 7.06 / 7.27 ms, 24 rhs 40x20^3 1.02 / 1.09 ms,
-// even/odd 12 rhs at 40x20^3 3 % slower.
-static void best_columns(const Lattice &L, int N, int K, uint32_t &bx, uint32_t &yb) {
+// 1.5 MB and 0.3, 4-6 % at 1.2 and 2.4 MB.  1.8 MB against 1.5 MB, FP64: whole lattice, 48
+// rhs 64x32^3 14.7 / 16.5 ms (2 x 4 columns), 24 rhs 7.06 / 7.27 ms, 24 rhs 40x20^3 1.02 /
+// 1.09 ms, but even/odd, 12 rhs 40x20^3, 285 / 265 us.
+static void best_columns(const Lattice &L, int N, int K, bool eo, uint32_t &bx, uint32_t &yb) {
   const double site = 12. * 16 / K * N;   // bytes of a site's spinors
-  const double budget = 1.8e6, hw = 0.3;
+  const double budget = eo ? 1.5e6 : 1.8e6, hw = 0.3;   // even/odd forms stream own spinors too
   double best = 0.;
   bx = yb = 1;
   for (int cx = 1; cx <= L.LX; cx++) {
@@ -1145,7 +1145,7 @@ static void best_columns(const Lattice &L, int N, int K, uint32_t &bx, uint32_t 
 // FP16+norm).  The FP32 operator on the whole lattice marches in t (mode 6,
 // marches of 4 slices) where a set of up to 16 rhs is 2 GiB or more: 1.73 ms
 // against 1.87 ms for the columns at 64x32^3 with 12 rhs; on smaller lattices the
-// columns win (40x20^3 268 against 431 us, 32x16^3 110 against 139 us, 32^4 with
+// columns win (40x20^3 285 against 431 us, 32x16^3 110 against 139 us, 32^4 with
 // 20 rhs 1.54 against 1.56 ms).
 static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
   Lattice L = c->lat;
@@ -1168,7 +1168,7 @@ static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
   uint32_t yb = (uint32_t)((c->dslash_policy >> 8) & 255);
   uint32_t bx = (uint32_t)((c->dslash_policy >> 20) & 15);
   if (want == 0 && N >= 8) {
-    best_columns(L, N, K, bx, yb);
+    best_columns(L, N, K, eo, bx, yb);
     want = 4;
   }
   if (want == 0) want = 1;
