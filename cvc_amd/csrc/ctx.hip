@@ -23,6 +23,7 @@ void set_error(const char *fmt, ...) {
 }
 
 int hip_fail(hipError_t e, const char *what, const char *file, int line) {
+  (void)hipGetLastError();   // reported here: the next launch check must not find it again
   set_error("HIP error %d (%s) in %s at %s:%d", (int)e, hipGetErrorString(e), what, file, line);
   if (e == hipErrorOutOfMemory) return CVCHIP_ERR_OOM;
   return CVCHIP_ERR_HIP;
@@ -33,7 +34,7 @@ int ensure_stage(cvchip_ctx *c, size_t bytes) {
   if (c->stage) CVC_HIP(hipFree(c->stage));
   c->stage = nullptr;
   c->stage_bytes = 0;
-  CVC_HIP(hipMalloc(&c->stage, bytes));
+  CVC_TRY(device_malloc(c, (void **)&c->stage, bytes));
   c->stage_bytes = bytes;
   return 0;
 }
@@ -172,7 +173,7 @@ int ensure_red(cvchip_ctx *c, size_t bytes) {
   if (c->red.ptr) CVC_HIP(hipFree(c->red.ptr));
   c->red.ptr = nullptr;
   c->red.bytes = 0;
-  CVC_HIP(hipMalloc(&c->red.ptr, bytes));
+  CVC_TRY(device_malloc(c, &c->red.ptr, bytes));
   c->red.bytes = bytes;
   return 0;
 }
@@ -182,7 +183,7 @@ int ensure_red2(cvchip_ctx *c, size_t bytes) {
   if (c->red2.ptr) CVC_HIP(hipFree(c->red2.ptr));
   c->red2.ptr = nullptr;
   c->red2.bytes = 0;
-  CVC_HIP(hipMalloc(&c->red2.ptr, bytes));
+  CVC_TRY(device_malloc(c, &c->red2.ptr, bytes));
   c->red2.bytes = bytes;
   return 0;
 }
@@ -198,7 +199,7 @@ static size_t elem_bytes(int prec) {
 // (Releasing the whole pool instead made a 60-column even/odd solve, repeated
 // after solves of other widths near the device's capacity, allocate its
 // workspaces anew on every call: 4.4 s against 1.9 s.)
-static int device_malloc(cvchip_ctx *c, void **p, size_t bytes) {
+int device_malloc(cvchip_ctx *c, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   while (e != hipSuccess && !c->idle.empty()) {
     (void)hipGetLastError();   // clear the failed allocation's error, then retry with fewer idle buffers

@@ -1,0 +1,227 @@
+// The library's host paths on a CPU: its sources compiled for the host alone and
+// linked against the stand-in HIP runtime below.  Device memory is host memory,
+// copies are made at once, kernels are only noted, except that the solver's test
+// kernels report the iteration at which a solve is to converge.  A chosen runtime
+// call can be made to fail, so that every error path of an entry point runs.
+//
+// One scenario per run: host_paths <scenario>; exit code 0 and a last line "ok".
+#include <stdio.h>
+#include <stdint.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "../../cvc_amd/csrc/solver.hip"
+
+namespace fake {
+
+// ---------------------------------------------------------------- state
+std::map<void *, size_t> dev, pinned;          // live allocations
+std::set<void *> events, streams;
+std::map<const void *, std::string> &names() {   // kernels by host stub (registered before main)
+  static std::map<const void *, std::string> n;
+  return n;
+}
+struct Launch {
+  std::string name;
+  dim3 grid, block;
+};
+std::vector<Launch> launches;
+hipError_t last = hipSuccess;
+long allocs = 0, fail_alloc = 0;               // allocation number that fails (0: none)
+size_t capacity = SIZE_MAX, used = 0;          // device memory
+
+// convergence that the solver's kernels report
+int conv_it = 3, conv_rhs = 1 << 30;           // columns below conv_rhs converge at iteration conv_it
+
+hipError_t ok_or(bool bad, hipError_t e) {
+  if (bad) last = e;
+  return bad ? e : hipSuccess;
+}
+hipError_t alloc(std::map<void *, size_t> &live, void **p, size_t n) {
+  if (++allocs == fail_alloc || (&live == &dev && n > capacity - used)) return last = hipErrorOutOfMemory;
+  *p = calloc(n ? n : 1, 1);
+  live[*p] = n;
+  if (&live == &dev) used += n;
+  return hipSuccess;
+}
+hipError_t release(std::map<void *, size_t> &live, void *p) {
+  if (!p) return hipSuccess;
+  if (!live.count(p)) {
+    fprintf(stderr, "free of %p, which is not allocated\n", p);
+    abort();
+  }
+  if (&live == &dev) used -= live[p];
+  live.erase(p);
+  free(p);
+  return hipSuccess;
+}
+
+template <typename T> T arg(void **a, int k) { return *(T *)a[k]; }
+
+void kernel(const std::string &n, dim3 grid, void **a) {
+  using namespace cvchip;
+  const bool test = n.find("k_sc_test") != std::string::npos, beta = n.find("k_sc_beta") != std::string::npos;
+  if (test || beta) {
+    RhsState *st = arg<RhsState *>(a, 0);
+    RhsMirror *m = arg<RhsMirror *>(a, 1);
+    const int it = arg<int>(a, beta ? 5 : 4), mixed = beta ? arg<int>(a, 6) : 0;
+    for (int r = 0; r < (int)grid.x; r++) {
+      if (!mixed && it >= conv_it && r < conv_rhs && !st[r].done) st[r].done = 1, st[r].iter = it;
+      st[r].upd = mixed && !st[r].done && (it == 1 || it == conv_it);
+      m[r].norm = m[r].normb = 1.;
+      m[r].done = st[r].done;
+      m[r].upd = st[r].upd;
+      m[r].seq = it + 1;
+    }
+  }
+  if (n.find("k_sc_reliable") != std::string::npos) {
+    RhsState *st = arg<RhsState *>(a, 0);
+    const int N = arg<int>(a, 2), it = arg<int>(a, 3);
+    for (int r = 0; r < N && r < conv_rhs; r++)
+      if (it >= conv_it && !st[r].done) st[r].done = 1, st[r].iter = it;
+  }
+}
+
+}  // namespace fake
+
+// ---------------------------------------------------------------- the runtime
+using namespace fake;
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) { return alloc(dev, p, n); }
+hipError_t hipFree(void *p) { return release(dev, p); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return alloc(pinned, p, n); }
+hipError_t hipHostFree(void *p) { return release(pinned, p); }
+hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
+hipError_t hipGetLastError(void) {
+  const hipError_t e = last;
+  last = hipSuccess;
+  return e;
+}
+const char *hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipGetSymbolAddress(void **p, const void *) {
+  static char buf[1 << 21];
+  return *p = buf, hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+  *s = (hipStream_t)malloc(1);
+  streams.insert(*s);
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s) { return streams.erase(s), free(s), hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  *e = (hipEvent_t)malloc(1);
+  events.insert(*e);
+  return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventDestroy(hipEvent_t e) { return events.erase(e), free(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *t, hipEvent_t, hipEvent_t) { return *t = 0.f, hipSuccess; }
+// (what kernels alone would use stays zero, so that large sets are never touched)
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) {
+  if (k != hipMemcpyDeviceToDevice) memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t) {
+  if (n < (size_t)1 << 20) memset(p, v, n);
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t, hipStream_t) {
+  launches.push_back({names()[f], g, b});
+  kernel(names()[f], g, a);
+  return hipSuccess;
+}
+struct Config {
+  dim3 g, b;
+  size_t lds;
+  hipStream_t s;
+};
+static Config config;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s) { return config = {g, b, lds, s}, hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s) {
+  *g = config.g, *b = config.b, *lds = config.lds, *s = config.s;
+  return hipSuccess;
+}
+void **__hipRegisterFatBinary(const void *) {
+  static void *m;
+  return &m;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *,
+                           int *) {
+  names()[f] = name;
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+}
+
+// ---------------------------------------------------------------- scenarios
+#define CHECK(cond, ...)                                                \
+  do {                                                                  \
+    if (!(cond)) {                                                      \
+      fprintf(stderr, "%s:%d: %s: ", __FILE__, __LINE__, #cond);        \
+      fprintf(stderr, __VA_ARGS__);                                     \
+      fprintf(stderr, " (last error: %s)\n", cvchip_last_error());      \
+      exit(1);                                                          \
+    }                                                                   \
+  } while (0)
+
+struct Ctx {
+  cvchip_ctx *c = nullptr;
+  size_t V;
+  std::vector<double> gauge;
+  explicit Ctx(int T, int X, int Y, int Z) : V((size_t)T * X * Y * Z), gauge(72 * V) {
+    const int d[4] = {T, X, Y, Z};
+    const double bc[4] = {1, 0, 0, 0};
+    CHECK(!cvchip_ctx_create(&c, d, bc, 0.15, 0.01), "create");
+    CHECK(!cvchip_set_gauge(c, gauge.data()), "gauge");
+  }
+  ~Ctx() {
+    cvchip_ctx_destroy(c);
+    CHECK(dev.empty() && pinned.empty() && events.empty() && streams.empty(),
+          "left behind: %zu device, %zu pinned, %zu events, %zu streams", dev.size(), pinned.size(), events.size(),
+          streams.size());
+  }
+};
+
+static int solve(Ctx &x, int nrhs, int prec, unsigned flags, cvchip_stats *st = nullptr, bool her = true) {
+  std::vector<double> b(24 * x.V * nrhs), y(b.size());
+  cvchip_stats s;
+  return (her ? cvchip_invert_Qtm_her : cvchip_invert_Qtm)(x.c, y.data(), b.data(), nrhs, 1e-20, 20, prec, 0.1, flags,
+                                                           st ? st : &s);
+}
+
+// scratch that does not fit beside the context's idle buffers takes their place, and
+// one that does not fit at all leaves no error for the next call to find
+static void scratch() {
+  using namespace cvchip;
+  int (*const ensure[3])(cvchip_ctx *, size_t) = {ensure_stage, ensure_red, ensure_red2};
+  for (auto f : ensure) {
+    Ctx x(4, 2, 2, 4);
+    Field idle;
+    CHECK(!field_alloc(x.c, idle, 60, CVCHIP_PREC_F64), "field");
+    field_free(idle);
+    capacity = used;
+    CHECK(!f(x.c, idle.bytes / 2), "scratch beside idle buffers");
+    CHECK(f(x.c, 4 * idle.bytes) == CVCHIP_ERR_OOM, "scratch beyond the device");
+    capacity = SIZE_MAX;
+    CHECK(hipGetLastError() == hipSuccess, "error left behind");
+  }
+}
+
+int main(int argc, char **argv) {
+  const std::map<std::string, void (*)()> all = {{"scratch", scratch}};
+  const auto it = argc == 2 ? all.find(argv[1]) : all.end();
+  if (it == all.end()) return 2;
+  it->second();
+  puts("ok");
+  return 0;
+}
