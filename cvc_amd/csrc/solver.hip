@@ -712,6 +712,28 @@ struct OpMask {
   ~OpMask() { clear(); }
 };
 
+// The small buffers of a solve, for the largest N: all of them or, on failure, none
+// (a later solve finds them complete or makes them).
+constexpr int kMaxRhs = 256;
+static int solve_buffers(cvchip_ctx *c, SolveBuffers &B) {
+  if (B.st) return 0;
+  SolveBuffers n;
+  int rc = device_malloc(c, &n.st, sizeof(RhsState) * kMaxRhs);
+  if (!rc) rc = device_malloc(c, &n.res, sizeof(double) * 4 * kMaxRhs);
+  if (!rc) {
+    const hipError_t e = hipHostMalloc(&n.hst, (sizeof(RhsState) + sizeof(RhsMirror)) * kMaxRhs,
+                                       hipHostMallocCoherent | hipHostMallocMapped);
+    if (e != hipSuccess) rc = hip_fail(e, "pinned solver state", __FILE__, __LINE__);
+  }
+  if (rc) {
+    if (n.st) (void)hipFree(n.st);
+    if (n.res) (void)hipFree(n.res);
+    return rc;
+  }
+  B = n;
+  return 0;
+}
+
 // V: sites of the solver's vectors (the lattice, or one parity of it)
 static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   S.c = c;
@@ -727,25 +749,15 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 7 * N + 64 * 256)));
   // The small buffers are made once per context, for the largest N; a second
   // solve running at the same time on the context gets its own.
-  constexpr int kMaxN = 256;
-  cvchip::SolveBuffers &B = c->solve_bufs;
+  cvchip::SolveBuffers own, &B = c->solve_bufs;
   S.kept = !B.in_use;
-  if (S.kept && !B.st) {
-    CVC_HIP(hipMalloc(&B.st, sizeof(RhsState) * kMaxN));
-    CVC_HIP(hipMalloc(&B.res, sizeof(double) * 4 * kMaxN));
-    CVC_HIP(hipHostMalloc(&B.hst, (sizeof(RhsState) + sizeof(RhsMirror)) * kMaxN, hipHostMallocCoherent | hipHostMallocMapped));
-  }
-  if (S.kept) {
-    B.in_use = true;
-    S.st = (RhsState *)B.st;
-    S.res = (double *)B.res;
-    S.hst = (RhsState *)B.hst;
-  } else {
-    CVC_HIP(hipMalloc(&S.st, sizeof(RhsState) * N));
-    CVC_HIP(hipMalloc(&S.res, sizeof(double) * 4 * N));
-    CVC_HIP(hipHostMalloc(&S.hst, (sizeof(RhsState) + sizeof(RhsMirror)) * kMaxN, hipHostMallocCoherent | hipHostMallocMapped));
-  }
-  S.mir = (RhsMirror *)(S.hst + kMaxN);
+  CVC_TRY(solve_buffers(c, S.kept ? B : own));
+  const cvchip::SolveBuffers &use = S.kept ? B : own;
+  if (S.kept) B.in_use = true;
+  S.st = (RhsState *)use.st;
+  S.res = (double *)use.res;
+  S.hst = (RhsState *)use.hst;
+  S.mir = (RhsMirror *)(S.hst + kMaxRhs);
   for (int r = 0; r < N; r++) S.mir[r].seq = 0;
   // The next iteration's first operator goes out before the host has seen this
   // iteration's residual while that operator is short: it hides the host's wait and

@@ -217,8 +217,23 @@ static void scratch() {
   }
 }
 
+// a solve none of whose allocations fails works after one that lacked any of them
+static void solver_buffers() {
+  for (long k = 1;; k++) {
+    fprintf(stderr, "allocation %ld refused\n", k);
+    Ctx x(4, 2, 2, 4);
+    fail_alloc = allocs + k;
+    const int rc = solve(x, 3, CVCHIP_PREC_F64, 0);
+    const bool reached = allocs >= fail_alloc;
+    fail_alloc = 0;
+    CHECK(reached ? rc < 0 : rc >= 0, "allocation %ld: %d", k, rc);
+    CHECK(solve(x, 3, CVCHIP_PREC_F64, 0) >= 0, "solve after allocation %ld failed", k);
+    if (!reached) break;
+  }
+}
+
 int main(int argc, char **argv) {
-  const std::map<std::string, void (*)()> all = {{"scratch", scratch}};
+  const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();
