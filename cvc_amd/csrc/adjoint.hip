@@ -474,7 +474,7 @@ extern "C" int cvchip_cvc_gradient(cvchip_ctx *c, const int src[4], double qmax,
       ysp[nu] = site_of(c, src[0] + d[0], src[1] + d[1], src[2] + d[2], src[3] + d[3]);
     }
 
-    Field up, dn, xu, xd;
+    TmpField up, dn, xu, xd;
     double *cw = nullptr, *dqs = nullptr;
     double2 *psi = nullptr, *K = nullptr, *blk = nullptr;
     std::vector<double> conn((size_t)32 * V);
@@ -708,10 +708,6 @@ extern "C" int cvchip_cvc_gradient(cvchip_ctx *c, const int src[4], double qmax,
     *L_out = Lval;
     *dmu_out = dmu;
     if (stats) *stats = tot;
-    field_free(up);
-    field_free(dn);
-    field_free(xu);
-    field_free(xd);
     if (cw) (void)hipFree(cw);
     if (dqs) (void)hipFree(dqs);
     if (psi) (void)hipFree(psi);

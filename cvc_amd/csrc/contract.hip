@@ -568,13 +568,11 @@ extern "C" int cvchip_cvc_contract(cvchip_ctx *c, double *conn, double contact[8
         set_error("propagator %d is NULL", k);
         return CVCHIP_ERR_NULL;
       }
-    Field up, dn;
+    TmpField up, dn;
     int rc = field_alloc(c, up, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, dn, 60, CVCHIP_PREC_F64);
     for (int k = 0; k < 120 && !rc; k++) rc = upload_aos(c, k < 60 ? up : dn, props[k], k % 60, 1);
     if (!rc) rc = contract_fields(c, conn, contact, up, dn, src);
-    field_free(up);
-    field_free(dn);
     return rc;
   });
 }
@@ -643,13 +641,20 @@ int solve_five_sources(cvchip_ctx *c, Field &out, double mu, const std::function
                        double sp, int niter_max, int prec, double delta, cvchip_stats *tot) {
   // solves the 12 ns columns of b into x
   auto solve = [&](Field &x, const Field &b, int ns) -> int {
-    if (hipMemsetAsync(x.data, 0, x.bytes, c->stream) != hipSuccess) return CVCHIP_ERR_HIP;
+    CVC_HIP(hipMemsetAsync(x.data, 0, x.bytes, c->stream));
     cvchip_stats st;
     memset(&st, 0, sizeof(st));
-    const double mu0 = c->mu;
-    c->mu = mu;
-    const int rc = invert_her_fields(c, x, b, sp, niter_max, prec, delta, 0, &st);
-    c->mu = mu0;
+    struct Mass {   // the context's own mass again on every path
+      cvchip_ctx *c;
+      double mu0;
+      ~Mass() { c->mu = mu0; }
+    };
+    int rc;
+    {
+      const Mass restore{c, c->mu};
+      c->mu = mu;
+      rc = invert_her_fields(c, x, b, sp, niter_max, prec, delta, 0, &st);
+    }
     if (rc < 0) return rc;
     if (tot) {
       // the iterations of 12 columns are those of the slowest of them
@@ -663,7 +668,7 @@ int solve_five_sources(cvchip_ctx *c, Field &out, double mu, const std::function
     }
     return 0;
   };
-  Field all, b, x;
+  TmpField all, b, x;
   bool have_all = c->lat.V <= kBatchSites;
   int rc = 0;
   if (have_all && field_alloc(c, all, 60, CVCHIP_PREC_F64)) have_all = false;
@@ -680,9 +685,6 @@ int solve_five_sources(cvchip_ctx *c, Field &out, double mu, const std::function
       if (!rc) rc = copy_columns(c, out, 12 * s, x, 0, 12);
     }
   }
-  field_free(all);
-  field_free(b);
-  field_free(x);
   return rc;
 }
 
@@ -710,7 +712,7 @@ extern "C" int cvchip_cvc_source(cvchip_ctx *c, double *conn, double contact[8],
       set_error("NULL argument to cvchip_cvc_source");
       return CVCHIP_ERR_NULL;
     }
-    Field up, dn;
+    TmpField up, dn;
     int rc = field_alloc(c, up, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, dn, 60, CVCHIP_PREC_F64);
     cvchip_stats tot;
@@ -718,8 +720,6 @@ extern "C" int cvchip_cvc_source(cvchip_ctx *c, double *conn, double contact[8],
     if (!rc) rc = solve_source_props(c, src, sp, niter_max, prec, delta, up, dn, &tot);
     if (!rc) rc = contract_fields(c, conn, contact, up, dn, src);
     if (stats) *stats = tot;
-    field_free(up);
-    field_free(dn);
     return rc;
   });
 }
@@ -737,7 +737,7 @@ extern "C" int cvchip_cvc_propagators(cvchip_ctx *c, double *const *props, const
         set_error("propagator %d is NULL", k);
         return CVCHIP_ERR_NULL;
       }
-    Field up, dn;
+    TmpField up, dn;
     int rc = field_alloc(c, up, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, dn, 60, CVCHIP_PREC_F64);
     cvchip_stats tot;
@@ -745,8 +745,6 @@ extern "C" int cvchip_cvc_propagators(cvchip_ctx *c, double *const *props, const
     if (!rc) rc = solve_source_props(c, src, sp, niter_max, prec, delta, up, dn, &tot);
     for (int k = 0; k < 120 && !rc; k++) rc = download_aos(c, k < 60 ? up : dn, props[k], k % 60, 1);
     if (stats) *stats = tot;
-    field_free(up);
-    field_free(dn);
     return rc;
   });
 }

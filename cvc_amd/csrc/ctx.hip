@@ -237,7 +237,12 @@ int pool_get(cvchip_ctx *c, void **p, size_t bytes) {
 // cannot overtake an earlier kernel.
 void pool_put(cvchip_ctx *c, void *p, size_t bytes) {
   if (!p) return;
-  c->idle.emplace_back(p, bytes);
+  try {
+    c->idle.emplace_back(p, bytes);
+  } catch (...) {   // no room to note it (called from destructors: nothing may escape)
+    (void)hipFree(p);
+    return;
+  }
   c->idle_bytes += bytes;
   while (c->idle_bytes > kPoolIdleMax && !c->idle.empty()) {   // oldest first
     (void)hipFree(c->idle.front().first);

@@ -127,10 +127,9 @@ struct Traversal {
 };
 
 // A solve's per-rhs state on the device and its pinned host side (solver.hip),
-// kept by the context between solves
+// kept by the context between solves (one at a time runs on a context)
 struct SolveBuffers {
   void *st = nullptr, *res = nullptr, *hst = nullptr;
-  bool in_use = false;
 };
 
 struct Scratch {
@@ -244,6 +243,14 @@ constexpr size_t kPoolIdleMax = (size_t)160 << 30;   // of 288 GB: the workspace
 int pool_get(cvchip_ctx *c, void **p, size_t bytes);
 void pool_put(cvchip_ctx *c, void *p, size_t bytes);
 void pool_release(cvchip_ctx *c);
+
+// A temporary set that returns to the pool where its scope ends, on every path
+struct TmpField : Field {
+  TmpField() = default;
+  TmpField(const TmpField &) = delete;
+  TmpField &operator=(const TmpField &) = delete;
+  ~TmpField() { field_free(*this); }
+};
 
 // host AoS [V][24] (nrhs contiguous fields) <-> device field rhs range
 int upload_aos(cvchip_ctx *c, Field &f, const double *host, int rhs0, int n);

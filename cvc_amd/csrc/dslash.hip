@@ -1634,14 +1634,12 @@ extern "C" int cvchip_Q_phi(cvchip_ctx *c, double *xi, const double *phi, double
       set_error("NULL argument to cvchip_Q_phi");
       return CVCHIP_ERR_NULL;
     }
-    Field a, b;
+    TmpField a, b;
     int rc = field_alloc(c, a, 1, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, b, 1, CVCHIP_PREC_F64);
     if (!rc) rc = upload_aos(c, a, phi, 0, 1);
     if (!rc) rc = dslash(c, b, a, mutm, gamma5_out);
     if (!rc) rc = download_aos(c, b, xi, 0, 1);
-    field_free(a);
-    field_free(b);
     return rc;
   });
 }

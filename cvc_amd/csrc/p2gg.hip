@@ -142,7 +142,7 @@ extern "C" int cvchip_p2gg_source(cvchip_ctx *c, double *conn, double contact[8]
     const int T = c->lat.T;
     const int tseq = (((src[0] + seq_timeslice) % T) + T) % T;   // p2gg_xspace.c:446
     const double sgn = 1. - 2. * propagator_position;
-    Field up, dn, seq;
+    TmpField up, dn, seq;
     int rc = field_alloc(c, up, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, dn, 60, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, seq, 60, CVCHIP_PREC_F64);
@@ -159,9 +159,6 @@ extern "C" int cvchip_p2gg_source(cvchip_ctx *c, double *conn, double contact[8]
                               sp, niter_max, prec, delta, &tot);
     if (!rc) rc = contract_fields(c, conn, contact, seq, Q, src);
     if (stats) *stats = tot;
-    field_free(up);
-    field_free(dn);
-    field_free(seq);
     return rc;
   });
 }

@@ -682,18 +682,24 @@ __global__ void __launch_bounds__(256) k_p_update(IO p, IO r1, IO p2, const RhsS
 // ------------------------------------------------------------------ driver
 
 struct Solve {
-  cvchip_ctx *c;
-  int N;
-  uint32_t VN;
-  int B;
-  unsigned nblk;
+  cvchip_ctx *c = nullptr;
+  int N = 0;
+  uint32_t VN = 0;
+  int B = 0;
+  unsigned nblk = 0;
   RhsState *st = nullptr;     // device
   double *res = nullptr;      // device [4][N]
   RhsState *hst = nullptr;    // pinned host copy
   RhsMirror *mir = nullptr;   // pinned, written by the device each iteration
-  bool kept = false;          // st .. mir are the context's kept buffers
   int ahead = 0;              // the next iteration's first operator is enqueued before this one's test
   int nt = 0;                 // streaming stores in the vector kernels
+  Solve() = default;
+  Solve(const Solve &) = delete;
+  Solve &operator=(const Solve &) = delete;
+  // nothing of this solve may still write to the context's buffers when the next takes them
+  ~Solve() {
+    if (st) (void)hipStreamSynchronize(c->stream);
+  }
 };
 
 // The operator applications of a running solve skip converged right-hand
@@ -712,8 +718,8 @@ struct OpMask {
   ~OpMask() { clear(); }
 };
 
-// The small buffers of a solve, for the largest N: all of them or, on failure, none
-// (a later solve finds them complete or makes them).
+// The small buffers of a context's solves, for the largest N: all of them or, on
+// failure, none (a later solve finds them complete or makes them).
 constexpr int kMaxRhs = 256;
 static int solve_buffers(cvchip_ctx *c, SolveBuffers &B) {
   if (B.st) return 0;
@@ -747,16 +753,10 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   const size_t nb_max = std::max<size_t>(S.nblk, dslash_blocks(c, N));
   // (two launches' norms side by side in Op::apply_omega)
   CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 7 * N + 64 * 256)));
-  // The small buffers are made once per context, for the largest N; a second
-  // solve running at the same time on the context gets its own.
-  cvchip::SolveBuffers own, &B = c->solve_bufs;
-  S.kept = !B.in_use;
-  CVC_TRY(solve_buffers(c, S.kept ? B : own));
-  const cvchip::SolveBuffers &use = S.kept ? B : own;
-  if (S.kept) B.in_use = true;
-  S.st = (RhsState *)use.st;
-  S.res = (double *)use.res;
-  S.hst = (RhsState *)use.hst;
+  CVC_TRY(solve_buffers(c, c->solve_bufs));
+  S.st = (RhsState *)c->solve_bufs.st;
+  S.res = (double *)c->solve_bufs.res;
+  S.hst = (RhsState *)c->solve_bufs.hst;
   S.mir = (RhsMirror *)(S.hst + kMaxRhs);
   for (int r = 0; r < N; r++) S.mir[r].seq = 0;
   // The next iteration's first operator goes out before the host has seen this
@@ -767,19 +767,6 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   S.ahead = (uint64_t)S.VN <= ((uint64_t)1 << 20);
   CVC_HIP(hipMemsetAsync(S.st, 0, sizeof(RhsState) * N, c->stream));
   return 0;
-}
-
-static void solve_free(Solve &S) {
-  if (S.kept) {
-    // nothing of this solve may still write to the buffers when the next takes them
-    (void)hipStreamSynchronize(S.c->stream);
-    S.c->solve_bufs.in_use = false;
-    S.kept = false;
-    return;
-  }
-  if (S.st) (void)hipFree(S.st);
-  if (S.res) (void)hipFree(S.res);
-  if (S.hst) (void)hipHostFree(S.hst);
 }
 
 static int reduce(Solve &S, int nblk, int Q) {
@@ -967,19 +954,12 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
   const int N = b.nrhs;
   Solve S;
   int rc = solve_setup(c, S, N, x.V);
-  Field r1, r2, s, t, p, p2, aux, tmp;
+  TmpField r1, r2, s, t, p, p2, aux, tmp;
   Field *all[8] = {&r1, &r2, &s, &t, &p, &p2, &aux, &tmp};
   for (int k = 0; k < 6 + (her ? 1 : 0) && !rc; k++) rc = field_alloc(c, *all[k], N, CVCHIP_PREC_F64, x.V);
   if (!rc && eo) rc = field_alloc(c, tmp, N, CVCHIP_PREC_F64, x.V);
-  auto cleanup = [&]() {
-    for (int k = 0; k < 8; k++) field_free(*all[k]);
-    solve_free(S);
-  };
   Op op{c, her, &aux, eo, &tmp};
-  if (rc) {
-    cleanup();
-    return rc;
-  }
+  if (rc) return rc;
   using IO = IOPlain<double>;
   IO ir1 = mkio<IO>(r1), ir2 = mkio<IO>(r2), is = mkio<IO>(s), iT = mkio<IO>(t), ip = mkio<IO>(p),
      ip2 = mkio<IO>(p2), ix = mkio<IO>(x), ib = mkio<IO>(b);
@@ -988,24 +968,15 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
   int dcalls = 0, nb = 0;
   int iters = 0, all_done = 0;
 
-#define TRY(x)                                                                                   \
-  do {                                                                                           \
-    rc = (x);                                                                                    \
-    if (rc) {                                                                                    \
-      cleanup();                                                                                 \
-      return rc;                                                                                 \
-    }                                                                                            \
-  } while (0)
-
   // r = b - D x ; r2 = p = r ; <r,r>, <b,b>
-  TRY(op.apply(t, x, DOT_NONE, nullptr, nullptr));
+  CVC_TRY(op.apply(t, x, DOT_NONE, nullptr, nullptr));
   dcalls++;
   hipLaunchKernelGGL((k_residual<IO, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, ir2, ip, ib, iT, 1,
                      S.st, 0, S.VN, N, (double *)c->red.ptr);
-  TRY(reduce(S, (int)S.nblk, 2));
+  CVC_TRY(reduce(S, (int)S.nblk, 2));
   hipLaunchKernelGGL(k_sc_init, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N, sp, 0);
   OpMask mask(c, S.st);
-  TRY(pull_state(S));
+  CVC_TRY(pull_state(S));
   all_done = 1;
   for (int r = 0; r < N; r++) all_done &= S.hst[r].done;
   // p2 = A p and alpha
@@ -1016,7 +987,7 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
     });
   };
   if (!all_done) {
-    TRY(advance());
+    CVC_TRY(advance());
     dcalls++;
     for (int it = 0; it <= niter_max; it++) {
       // a lagged solve needs |r1|^2 before x moves, so it keeps the separate passes
@@ -1026,7 +997,7 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
       else
         hipLaunchKernelGGL((k_s_update<IO, 1>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N,
                            S.nt, ir2, (double *)c->red.ptr);
-      TRY(op.apply_omega(t, s, c, N, S.st, lagged ? nullptr : &r2, (int)S.nblk));
+      CVC_TRY(op.apply_omega(t, s, c, N, S.st, lagged ? nullptr : &r2, (int)S.nblk));
       dcalls++;
       if (!lagged) {
         if (S.nt)
@@ -1035,13 +1006,13 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
         else
           hipLaunchKernelGGL(k_step<0>, dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, ix, ip, is, iT, ip2, S.st, S.VN, N,
                              (double *)c->red.ptr);
-        TRY(scalar_rows(S, (int)S.nblk, 1, [&](const double *q, int n) {
+        CVC_TRY(scalar_rows(S, (int)S.nblk, 1, [&](const double *q, int n) {
           hipLaunchKernelGGL(k_sc_test, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, it);
         }));
       } else {
         hipLaunchKernelGGL((k_r1_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
                            S.VN, N, (double *)c->red.ptr, S.nt);
-        TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
+        CVC_TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
           hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, 0, 0.0);
         }));
         hipLaunchKernelGGL((k_xp_update<IO, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ix, ip, is, ir1, ip2,
@@ -1050,19 +1021,19 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
       }
       iters = it + 1;
       const bool ahead = S.ahead && it < niter_max;
-      if (ahead) TRY(advance());
-      TRY(wait_state(S, it));
+      if (ahead) CVC_TRY(advance());
+      CVC_TRY(wait_state(S, it));
       all_done = 1;
       for (int r = 0; r < N; r++) all_done &= S.mir[r].done;
       if (verbose)
         for (int r = 0; r < N; r++)
           printf("# [%d] residuum after iteration %d: %25.16e\n", r, it, S.mir[r].norm);
       if (all_done) break;
-      if (!ahead) TRY(advance());
+      if (!ahead) CVC_TRY(advance());
       dcalls++;
     }
   }
-  TRY(pull_state(S));
+  CVC_TRY(pull_state(S));
   record_iterations(S, iters);
   int nconv = 0, maxit = 0;
   for (int r = 0; r < N; r++) {
@@ -1074,7 +1045,7 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
   double tr = 0.;
   mask.clear();
   if (!her && !eo) {
-    TRY(true_residual(S, x, b, t, c->mu, &tr, nullptr));
+    CVC_TRY(true_residual(S, x, b, t, c->mu, &tr, nullptr));
     dcalls++;
   }
   if (stats) {
@@ -1084,8 +1055,6 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
     stats->dslash_calls = dcalls;
     stats->true_res2_max = tr;
   }
-  cleanup();
-#undef TRY
   if (nconv < N) {
     set_error("BiCGStab: %d of %d right-hand sides not converged after %d iterations", N - nconv, N,
               niter_max + 1);
@@ -1102,7 +1071,7 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
   const int N = b.nrhs;
   Solve S;
   int rc = solve_setup(c, S, N, x.V);
-  Field r1, r2, s, t, p, p2, xl, t64, auxl, aux64, tmpl, tmp64;
+  TmpField r1, r2, s, t, p, p2, xl, t64, auxl, aux64, tmpl, tmp64;
   Field *lo[7] = {&r1, &r2, &s, &t, &p, &p2, &xl};
   const int64_t V = x.V;
   // The shadow residual r2 (r^ of BiCGStab) stays fixed through an FP32 solve
@@ -1119,23 +1088,11 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
   if (!rc && her) rc = field_alloc(c, aux64, N, CVCHIP_PREC_F64, V);
   if (!rc && eo) rc = field_alloc(c, tmpl, N, prec, V);
   if (!rc && eo) rc = field_alloc(c, tmp64, N, CVCHIP_PREC_F64, V);
-  auto cleanup = [&]() {
-    for (int k = 0; k < 7; k++) field_free(*lo[k]);
-    field_free(t64);
-    field_free(auxl);
-    field_free(aux64);
-    field_free(tmpl);
-    field_free(tmp64);
-    solve_free(S);
-  };
   Op opl{c, her, &auxl, eo, &tmpl}, op64{c, her, &aux64, eo, &tmp64};
   // FP16 storage keeps too few digits for the Krylov space to survive a
   // residual replacement: restart the recurrence at every reliable update
   const bool restart = prec == CVCHIP_PREC_F16;
-  if (rc) {
-    cleanup();
-    return rc;
-  }
+  if (rc) return rc;
   using IO = IOL;
   using I64 = IOPlain<double>;
   IO ir1 = mkio<IO>(r1), is = mkio<IO>(s), iT = mkio<IO>(t), ip = mkio<IO>(p), ip2 = mkio<IO>(p2);
@@ -1145,32 +1102,23 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
   const double delta2 = delta * delta;
   int dcalls = 0, nb = 0, nrel = 0, iters = 0, all_done = 0;
 
-#define TRY(x)                                                                                   \
-  do {                                                                                           \
-    rc = (x);                                                                                    \
-    if (rc) {                                                                                    \
-      cleanup();                                                                                 \
-      return rc;                                                                                 \
-    }                                                                                            \
-  } while (0)
-
   // r = b - D x in FP64, converted; r2 = p = r; xl = 0
-  TRY(op64.apply(t64, x, DOT_NONE, nullptr, nullptr));
+  CVC_TRY(op64.apply(t64, x, DOT_NONE, nullptr, nullptr));
   dcalls++;
   hipLaunchKernelGGL((k_residual<I64, IO, IOR>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, ir2, ip, ib, it64, 1,
                      S.st, 0, S.VN, N, (double *)c->red.ptr);
-  TRY(reduce(S, (int)S.nblk, 2));
+  CVC_TRY(reduce(S, (int)S.nblk, 2));
   hipLaunchKernelGGL(k_sc_init, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N, sp, 1);
   if constexpr (!std::is_same<IOR, IO>::value) {
     // r0rn = <r2, r> with the stored (FP16) shadow residual, not |r|^2
     hipLaunchKernelGGL((k_dot3<IOR, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir2, ir1, S.VN, N,
                        (double *)c->red.ptr);
-    TRY(reduce(S, (int)S.nblk, 3));
+    CVC_TRY(reduce(S, (int)S.nblk, 3));
     hipLaunchKernelGGL(k_sc_set_r0rn, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N);
   }
   CVC_HIP(hipMemsetAsync(xl.data, 0, xl.bytes, c->stream));
   OpMask mask(c, S.st);
-  TRY(pull_state(S));
+  CVC_TRY(pull_state(S));
   all_done = 1;
   for (int r = 0; r < N; r++) all_done &= S.hst[r].done;
   // p2 = A p and alpha (of the rhs that do not hold their p2)
@@ -1181,16 +1129,16 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
     });
   };
   if (!all_done) {
-    TRY(advance());
+    CVC_TRY(advance());
     dcalls++;
     for (int it = 0; it <= niter_max; it++) {
       hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt,
                          ir1, nullptr);
-      TRY(opl.apply_omega(t, s, c, N, S.st));
+      CVC_TRY(opl.apply_omega(t, s, c, N, S.st));
       dcalls++;
       hipLaunchKernelGGL((k_r1_update<IO, IOR>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, is, iT, ir2, S.st,
                          S.VN, N, (double *)c->red.ptr, S.nt);
-      TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
+      CVC_TRY(scalar_rows(S, (int)S.nblk, 3, [&](const double *q, int n) {
         hipLaunchKernelGGL(k_sc_beta, dim3(N), dim3(kScThreads), 0, c->stream, S.st, S.mir, q, n, N, it, 1, delta2);
       }));
       // xl += omega s + alpha p ; p = r1 + beta (p - omega p2)
@@ -1201,8 +1149,8 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
       // ahead of the test: a rhs whose own update was triggered holds its p2 and
       // alpha, which that update needs; after an update this is done again
       const bool ahead = S.ahead && it < niter_max;
-      if (ahead) TRY(advance());
-      TRY(wait_state(S, it));
+      if (ahead) CVC_TRY(advance());
+      CVC_TRY(wait_state(S, it));
       int any_upd = 0;
       all_done = 1;
       for (int r = 0; r < N; r++) {
@@ -1224,14 +1172,14 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
         hipLaunchKernelGGL(k_sc_upd_all, dim3(1), dim3(256), 0, c->stream, S.st, N);
         hipLaunchKernelGGL((k_accum_zero<I64, IOPlain<float>>), dim3(S.nblk), dim3(S.B), 0, c->stream, ix, ixl, S.st,
                            S.VN, N);
-        TRY(op64.apply(t64, x, DOT_NONE, nullptr, nullptr));
+        CVC_TRY(op64.apply(t64, x, DOT_NONE, nullptr, nullptr));
         dcalls++;
         hipLaunchKernelGGL((k_residual<I64, IO, IOR>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir1, ir2, ip, ib,
                            it64, restart ? 1 : 0, S.st, 1, S.VN, N, (double *)c->red.ptr);
-        TRY(reduce(S, (int)S.nblk, 2));
+        CVC_TRY(reduce(S, (int)S.nblk, 2));
         hipLaunchKernelGGL(k_sc_reliable, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N, it);
         if (verbose) {
-          TRY(pull_state(S));
+          CVC_TRY(pull_state(S));
           double mx = 0.;
           for (int r = 0; r < N; r++) {
             const double q = S.hst[r].norm / S.hst[r].normb;
@@ -1246,22 +1194,22 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
           // r0rn and beta with the replaced residual: <r2, r>
           hipLaunchKernelGGL((k_dot3<IOR, IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ir2, ir1, S.VN, N,
                              (double *)c->red.ptr);
-          TRY(reduce(S, (int)S.nblk, 3));
+          CVC_TRY(reduce(S, (int)S.nblk, 3));
           hipLaunchKernelGGL(k_sc_r0rn, dim3(1), dim3(256), 0, c->stream, S.st, S.res, N);
           hipLaunchKernelGGL((k_p_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, ip, ir1, ip2, S.st, S.VN, N);
           hipLaunchKernelGGL(k_sc_clear_upd, dim3(1), dim3(256), 0, c->stream, S.st, N);
         }
         CVC_HIP(hipGetLastError());
-        TRY(pull_state(S));
+        CVC_TRY(pull_state(S));
         all_done = 1;
         for (int r = 0; r < N; r++) all_done &= S.hst[r].done;
       }
       if (all_done) break;
-      if (!ahead || any_upd) TRY(advance());
+      if (!ahead || any_upd) CVC_TRY(advance());
       dcalls++;
     }
   }
-  TRY(pull_state(S));
+  CVC_TRY(pull_state(S));
   record_iterations(S, iters);
   int nconv = 0, maxit = 0, nstall = 0;
   for (int r = 0; r < N; r++)
@@ -1282,7 +1230,7 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
   double tr = 0.;
   mask.clear();
   if (!her && !eo) {
-    TRY(true_residual(S, x, b, t64, c->mu, &tr, nullptr));
+    CVC_TRY(true_residual(S, x, b, t64, c->mu, &tr, nullptr));
     dcalls++;
   }
   if (stats) {
@@ -1292,8 +1240,6 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
     stats->dslash_calls = dcalls;
     stats->true_res2_max = tr;
   }
-  cleanup();
-#undef TRY
   if (nconv < N) {
     if (nstall)
       set_error("mixed BiCGStab: %d of %d right-hand sides not converged (%d stopped at the floor of the FP64 true "
@@ -1380,32 +1326,18 @@ static int invert_eo(cvchip_ctx *c, Field &x, const Field &b, double sp, int nit
   const int N = b.nrhs;
   const int64_t Vh = c->lat.V / 2;
   const double mu = c->mu;
-  Field be, bo, xe, xo, bp, y;
+  TmpField be, bo, xe, xo, bp, y;
   int rc = 0;
   Field *hf[6] = {&be, &bo, &xe, &xo, &bp, &y};
   for (int k = 0; k < 5 + (her ? 1 : 0) && !rc; k++) rc = field_alloc(c, *hf[k], N, CVCHIP_PREC_F64, Vh);
-  auto cleanup = [&]() {
-    for (int k = 0; k < 6; k++) field_free(*hf[k]);
-  };
-#define TRY(x)                                                                                   \
-  do {                                                                                           \
-    rc = (x);                                                                                    \
-    if (rc) {                                                                                    \
-      cleanup();                                                                                 \
-      return rc;                                                                                 \
-    }                                                                                            \
-  } while (0)
-  if (rc) {
-    cleanup();
-    return rc;
-  }
-  TRY(eo_split(c, const_cast<Field &>(b), be, bo, 0));
-  TRY(eo_split(c, x, xe, xo, 0));
+  if (rc) return rc;
+  CVC_TRY(eo_split(c, const_cast<Field &>(b), be, bo, 0));
+  CVC_TRY(eo_split(c, x, xe, xo, 0));
   const uint32_t VhN = (uint32_t)(Vh * N);
   const double k2 = 0.5 / c->kappa, dinv = 1.0 / (k2 * k2 + mu * mu);
   hipLaunchKernelGGL(k_diag_inv, dim3((VhN + 255) / 256), dim3(256), 0, c->stream, (double2 *)xe.data,
                      (const double2 *)be.data, VhN, k2, mu, dinv);
-  TRY(dslash_eo(c, bp, xe, &bo, mu, 1, 2, 0.5, 0));      // b'_o = b_o + H_oe A_ee^-1 b_e / 2
+  CVC_TRY(dslash_eo(c, bp, xe, &bo, mu, 1, 2, 0.5, 0));      // b'_o = b_o + H_oe A_ee^-1 b_e / 2
   int ret;
   if (her) {
     hipLaunchKernelGGL(k_g5, dim3((VhN + 255) / 256), dim3(256), 0, c->stream, (double2 *)bp.data, VhN);
@@ -1419,7 +1351,7 @@ static int invert_eo(cvchip_ctx *c, Field &x, const Field &b, double sp, int nit
                                    (flags & CVCHIP_SOLVE_VERBOSE) ? 1 : 0, 1);
     if (ret >= 0 || ret == CVCHIP_ERR_NOCONV) {
       Op m{c, 0, nullptr, 1, &xe};
-      TRY(m.applyM(xo, y, -mu, 1, DOT_NONE, nullptr, nullptr));    // x_o = gamma5 M(-mu) y
+      CVC_TRY(m.applyM(xo, y, -mu, 1, DOT_NONE, nullptr, nullptr));    // x_o = gamma5 M(-mu) y
     }
   } else {
     if (prec == CVCHIP_PREC_F64) ret = bicgstab64(c, xo, bp, sp, niter_max, flags, stats, 0, 1);
@@ -1431,24 +1363,20 @@ static int invert_eo(cvchip_ctx *c, Field &x, const Field &b, double sp, int nit
                                    (flags & CVCHIP_SOLVE_VERBOSE) ? 1 : 0, 1);
   }
   if (ret >= 0 || ret == CVCHIP_ERR_NOCONV) {
-    TRY(dslash_eo(c, xe, xo, &be, mu, 0, 3, 0.5, 0));    // x_e = A_ee^-1 (b_e + H_eo x_o / 2)
-    TRY(eo_split(c, x, xe, xo, 1));
+    CVC_TRY(dslash_eo(c, xe, xo, &be, mu, 0, 3, 0.5, 0));    // x_e = A_ee^-1 (b_e + H_eo x_o / 2)
+    CVC_TRY(eo_split(c, x, xe, xo, 1));
     if (stats) {
       Solve S;
-      Field tmp;
+      TmpField tmp;
       double tr = 0.;
       int rc3 = solve_setup(c, S, N);
       if (!rc3) rc3 = field_alloc(c, tmp, N, CVCHIP_PREC_F64);
       if (!rc3) rc3 = true_residual(S, x, b, tmp, mu, &tr, nullptr);
-      field_free(tmp);
-      solve_free(S);
       if (rc3) ret = rc3;
       stats->true_res2_max = tr;
       stats->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     }
   }
-  cleanup();
-#undef TRY
   return ret;
 }
 
@@ -1468,51 +1396,41 @@ int invert_her_fields(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
     return invert_eo(c, x, b, sp, niter_max, prec, delta, flags, stats, 1);
   }
   auto t0 = std::chrono::steady_clock::now();
-  Field g5b, y;
-  int rc = field_alloc(c, g5b, b.nrhs, CVCHIP_PREC_F64);
-  if (!rc) rc = field_alloc(c, y, b.nrhs, CVCHIP_PREC_F64);
-  if (!rc) {
-    const uint32_t VN = (uint32_t)(b.V * b.nrhs);
-    rc = hipMemcpyAsync(g5b.data, b.data, b.bytes, hipMemcpyDeviceToDevice, c->stream) == hipSuccess ? 0 : CVCHIP_ERR_HIP;
-    if (!rc && hipMemcpyAsync(y.data, x.data, x.bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess) rc = CVCHIP_ERR_HIP;
-    if (!rc) {
-      hipLaunchKernelGGL(k_g5, dim3((VN + 255) / 256), dim3(256), 0, c->stream, (double2 *)g5b.data, VN);
-      if (prec == CVCHIP_PREC_F64) rc = bicgstab64(c, y, g5b, sp, niter_max, flags, stats, 1);
-      else if (!(delta > 0. && delta < 1.)) {
-        set_error("reliable-update factor delta must lie in (0,1), got %g", delta);
-        rc = CVCHIP_ERR_ARG;
-      } else if (prec == CVCHIP_PREC_F32)
-        rc = bicgstab_mixed<IOPlain<float>>(c, y, g5b, sp, niter_max, prec, delta, stats, 1,
-                                            (flags & CVCHIP_SOLVE_VERBOSE) ? 1 : 0);
-      else if (prec == CVCHIP_PREC_F16)
-        rc = bicgstab_mixed<IOHalf>(c, y, g5b, sp, niter_max, prec, delta, stats, 1,
-                                    (flags & CVCHIP_SOLVE_VERBOSE) ? 1 : 0);
-      else {
-        set_error("unknown precision %d", prec);
-        rc = CVCHIP_ERR_ARG;
-      }
-    }
-    // x = gamma5 D(-mu) y, done whether or not the solve converged (invert_Qtm.c:441-446)
-    if (rc >= 0 || rc == CVCHIP_ERR_NOCONV) {
-      const int rc2 = dslash(c, x, y, -c->mu, 1);
-      if (rc2) rc = rc2;
-    }
-    if (stats && (rc >= 0 || rc == CVCHIP_ERR_NOCONV)) {
-      Solve S;
-      double tr = 0.;
-      Field tmp;
-      int rc3 = solve_setup(c, S, b.nrhs);
-      if (!rc3) rc3 = field_alloc(c, tmp, b.nrhs, CVCHIP_PREC_F64);
-      if (!rc3) rc3 = true_residual(S, x, b, tmp, c->mu, &tr, nullptr);
-      field_free(tmp);
-      solve_free(S);
-      if (rc3) rc = rc3;
-      stats->true_res2_max = tr;
-      stats->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    }
+  TmpField g5b, y;
+  CVC_TRY(field_alloc(c, g5b, b.nrhs, CVCHIP_PREC_F64));
+  CVC_TRY(field_alloc(c, y, b.nrhs, CVCHIP_PREC_F64));
+  const uint32_t VN = (uint32_t)(b.V * b.nrhs);
+  CVC_HIP(hipMemcpyAsync(g5b.data, b.data, b.bytes, hipMemcpyDeviceToDevice, c->stream));
+  CVC_HIP(hipMemcpyAsync(y.data, x.data, x.bytes, hipMemcpyDeviceToDevice, c->stream));
+  hipLaunchKernelGGL(k_g5, dim3((VN + 255) / 256), dim3(256), 0, c->stream, (double2 *)g5b.data, VN);
+  int rc;
+  if (prec == CVCHIP_PREC_F64) rc = bicgstab64(c, y, g5b, sp, niter_max, flags, stats, 1);
+  else if (!(delta > 0. && delta < 1.)) {
+    set_error("reliable-update factor delta must lie in (0,1), got %g", delta);
+    rc = CVCHIP_ERR_ARG;
+  } else if (prec == CVCHIP_PREC_F32)
+    rc = bicgstab_mixed<IOPlain<float>>(c, y, g5b, sp, niter_max, prec, delta, stats, 1,
+                                        (flags & CVCHIP_SOLVE_VERBOSE) ? 1 : 0);
+  else if (prec == CVCHIP_PREC_F16)
+    rc = bicgstab_mixed<IOHalf>(c, y, g5b, sp, niter_max, prec, delta, stats, 1,
+                                (flags & CVCHIP_SOLVE_VERBOSE) ? 1 : 0);
+  else {
+    set_error("unknown precision %d", prec);
+    rc = CVCHIP_ERR_ARG;
   }
-  field_free(g5b);
-  field_free(y);
+  if (rc < 0 && rc != CVCHIP_ERR_NOCONV) return rc;
+  // x = gamma5 D(-mu) y, done whether or not the solve converged (invert_Qtm.c:441-446)
+  CVC_TRY(dslash(c, x, y, -c->mu, 1));
+  if (stats) {
+    Solve S;
+    double tr = 0.;
+    TmpField tmp;
+    CVC_TRY(solve_setup(c, S, b.nrhs));
+    CVC_TRY(field_alloc(c, tmp, b.nrhs, CVCHIP_PREC_F64));
+    CVC_TRY(true_residual(S, x, b, tmp, c->mu, &tr, nullptr));
+    stats->true_res2_max = tr;
+    stats->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  }
   return rc;
 }
 
@@ -1575,7 +1493,7 @@ extern "C" int cvchip_invert_Qtm(cvchip_ctx *c, double *x, const double *b, int 
       set_error("NULL argument to cvchip_invert_Qtm");
       return CVCHIP_ERR_NULL;
     }
-    Field fx, fb;
+    TmpField fx, fb;
     int rc = field_alloc(c, fx, nrhs, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, fb, nrhs, CVCHIP_PREC_F64);
     if (!rc) rc = upload_aos(c, fx, x, 0, nrhs);
@@ -1589,8 +1507,6 @@ extern "C" int cvchip_invert_Qtm(cvchip_ctx *c, double *x, const double *b, int 
         if (rc2) ret = rc2;
       }
     }
-    field_free(fx);
-    field_free(fb);
     return ret;
   });
 }
@@ -1603,7 +1519,7 @@ extern "C" int cvchip_invert_Qtm_her(cvchip_ctx *c, double *x, const double *b, 
       set_error("NULL argument to cvchip_invert_Qtm_her");
       return CVCHIP_ERR_NULL;
     }
-    Field fx, fb;
+    TmpField fx, fb;
     int rc = field_alloc(c, fx, nrhs, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, fb, nrhs, CVCHIP_PREC_F64);
     if (!rc) rc = upload_aos(c, fx, x, 0, nrhs);
@@ -1616,15 +1532,13 @@ extern "C" int cvchip_invert_Qtm_her(cvchip_ctx *c, double *x, const double *b, 
         if (rc2) ret = rc2;
       }
     }
-    field_free(fx);
-    field_free(fb);
     return ret;
   });
 }
 
 // spinor_scalar_product_co / _re (invert_Qtm.c:28-84) on host arrays
 static int scalar_product(cvchip_ctx *c, double w[3], const double *xi, const double *phi) {
-  Field a, b;
+  TmpField a, b;
   Solve S;
   int rc = field_alloc(c, a, 1, CVCHIP_PREC_F64);
   if (!rc) rc = field_alloc(c, b, 1, CVCHIP_PREC_F64);
@@ -1642,9 +1556,6 @@ static int scalar_product(cvchip_ctx *c, double w[3], const double *xi, const do
       if (e != hipSuccess) rc = hip_fail(e, "scalar product", __FILE__, __LINE__);
     }
   }
-  solve_free(S);
-  field_free(a);
-  field_free(b);
   return rc;
 }
 

@@ -326,7 +326,7 @@ extern "C" int cvchip_contract_twopoint(cvchip_ctx *c, double *contr, int idsour
       set_error("n_c must be 1..3, got %d", n_c);
       return CVCHIP_ERR_ARG;
     }
-    Field fc, fp;
+    TmpField fc, fp;
     const int N = 4 * n_c;
     int rc = field_alloc(c, fc, N, CVCHIP_PREC_F64);
     if (!rc) rc = field_alloc(c, fp, N, CVCHIP_PREC_F64);
@@ -340,8 +340,6 @@ extern "C" int cvchip_contract_twopoint(cvchip_ctx *c, double *contr, int idsour
       if (!rc) rc = upload_aos(c, fp, phi[k], k, 1);
     }
     if (!rc) rc = twopoint_fields(c, contr, idsource, idsink, fc, fp, n_c, snk_mom, src);
-    field_free(fc);
-    field_free(fp);
     return rc;
   });
 }

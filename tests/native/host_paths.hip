@@ -10,7 +10,9 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <functional>
 #include <map>
+#include <new>
 #include <set>
 #include <string>
 #include <vector>
@@ -34,16 +36,22 @@ std::vector<Launch> launches;
 hipError_t last = hipSuccess;
 long allocs = 0, fail_alloc = 0;               // allocation number that fails (0: none)
 size_t capacity = SIZE_MAX, used = 0;          // device memory
+long calls = 0, fail_call = 0;                 // any runtime call that can fail, allocations among them
+long news = 0, fail_new = 0;                   // the library's host allocations on the main thread
+thread_local bool counted = false;
+struct Own {                                   // the stand-in's own allocations are not counted
+  bool was = counted;
+  Own() { counted = false; }
+  ~Own() { counted = was; }
+};
 
 // convergence that the solver's kernels report
 int conv_it = 3, conv_rhs = 1 << 30;           // columns below conv_rhs converge at iteration conv_it
 
-hipError_t ok_or(bool bad, hipError_t e) {
-  if (bad) last = e;
-  return bad ? e : hipSuccess;
-}
+hipError_t call() { return ++calls == fail_call ? last = hipErrorUnknown : hipSuccess; }
 hipError_t alloc(std::map<void *, size_t> &live, void **p, size_t n) {
-  if (++allocs == fail_alloc || (&live == &dev && n > capacity - used)) return last = hipErrorOutOfMemory;
+  const Own own;
+  if (++calls == fail_call || ++allocs == fail_alloc || (&live == &dev && n > capacity - used)) return last = hipErrorOutOfMemory;
   *p = calloc(n ? n : 1, 1);
   live[*p] = n;
   if (&live == &dev) used += n;
@@ -108,34 +116,42 @@ hipError_t hipGetSymbolAddress(void **p, const void *) {
   return *p = buf, hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+  if (const hipError_t e_ = call()) return e_;
+  const Own own;
   *s = (hipStream_t)malloc(1);
   streams.insert(*s);
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t s) { return streams.erase(s), free(s), hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return call(); }
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return call(); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  if (const hipError_t e_ = call()) return e_;
+  const Own own;
   *e = (hipEvent_t)malloc(1);
   events.insert(*e);
   return hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t e) { return events.erase(e), free(e), hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return call(); }
+hipError_t hipEventSynchronize(hipEvent_t) { return call(); }
 hipError_t hipEventElapsedTime(float *t, hipEvent_t, hipEvent_t) { return *t = 0.f, hipSuccess; }
 // (what kernels alone would use stays zero, so that large sets are never touched)
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) {
+  if (const hipError_t e_ = call()) return e_;
   if (k != hipMemcpyDeviceToDevice) memcpy(d, s, n);
   return hipSuccess;
 }
 hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t) {
+  if (const hipError_t e_ = call()) return e_;
   if (n < (size_t)1 << 20) memset(p, v, n);
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t, hipStream_t) {
+  if (const hipError_t e_ = call()) return e_;
+  const Own own;
   launches.push_back({names()[f], g, b});
   kernel(names()[f], g, a);
   return hipSuccess;
@@ -162,6 +178,15 @@ void __hipRegisterFunction(void **, const void *f, char *, const char *name, uns
 }
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 }
+
+void *operator new(size_t n) {
+  if (counted && ++news == fail_new) throw std::bad_alloc();
+  void *p = malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
 
 // ---------------------------------------------------------------- scenarios
 #define CHECK(cond, ...)                                                \
@@ -232,8 +257,70 @@ static void solver_buffers() {
   }
 }
 
+// Entry points that solve, on small sets; the host arrays are made once.
+struct Entry {
+  const char *name;
+  std::function<int(Ctx &)> call;
+};
+static std::vector<Entry> entries() {
+  static std::vector<double> conn(1 << 16), force(1 << 16), store(1 << 20), b(1 << 14), y(1 << 14);
+  static double contact[8], L, dmu;
+  static double *props[120];
+  static const int src[4] = {1, 0, 1, 2}, mom[3] = {0, 1, 0};
+  for (int k = 0; k < 120; k++) props[k] = &store[4096 * k];
+  std::vector<Entry> v;
+  for (int her = 0; her < 2; her++)
+    for (unsigned f : {0u, CVCHIP_SOLVE_LAGGED, CVCHIP_SOLVE_EO})
+      for (int prec = 0; prec < 3; prec++)
+        v.push_back({her ? "invert_Qtm_her" : "invert_Qtm", [=](Ctx &x) {
+                       cvchip_stats st;
+                       return (her ? cvchip_invert_Qtm_her : cvchip_invert_Qtm)(x.c, y.data(), b.data(), 2, 1e-20, 20, prec,
+                                                                                0.1, f, &st);
+                     }});
+  v.push_back({"Q_phi", [](Ctx &x) { return cvchip_Q_phi(x.c, y.data(), b.data(), 0.1, 0); }});
+  v.push_back({"scalar_product", [](Ctx &x) { return cvchip_scalar_product_co(x.c, contact, y.data(), b.data()); }});
+  v.push_back({"cvc_source", [](Ctx &x) { return cvchip_cvc_source(x.c, conn.data(), contact, src, 1e-20, 20, 0, 0.1, nullptr); }});
+  v.push_back({"cvc_propagators", [](Ctx &x) { return cvchip_cvc_propagators(x.c, props, src, 1e-20, 20, 1, 0.1, nullptr); }});
+  v.push_back({"p2gg_source", [](Ctx &x) {
+                 return cvchip_p2gg_source(x.c, conn.data(), contact, src, 1, 5, mom, 1, 1e-20, 20, 2, 0.1, nullptr);
+               }});
+  v.push_back({"cvc_gradient", [](Ctx &x) {
+                 return cvchip_cvc_gradient(x.c, src, 2., 1e-20, 20, 0, 0.1, &L, &dmu, force.data(), nullptr);
+               }});
+  return v;
+}
+
+// Every entry point with each of its `count`ed events refused in turn: the call ends
+// (an error, or a result where there is another way), the context is as it was, the
+// same call then works, and nothing is left allocated.
+static void refuse_each(long &count, long &fail, const char *what, const std::vector<Entry> &list) {
+  for (const Entry &e : list)
+    for (long k = 1;; k++) {
+      std::string at = std::string(e.name) + ", " + what + " " + std::to_string(k);
+      Ctx x(2, 2, 2, 4);
+      fail = count + k;
+      const int rc = e.call(x);
+      const bool reached = count >= fail;
+      fail = 0;
+      CHECK(reached || rc >= 0, "%s: %d", at.c_str(), rc);
+      CHECK(x.c->mu == 0.01 && !x.c->op_mask && !x.c->red_off, "%s: context changed", at.c_str());
+      CHECK(hipGetLastError() == hipSuccess || rc >= 0, "%s: error left behind (returned %d)", at.c_str(), rc);
+      CHECK(e.call(x) >= 0, "%s: the same call again", at.c_str());
+      launches.clear();
+      if (!reached) break;
+    }
+}
+static void refused_calls() { refuse_each(calls, fail_call, "call", entries()); }
+static void refused_host_memory() {
+  std::vector<Entry> list = entries();
+  list.pop_back();   // (cvc_gradient)
+  counted = true;
+  refuse_each(news, fail_new, "host allocation", list);
+}
+
 int main(int argc, char **argv) {
-  const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers}};
+  const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
+                                                {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();
