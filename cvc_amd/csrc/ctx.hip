@@ -109,9 +109,11 @@ int HostStream::push(void *host, const void *dev, size_t bytes) {
     return copy_to_host(c_, host, dev, bytes);
   }
   if (!c_->copy_stream) {
+    // (an earlier call may have made some of the events; the stream comes last)
     CVC_TRY(ensure_pinned(c_));
-    CVC_HIP(hipEventCreateWithFlags(&c_->copy_after, hipEventDisableTiming));
-    for (auto &e : c_->slot_ev) CVC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (!c_->copy_after) CVC_HIP(hipEventCreateWithFlags(&c_->copy_after, hipEventDisableTiming));
+    for (auto &e : c_->slot_ev)
+      if (!e) CVC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     CVC_HIP(hipStreamCreateWithFlags(&c_->copy_stream, hipStreamNonBlocking));
   }
   if (head_ - tail_ == kSlots) CVC_TRY(drain());

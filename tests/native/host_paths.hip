@@ -293,11 +293,12 @@ static std::vector<Entry> entries() {
 // Every entry point with each of its `count`ed events refused in turn: the call ends
 // (an error, or a result where there is another way), the context is as it was, the
 // same call then works, and nothing is left allocated.
-static void refuse_each(long &count, long &fail, const char *what, const std::vector<Entry> &list) {
+static void refuse_each(long &count, long &fail, const char *what, const std::vector<Entry> &list, int T = 2, int L = 2,
+                        int LZ = 4) {
   for (const Entry &e : list)
     for (long k = 1;; k++) {
       std::string at = std::string(e.name) + ", " + what + " " + std::to_string(k);
-      Ctx x(2, 2, 2, 4);
+      Ctx x(T, L, L, LZ);
       fail = count + k;
       const int rc = e.call(x);
       const bool reached = count >= fail;
@@ -318,9 +319,26 @@ static void refused_host_memory() {
   refuse_each(news, fail_new, "host allocation", list);
 }
 
+// the contraction of a lattice whose conn leaves in pieces (16 MB)
+static void streamed_conn() {
+  static std::vector<double> conn((size_t)32 << 16);
+  static double contact[8];
+  static const int src[4] = {1, 0, 1, 2};
+  refuse_each(calls, fail_call, "call", {{"field_cvc_contract", [](Ctx &x) {
+                cvchip_field *up = nullptr, *dn = nullptr;
+                int rc = cvchip_field_create(x.c, 60, CVCHIP_PREC_F64, &up);
+                if (!rc) rc = cvchip_field_create(x.c, 60, CVCHIP_PREC_F64, &dn);
+                if (!rc) rc = cvchip_field_cvc_contract(x.c, conn.data(), contact, up, dn, src);
+                cvchip_field_destroy(up);
+                cvchip_field_destroy(dn);
+                return rc;
+              }}}, 16, 16, 16);
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
-                                                {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory}};
+                                                {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory},
+                                                {"streamed_conn", streamed_conn}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();
