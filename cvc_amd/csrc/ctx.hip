@@ -118,11 +118,18 @@ int HostStream::push(void *host, const void *dev, size_t bytes) {
   }
   if (head_ - tail_ == kSlots) CVC_TRY(drain());
   const size_t k = head_ % kSlots;
-  CVC_HIP(hipEventRecord(c_->copy_after, c_->stream));
-  CVC_HIP(hipStreamWaitEvent(c_->copy_stream, c_->copy_after, 0));
-  CVC_HIP(hipMemcpyAsync((char *)c_->pin[k / 4] + (k % 4) * kSlotBytes, dev, bytes, hipMemcpyDeviceToHost,
-                         c_->copy_stream));
-  CVC_HIP(hipEventRecord(c_->slot_ev[k], c_->copy_stream));
+  auto enqueue = [&]() -> int {
+    CVC_HIP(hipEventRecord(c_->copy_after, c_->stream));
+    CVC_HIP(hipStreamWaitEvent(c_->copy_stream, c_->copy_after, 0));
+    CVC_HIP(hipMemcpyAsync((char *)c_->pin[k / 4] + (k % 4) * kSlotBytes, dev, bytes, hipMemcpyDeviceToHost,
+                           c_->copy_stream));
+    CVC_HIP(hipEventRecord(c_->slot_ev[k], c_->copy_stream));
+    return 0;
+  };
+  if (const int rc = enqueue()) {
+    unplaced_ = true;
+    return rc;
+  }
   piece_[k] = Piece{host, bytes};
   head_++;
   return 0;
@@ -131,7 +138,11 @@ int HostStream::push(void *host, const void *dev, size_t bytes) {
 int HostStream::drain() {
   const size_t k = tail_ % kSlots;
   tail_++;
-  CVC_HIP(hipEventSynchronize(c_->slot_ev[k]));
+  const hipError_t e = hipEventSynchronize(c_->slot_ev[k]);
+  if (e != hipSuccess) {
+    unplaced_ = true;
+    return hip_fail(e, "piece of a copy to the host", __FILE__, __LINE__);
+  }
   par_memcpy(piece_[k].host, (char *)c_->pin[k / 4] + (k % 4) * kSlotBytes, piece_[k].bytes);
   return 0;
 }
@@ -141,6 +152,10 @@ int HostStream::finish() {
   while (tail_ < head_) {
     const int r = drain();
     if (r && !rc) rc = r;
+  }
+  if (unplaced_) {
+    (void)hipStreamSynchronize(c_->copy_stream);
+    unplaced_ = false;
   }
   return rc;
 }

@@ -221,6 +221,7 @@ class HostStream {
   cvchip_ctx *c_;
   Piece piece_[kSlots];
   size_t head_ = 0, tail_ = 0;   // pieces pushed and placed
+  bool unplaced_ = false;        // a copy may be in flight that no slot's event covers
 };
 // device address of the allocation-free two-point entry point's scratch on
 // `device` (the current device), taken once per device

@@ -28,6 +28,11 @@ std::map<const void *, std::string> &names() {   // kernels by host stub (regist
   static std::map<const void *, std::string> n;
   return n;
 }
+struct Copies {                                // device-to-host copies of a stream
+  long issued = 0, ended = 0;
+};
+std::map<void *, Copies> to_host;
+std::map<void *, std::pair<void *, long>> recorded;   // event: stream, copies issued before it
 struct Launch {
   std::string name;
   dim3 grid, block;
@@ -122,8 +127,13 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
   streams.insert(*s);
   return hipSuccess;
 }
-hipError_t hipStreamDestroy(hipStream_t s) { return streams.erase(s), free(s), hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return call(); }
+hipError_t hipStreamDestroy(hipStream_t s) { return streams.erase(s), to_host.erase(s), free(s), hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (const hipError_t e_ = call()) return e_;
+  const Own own;
+  to_host[s].ended = to_host[s].issued;
+  return hipSuccess;
+}
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return call(); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
@@ -135,12 +145,25 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
 }
 hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t e) { return events.erase(e), free(e), hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return call(); }
-hipError_t hipEventSynchronize(hipEvent_t) { return call(); }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  if (const hipError_t e_ = call()) return e_;
+  const Own own;
+  recorded[e] = {s, to_host[s].issued};
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  if (const hipError_t e_ = call()) return e_;
+  const Own own;
+  const auto r = recorded[e];
+  if (r.second > to_host[r.first].ended) to_host[r.first].ended = r.second;
+  return hipSuccess;
+}
 hipError_t hipEventElapsedTime(float *t, hipEvent_t, hipEvent_t) { return *t = 0.f, hipSuccess; }
 // (what kernels alone would use stays zero, so that large sets are never touched)
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) {
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t q) {
   if (const hipError_t e_ = call()) return e_;
+  const Own own;
+  if (k == hipMemcpyDeviceToHost) to_host[q].issued++;
   if (k != hipMemcpyDeviceToDevice) memcpy(d, s, n);
   return hipSuccess;
 }
@@ -305,6 +328,8 @@ static void refuse_each(long &count, long &fail, const char *what, const std::ve
       fail = 0;
       CHECK(reached || rc >= 0, "%s: %d", at.c_str(), rc);
       CHECK(x.c->mu == 0.01 && !x.c->op_mask && !x.c->red_off, "%s: context changed", at.c_str());
+      const Copies q = x.c->copy_stream ? to_host[x.c->copy_stream] : Copies();
+      CHECK(q.ended == q.issued, "%s: %ld pieces still on their way", at.c_str(), q.issued - q.ended);
       CHECK(hipGetLastError() == hipSuccess || rc >= 0, "%s: error left behind (returned %d)", at.c_str(), rc);
       CHECK(e.call(x) >= 0, "%s: the same call again", at.c_str());
       launches.clear();
