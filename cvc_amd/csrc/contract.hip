@@ -668,24 +668,30 @@ int solve_five_sources(cvchip_ctx *c, Field &out, double mu, const std::function
     }
     return 0;
   };
-  TmpField all, b, x;
-  bool have_all = c->lat.V <= kBatchSites;
-  int rc = 0;
-  if (have_all && field_alloc(c, all, 60, CVCHIP_PREC_F64)) have_all = false;
-  if (have_all) {
-    rc = source(all, 0, 5);
-    if (!rc) rc = solve(out, all, 5);
-  }
-  if (!have_all || rc == CVCHIP_ERR_OOM) {
-    rc = field_alloc(c, b, 12, CVCHIP_PREC_F64);
-    if (!rc) rc = field_alloc(c, x, 12, CVCHIP_PREC_F64);
-    for (int s = 0; s < 5 && !rc; s++) {
-      rc = have_all ? copy_columns(c, b, 0, all, 12 * s, 12) : source(b, s, 1);
-      if (!rc) rc = solve(x, b, 1);
-      if (!rc) rc = copy_columns(c, out, 12 * s, x, 0, 12);
+  int rc = CVCHIP_ERR_OOM;
+  bool held = false;   // out holds the sources (its own columns may have been what source() reads)
+  if (c->lat.V <= kBatchSites) {
+    TmpField all;
+    if (!field_alloc(c, all, 60, CVCHIP_PREC_F64)) {
+      CVC_TRY(source(all, 0, 5));
+      rc = solve(out, all, 5);
+      if (rc == CVCHIP_ERR_OOM) {
+        CVC_HIP(hipMemcpyAsync(out.data, all.data, all.bytes, hipMemcpyDeviceToDevice, c->stream));
+        held = true;
+      }
     }
   }
-  return rc;
+  if (rc != CVCHIP_ERR_OOM) return rc;
+  // one by one, without the room for more than twelve columns
+  TmpField b, x;
+  CVC_TRY(field_alloc(c, b, 12, CVCHIP_PREC_F64));
+  CVC_TRY(field_alloc(c, x, 12, CVCHIP_PREC_F64));
+  for (int s = 0; s < 5; s++) {
+    CVC_TRY(held ? copy_columns(c, b, 0, out, 12 * s, 12) : source(b, s, 1));
+    CVC_TRY(solve(x, b, 1));
+    CVC_TRY(copy_columns(c, out, 12 * s, x, 0, 12));
+  }
+  return 0;
 }
 
 // 5 x 12 up (mu) and 5 x 12 down (-mu) propagators from point sources at y + s^

@@ -36,6 +36,7 @@ std::map<void *, std::pair<void *, long>> recorded;   // event: stream, copies i
 struct Launch {
   std::string name;
   dim3 grid, block;
+  std::vector<uint32_t> cols;                  // k_copy_columns: columns of both sets, first ones, count
 };
 std::vector<Launch> launches;
 hipError_t last = hipSuccess;
@@ -175,7 +176,9 @@ hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t) {
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t, hipStream_t) {
   if (const hipError_t e_ = call()) return e_;
   const Own own;
-  launches.push_back({names()[f], g, b});
+  launches.push_back({names()[f], g, b, {}});
+  if (names()[f].find("k_copy_columns") != std::string::npos)
+    for (int k = 3; k < 8; k++) launches.back().cols.push_back(arg<uint32_t>(a, k));
   kernel(names()[f], g, a);
   return hipSuccess;
 }
@@ -360,10 +363,37 @@ static void streamed_conn() {
               }}}, 16, 16, 16);
 }
 
+// A whole source on a device that holds the twelve-column solves but not the sixty-column
+// ones: the sources are solved one by one, and that takes no more memory than if the
+// larger solve had not been tried.
+static void one_by_one() {
+  static std::vector<double> conn(32 << 12);
+  static double contact[8];
+  static const int src[4] = {1, 0, 1, 2};
+  const size_t set12 = (size_t)2304 * 4096, set60 = 5 * set12;
+  // up and dn, b and x, the hermitian solver's nine sets; the links, scratch
+  const size_t enough = 2 * set60 + 11 * set12 + ((size_t)14 << 20);
+  Ctx x(8, 8, 8, 8);
+  capacity = enough;
+  launches.clear();
+  const int rc = cvchip_cvc_source(x.c, conn.data(), contact, src, 1e-20, 20, 0, 0.1, nullptr);
+  capacity = SIZE_MAX;
+  CHECK(rc >= 0, "whole source: %d", rc);
+  int k = 0;
+  for (const Launch &l : launches) {
+    if (l.cols.empty()) continue;
+    const uint32_t s = 12u * (uint32_t)(k / 2 % 5);
+    const std::vector<uint32_t> in = {12, 60, 0, s, 12}, out = {60, 12, s, 0, 12};
+    CHECK(l.cols == (k % 2 ? out : in), "copy of columns %d", k);
+    k++;
+  }
+  CHECK(k == 20, "%d copies of columns", k);
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
                                                 {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory},
-                                                {"streamed_conn", streamed_conn}};
+                                                {"streamed_conn", streamed_conn}, {"one_by_one", one_by_one}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();
