@@ -655,18 +655,22 @@ int solve_five_sources(cvchip_ctx *c, Field &out, double mu, const std::function
       c->mu = mu;
       rc = invert_her_fields(c, x, b, sp, niter_max, prec, delta, 0, &st);
     }
-    if (rc < 0) return rc;
-    if (tot) {
-      // the iterations of 12 columns are those of the slowest of them
-      for (int k = 0; k < ns; k++)
-        tot->iterations += *std::max_element(c->col_iters.begin() + 12 * k, c->col_iters.begin() + 12 * (k + 1));
-      tot->converged += st.converged;
+    if (rc < 0 && rc != CVCHIP_ERR_NOCONV) return rc;
+    // the sources before the first that did not converge count, as if solved in turn
+    int good = 0;
+    for (; good < ns; good++) {
+      const auto it = c->col_iters.begin() + 12 * good;
+      if (*std::min_element(it, it + 12) < 0) break;
+      if (tot) tot->iterations += *std::max_element(it, it + 12);   // of the slowest of 12 columns
+    }
+    if (tot && good) {
+      tot->converged += 12 * good;
       tot->reliable_updates += st.reliable_updates;
       tot->dslash_calls += st.dslash_calls;
       tot->seconds += st.seconds;
-      if (st.true_res2_max > tot->true_res2_max) tot->true_res2_max = st.true_res2_max;
+      if (good == ns && st.true_res2_max > tot->true_res2_max) tot->true_res2_max = st.true_res2_max;
     }
-    return 0;
+    return rc < 0 ? rc : 0;
   };
   int rc = CVCHIP_ERR_OOM;
   bool held = false;   // out holds the sources (its own columns may have been what source() reads)

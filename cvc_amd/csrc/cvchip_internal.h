@@ -164,7 +164,8 @@ struct cvchip_ctx {
   // right-hand side r has converged); the operator skips those rhs
   const int *op_mask = nullptr;
   int op_mask_stride = 0;
-  // iterations of each right-hand side of the last solve (0: an exact start vector)
+  // iterations of each right-hand side of the last solve (0: an exact start vector,
+  // -1: not converged)
   std::vector<int> col_iters;
   cvchip::SolveBuffers solve_bufs;
   // traversals already planned, by policy, rhs count, lattice half and precision

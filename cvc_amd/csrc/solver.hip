@@ -938,12 +938,12 @@ int gamma5_inplace(cvchip_ctx *c, Field &f) {
   return 0;
 }
 
-// per right-hand side, as stats->iterations counts them
+// per right-hand side, as stats->iterations counts them; -1: not converged
 static void record_iterations(Solve &S, int iters) {
   S.c->col_iters.resize(S.N);
   for (int r = 0; r < S.N; r++) {
     const RhsState &h = S.hst[r];
-    S.c->col_iters[r] = iters == 0 ? 0 : h.done ? h.iter + 1 : iters;
+    S.c->col_iters[r] = iters == 0 ? 0 : h.done && !h.stalled ? h.iter + 1 : -1;
   }
 }
 

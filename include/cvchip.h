@@ -60,6 +60,12 @@ typedef struct {
   double true_res2_max;     /* max over rhs of |D x - b|^2 / |b|^2, in FP64                 */
   double seconds;           /* wall time inside the call                                   */
 } cvchip_stats;
+/* Calls that solve several sources (cvchip_cvc_source, cvchip_cvc_propagators,
+ * cvchip_p2gg_source, cvchip_cvc_gradient) sum over their solves: iterations as if
+ * every source (12 right-hand sides) were solved by itself, reliable_updates and
+ * dslash_calls per solve made, which on lattices of up to 131072 sites takes five
+ * sources (60 right-hand sides) together.  When such a call returns -3, the sums
+ * cover the sources before the one that did not converge. */
 
 /* ------------------------------------------------------------ context */
 

@@ -145,7 +145,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
   return hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t *e) { return hipEventCreateWithFlags(e, 0); }
-hipError_t hipEventDestroy(hipEvent_t e) { return events.erase(e), free(e), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return events.erase(e), recorded.erase(e), free(e), hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   if (const hipError_t e_ = call()) return e_;
   const Own own;
@@ -390,10 +390,31 @@ static void one_by_one() {
   CHECK(k == 20, "%d copies of columns", k);
 }
 
+// A whole source whose third set of twelve does not converge: the statistics cover the
+// two before it.
+static void unconverged_source() {
+  static std::vector<double> conn(32 << 6);
+  static double contact[8];
+  static const int src[4] = {1, 0, 1, 2};
+  for (int prec = 0; prec < 3; prec++) {
+    Ctx x(4, 2, 2, 4);
+    cvchip_stats st;
+    CHECK(cvchip_cvc_source(x.c, conn.data(), contact, src, 1e-20, 20, prec, 0.1, &st) >= 0, "converging source");
+    CHECK(st.converged == 120 && st.iterations == 10 * (conv_it + 1), "%d, %d iterations", st.converged, st.iterations);
+    conv_rhs = 30;   // of each solve's sixty
+    const int rc = cvchip_cvc_source(x.c, conn.data(), contact, src, 1e-20, 20, prec, 0.1, &st);
+    conv_rhs = 1 << 30;
+    CHECK(rc == CVCHIP_ERR_NOCONV, "%d", rc);
+    CHECK(st.converged == 24 && st.iterations == 2 * (conv_it + 1) && st.dslash_calls > 0, "%d converged, %d iterations, %d applications",
+          st.converged, st.iterations, st.dslash_calls);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
                                                 {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory},
-                                                {"streamed_conn", streamed_conn}, {"one_by_one", one_by_one}};
+                                                {"streamed_conn", streamed_conn}, {"one_by_one", one_by_one},
+                                                {"unconverged_source", unconverged_source}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();
