@@ -982,13 +982,13 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
   // p2 = A p and alpha
   auto advance = [&]() -> int {
     CVC_TRY(op.apply(p2, p, DOT_R2, &r2, &nb));
+    dcalls++;
     return scalar_rows(S, nb, 2, [&](const double *q, int n) {
       hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
     });
   };
   if (!all_done) {
     CVC_TRY(advance());
-    dcalls++;
     for (int it = 0; it <= niter_max; it++) {
       // a lagged solve needs |r1|^2 before x moves, so it keeps the separate passes
       if (lagged)
@@ -1030,7 +1030,6 @@ static int bicgstab64(cvchip_ctx *c, Field &x, const Field &b, double sp, int ni
           printf("# [%d] residuum after iteration %d: %25.16e\n", r, it, S.mir[r].norm);
       if (all_done) break;
       if (!ahead) CVC_TRY(advance());
-      dcalls++;
     }
   }
   CVC_TRY(pull_state(S));
@@ -1124,13 +1123,13 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
   // p2 = A p and alpha (of the rhs that do not hold their p2)
   auto advance = [&]() -> int {
     CVC_TRY(opl.apply(p2, p, DOT_R2, &r2, &nb));
+    dcalls++;
     return scalar_rows(S, nb, 2, [&](const double *q, int n) {
       hipLaunchKernelGGL(k_sc_alpha, dim3(N), dim3(kScThreads), 0, c->stream, S.st, q, n, N);
     });
   };
   if (!all_done) {
     CVC_TRY(advance());
-    dcalls++;
     for (int it = 0; it <= niter_max; it++) {
       hipLaunchKernelGGL((k_s_update<IO>), dim3(S.nblk), dim3(S.B), 0, c->stream, is, ir1, ip2, S.st, S.VN, N, S.nt,
                          ir1, nullptr);
@@ -1206,7 +1205,6 @@ static int bicgstab_mixed(cvchip_ctx *c, Field &x, const Field &b, double sp, in
       }
       if (all_done) break;
       if (!ahead || any_upd) CVC_TRY(advance());
-      dcalls++;
     }
   }
   CVC_TRY(pull_state(S));

@@ -410,11 +410,27 @@ static void unconverged_source() {
   }
 }
 
+// dslash_calls is the number of operator applications launched: on small lattices one of
+// them goes out before the test that ends the solve, one more before a reliable update.
+static void counted_applications() {
+  for (int prec = 0; prec < 3; prec++) {
+    Ctx x(4, 2, 2, 4);
+    cvchip_stats st;
+    launches.clear();
+    CHECK(solve(x, 2, prec, 0, &st, false) >= 0, "solve");
+    int n = 0;
+    for (const Launch &l : launches) n += l.name.find("k_dslash") != std::string::npos;
+    CHECK(n > 2 * st.iterations && st.dslash_calls == n, "precision %d: %d of %d applications counted", prec,
+          st.dslash_calls, n);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
                                                 {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory},
                                                 {"streamed_conn", streamed_conn}, {"one_by_one", one_by_one},
-                                                {"unconverged_source", unconverged_source}};
+                                                {"unconverged_source", unconverged_source},
+                                                {"counted_applications", counted_applications}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();

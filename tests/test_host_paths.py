@@ -38,7 +38,8 @@ def host_paths(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["scratch", "solver_buffers", "refused_calls", "refused_host_memory", "streamed_conn", "one_by_one", "unconverged_source"])
+@pytest.mark.parametrize("scenario", ["scratch", "solver_buffers", "refused_calls", "refused_host_memory", "streamed_conn", "one_by_one", "unconverged_source",
+                                      "counted_applications"])
 def test_host_path(host_paths, scenario):
     r = subprocess.run([str(host_paths), scenario], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
