@@ -1109,15 +1109,16 @@ static uint32_t op_sites(int N, uint32_t len, int64_t V) {
 // 1.5 MB and 0.3, 4-6 % at 1.2 and 2.4 MB.  1.8 MB against 1.5 MB, FP64: whole lattice, 48
 // rhs 64x32^3 14.7 / 16.5 ms (2 x 4 columns), 24 rhs 7.06 / 7.27 ms, 24 rhs 40x20^3 1.02 /
 // 1.09 ms, but even/odd, 12 rhs 40x20^3, 285 / 265 us.
+// bx and yb that the policy gives (not 0) stay; only the other is chosen.
 static void best_columns(const Lattice &L, int N, int K, bool eo, uint32_t &bx, uint32_t &yb) {
   const double site = 12. * 16 / K * N;   // bytes of a site's spinors
   const double budget = eo ? 1.5e6 : 1.8e6, hw = 0.3;   // even/odd forms stream own spinors too
   double best = 0.;
-  bx = yb = 1;
+  const uint32_t bx0 = bx, yb0 = yb;
   for (int cx = 1; cx <= L.LX; cx++) {
-    if (L.LX % cx) continue;
+    if (L.LX % cx || (bx0 && (uint32_t)cx != bx0)) continue;
     for (int cy = 1; cy <= L.LY; cy++) {
-      if (L.LY % cy) continue;
+      if (L.LY % cy || (yb0 && (uint32_t)cy != yb0)) continue;
       const uint32_t len = (uint32_t)(cy * L.LZ), S = op_sites(N, len, L.V);
       const double pad = (double)((len + S - 1) / S * S) / len;
       const double npair = (double)(L.LX / cx) * (L.LY / cy) * L.T, npx = ceil(npair / kXcds);
@@ -1135,9 +1136,9 @@ static void best_columns(const Lattice &L, int N, int K, bool eo, uint32_t &bx, 
 }
 
 // Block-to-site mapping; the policy's bits 4-7 pick the mode (0: automatic),
-// bits 8-15 the y-block height of modes 2, 4 and 5 (0: automatic), bits 20-23
-// the columns' x extent of mode 4 (0: 4 or 1; its t extent in bits 16-19 does not
-// change the order); for mode 5, bits 16-19 are log2 of the column's z extent
+// bits 8-15 the y-block height of modes 2, 4 and 5 and of the automatic columns (0:
+// automatic), bits 20-23 the x extent of mode 4's and the automatic columns (0: 4 or
+// 1 in mode 4; its t extent in bits 16-19 does not change the order); for mode 5, bits 16-19 are log2 of the column's z extent
 // (0: 8) and bits 20-23 its x extent (0: 4).
 // Automatic: N >= 8 the columns of best_columns; below, XCD chunks of a slice
 // (one rhs at 64x32^3: 0.46 ms against 0.51-0.57 ms for the other traversals).

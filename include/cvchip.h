@@ -101,7 +101,7 @@ int cvchip_ctx_set_solver_flags(cvchip_ctx *ctx, unsigned flags);
  * 8 KiB units (caps the resident blocks).  Default 5: links in LDS,
  * streaming stores, automatic traversal (for N >= 8 traversal 4 with the divisors
  * bx of LX and yb of LY whose cross-section's spinors fit an XCD's L2 beside what
- * streams through; for the FP32 operator with 8 <= N <= 16 on sets of 2 GiB and more,
+ * streams through, or with those that bits 8-15 and 20-23 give; for the FP32 operator with 8 <= N <= 16 on sets of 2 GiB and more,
  * LX and LY multiples of 8, the t march over 4 slices in patches of 8x8
  * columns).  The operator output
  * does not depend on the traversal up to rounding (the t march sums the

@@ -17,6 +17,7 @@
 #include <string>
 #include <vector>
 
+#include "../../cvc_amd/csrc/dslash.hip"
 #include "../../cvc_amd/csrc/solver.hip"
 
 namespace fake {
@@ -425,12 +426,30 @@ static void counted_applications() {
   }
 }
 
+// The automatic columns of the multi-rhs operator keep the extents that a caller gives in
+// bits 8-15 and 20-23 of the policy.
+static void column_extents() {
+  using namespace cvchip;
+  Ctx x(8, 12, 12, 8);
+  for (int eo = 0; eo < 2; eo++)
+    for (int K : {1, 2, 4})
+      for (int N : {8, 12, 48})
+        for (int yb : {0, 1, 2, 6, 12})
+          for (int bx : {0, 1, 3, 12}) {
+            CHECK(!cvchip_ctx_set_dslash_policy(x.c, 5 | yb << 8 | bx << 20), "policy");
+            const Traversal t = plan_traversal(x.c, N, eo, K);
+            CHECK(t.mode == 4 && (!yb || t.yb == (unsigned)yb) && (!bx || t.bx == (unsigned)bx),
+                  "N %d, yb %d, bx %d: mode %d, columns %u x %u", N, yb, bx, t.mode, t.bx, t.yb);
+          }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
                                                 {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory},
                                                 {"streamed_conn", streamed_conn}, {"one_by_one", one_by_one},
                                                 {"unconverged_source", unconverged_source},
-                                                {"counted_applications", counted_applications}};
+                                                {"counted_applications", counted_applications},
+                                                {"column_extents", column_extents}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();

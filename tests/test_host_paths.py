@@ -18,11 +18,13 @@ def host_paths(tmp_path_factory):
         pytest.skip("hipcc is not available")
     d = tmp_path_factory.mktemp("host_paths")
     csrc = os.path.join(ROOT, "cvc_amd", "csrc")
-    srcs = [s for s in glob.glob(os.path.join(csrc, "*.hip")) if os.path.basename(s) != "solver.hip"]   # part of the program
+    part = ("dslash.hip", "solver.hip")   # included by the program
+    srcs = [s for s in glob.glob(os.path.join(csrc, "*.hip")) if os.path.basename(s) not in part]
     srcs.append(os.path.join(ROOT, "tests", "native", "host_paths.hip"))
     objs = [str(d / (os.path.basename(s) + ".o")) for s in srcs]
-    procs = [subprocess.Popen([HIPCC, "--cuda-host-only", "-O1", "-g", "-std=c++17", "-fPIC", f"-I{ROOT}/include", "-c", s, "-o", o],
-                              stdout=subprocess.PIPE, stderr=subprocess.STDOUT) for s, o in zip(srcs, objs)]
+    flags = ["--cuda-host-only", "-O1", "-g", "-std=c++17", "-fPIC", f"-I{ROOT}/include"]
+    procs = [subprocess.Popen([HIPCC, *flags, "-c", s, "-o", o], stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+             for s, o in zip(srcs, objs)]
     for p in procs:
         out = p.communicate(timeout=300)[0].decode(errors="replace")
         assert p.returncode == 0, out[-3000:]
@@ -33,13 +35,15 @@ def host_paths(tmp_path_factory):
     exe = d / "host_paths"
     r = subprocess.run(["gcc", "-c", str(stub), "-o", str(d / "device_code.o")], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
-    r = subprocess.run(["g++", *objs, str(d / "device_code.o"), "-o", str(exe), "-lpthread"], capture_output=True, text=True)
+    r = subprocess.run(["g++", *objs, str(d / "device_code.o"), "-o", str(exe), "-lpthread"], capture_output=True,
+                       text=True)
     assert r.returncode == 0, r.stderr[-3000:]
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["scratch", "solver_buffers", "refused_calls", "refused_host_memory", "streamed_conn", "one_by_one", "unconverged_source",
-                                      "counted_applications"])
+@pytest.mark.parametrize("scenario", ["scratch", "solver_buffers", "refused_calls", "refused_host_memory",
+                                      "streamed_conn", "one_by_one", "unconverged_source", "counted_applications",
+                                      "column_extents"])
 def test_host_path(host_paths, scenario):
     r = subprocess.run([str(host_paths), scenario], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
