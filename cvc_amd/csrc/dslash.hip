@@ -1078,15 +1078,20 @@ static bool march_geometry(const cvchip_ctx *c, int N, Traversal &t, bool explic
 
 
 // Sites per operator block for runs of len of a lattice's V sites: at most
-// launch_block's, the count that pads the run least, and among equals the largest whose
-// S N is a multiple of 8, so that a block's stores begin and end on 128-byte
-// lines (a line shared by two blocks is written twice, in halves).
+// launch_block's, the count that costs the run least, in lanes: the padded sites', a
+// quarter of those that idle in a block's last wave, half a site for each block
+// (its prologue), and a thirty-second where S N is not a multiple of 8, so that
+// a block's stores do not begin and end on 128-byte lines (a line shared by two blocks
+// is written twice, in halves).  36 rhs, FP16: 7 sites (252 lanes) 201 us at 32x16^3,
+// 3115 us at 64x32^3; 4 sites (144 lanes), the choice without the idle lanes, 220-230
+// and 3400-3500 us.  Twenty counts from 8 to 96 on eight lattices, geometric mean of
+// the former over the present time: FP64 1.012, FP32 1.008, FP16 1.020.
 static uint32_t op_sites(int N, uint32_t len, int64_t V) {
   const uint32_t S0 = (uint32_t)(launch_block(V, N) / N);
   if (N < 8) return S0;   // links from memory: blocks of 256 threads win although their last one is padded more
-  auto cost = [&](uint32_t S) {   // padded sites, and the halved lines as sites
-    const uint64_t nb = (len + S - 1) / S;
-    return 16 * nb * S + (S * (uint32_t)N % 8 ? nb * S / 2 + 16 : 0);
+  auto cost = [&](uint32_t S) {   // in 1/16 lanes
+    const uint64_t nb = (len + S - 1) / S, used = S * (uint64_t)N, lanes = (used + 63) / 64 * 64;
+    return nb * (12 * used + 4 * lanes + 8 * N) + (used % 8 ? nb * used / 2 + 16 * N : 0);
   };
   uint32_t best = S0;
   for (uint32_t S = S0; S > 0 && 2 * S >= S0; S--)

@@ -443,13 +443,29 @@ static void column_extents() {
           }
 }
 
+// The multi-rhs operator's blocks waste few lanes: over the sites of a run, at most a
+// quarter more than the least that any count from half a full block up takes.
+static void block_lanes() {
+  using namespace cvchip;
+  for (uint32_t N = 8; N <= 128; N++)
+    for (uint32_t len : {64, 96, 120, 128, 160, 192, 198, 255, 256, 285, 324, 396, 400, 512, 576, 1024}) {
+      auto lanes = [&](uint32_t S) { return (len + S - 1) / S * ((S * N + 63) / 64 * 64); };
+      const uint32_t full = 256 / N, S = op_sites((int)N, len, 1 << 24);
+      uint32_t least = ~0u;
+      for (uint32_t s = (full + 1) / 2; s <= full; s++) least = std::min(least, lanes(s));
+      CHECK(S >= 1 && S <= full && 4 * lanes(S) <= 5 * least, "N %u, run of %u: %u sites, %u lanes, not %u", N, len, S,
+            lanes(S), least);
+    }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
                                                 {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory},
                                                 {"streamed_conn", streamed_conn}, {"one_by_one", one_by_one},
                                                 {"unconverged_source", unconverged_source},
                                                 {"counted_applications", counted_applications},
-                                                {"column_extents", column_extents}};
+                                                {"column_extents", column_extents},
+                                                {"block_lanes", block_lanes}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();
