@@ -1148,11 +1148,15 @@ static void best_columns(const Lattice &L, int N, int K, bool eo, uint32_t &bx, 
 // Automatic: N >= 8 the columns of best_columns; below, XCD chunks of a slice
 // (one rhs at 64x32^3: 0.46 ms against 0.51-0.57 ms for the other traversals).
 // K: complexes per 16 bytes of the operator's spinors (1 FP64, 2 FP32, 4
-// FP16+norm).  The FP32 operator on the whole lattice marches in t (mode 6,
-// marches of 4 slices) where a set of up to 16 rhs is 2 GiB or more: 1.73 ms
-// against 1.87 ms for the columns at 64x32^3 with 12 rhs; on smaller lattices the
-// columns win (40x20^3 285 against 431 us, 32x16^3 110 against 139 us, 32^4 with
-// 20 rhs 1.54 against 1.56 ms).
+// FP16+norm).  The FP32 operator of 8 to 20 rhs on the whole lattice marches in t
+// (mode 6, marches of 4 slices) where the 8 x 8 patches of a cross-section divide
+// among the XCDs and a set is 256 MB or more: 12 rhs 32^4 845 against 940 us for the
+// columns, 64x32^3 1.68 against 1.87 ms, 32x32x16^2 (302 MB) 211 against 219 us; over
+// 8, 10, 12, 13, 16, 18 and 20 rhs on such lattices the columns take 1.03 times as
+// long (0.90 to 1.14).  Below 256 MB the columns win (16x32x16^2, 12 rhs, 151 MB: 80
+// against 90 us), and where the XCDs share patches unevenly (40x20^3, 12 rhs, 261
+// against 431 us; 20x40^3, 25 patches, 12 rhs, 1.47 GB, 1.14 against 1.63 ms; 48x24^3, 9
+// patches, 0.58 against 0.85 ms).
 static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
   Lattice L = c->lat;
   if (eo) {   // the half lattice of one parity: LZ/2 half-sites per z line
@@ -1166,8 +1170,8 @@ static Traversal plan_traversal(const cvchip_ctx *c, int N, bool eo, int K) {
     if (!eo && march_geometry(c, N, t, true, 16)) return t;
     want = 4;   // the even/odd operator does not march
   }
-  if (want == 0 && K == 2 && !eo && N >= 8 && N <= 16 && (uint64_t)V * N * 96 >= ((uint64_t)1 << 31) &&
-      L.LX % 8 == 0 && L.LY % 8 == 0) {
+  if (want == 0 && K == 2 && !eo && N >= 8 && N <= 20 && (uint64_t)V * N * 96 >= ((uint64_t)1 << 28) &&
+      L.LX % 8 == 0 && L.LY % 8 == 0 && L.LX / 8 * (L.LY / 8) % (int)kXcds == 0) {
     Traversal t{};
     if (march_geometry(c, N, t, false, 4)) return t;
   }

@@ -101,9 +101,9 @@ int cvchip_ctx_set_solver_flags(cvchip_ctx *ctx, unsigned flags);
  * 8 KiB units (caps the resident blocks).  Default 5: links in LDS,
  * streaming stores, automatic traversal (for N >= 8 traversal 4 with the divisors
  * bx of LX and yb of LY whose cross-section's spinors fit an XCD's L2 beside what
- * streams through, or with those that bits 8-15 and 20-23 give; for the FP32 operator with 8 <= N <= 16 on sets of 2 GiB and more,
- * LX and LY multiples of 8, the t march over 4 slices in patches of 8x8
- * columns).  The operator output
+ * streams through, or with those that bits 8-15 and 20-23 give; for the FP32 operator with 8 <= N <= 20 on sets of 256 MB and
+ * more, LX and LY multiples of 8 and LX LY one of 512, the t march over 4 slices
+ * in patches of 8x8 columns).  The operator output
  * does not depend on the traversal up to rounding (the t march sums the
  * diagonal term first); the fused dot products of the solvers differ at
  * rounding level. */

@@ -458,6 +458,26 @@ static void block_lanes() {
     }
 }
 
+// The FP32 operator marches in t where the XCDs share its patches evenly and its sets do
+// not stay in the caches.
+static void march_rule() {
+  using namespace cvchip;
+  struct Case {
+    int T, LX, LY, LZ, N, K, march;
+  };
+  for (const Case &k : {Case{32, 32, 32, 32, 12, 2, 1}, {64, 32, 32, 32, 8, 2, 1}, {32, 32, 16, 16, 20, 2, 1},
+                        {24, 32, 32, 20, 16, 2, 1}, {18, 16, 32, 18, 20, 2, 1}, {16, 32, 16, 16, 20, 2, 0},
+                        {64, 48, 48, 48, 12, 2, 0}, {20, 40, 40, 40, 16, 2, 0}, {32, 36, 32, 32, 12, 2, 0},
+                        {32, 32, 32, 32, 24, 2, 0}, {64, 32, 32, 32, 7, 2, 0}, {64, 32, 32, 32, 12, 1, 0},
+                        {64, 32, 32, 32, 12, 4, 0}}) {
+    cvchip_ctx c;
+    c.lat = Lattice{k.T, k.LX, k.LY, k.LZ, (int64_t)k.T * k.LX * k.LY * k.LZ};
+    const Traversal t = plan_traversal(&c, k.N, false, k.K);
+    CHECK((t.mode == 6) == (k.march == 1), "%d %d %d %d, %d rhs, K %d: mode %d", k.T, k.LX, k.LY, k.LZ, k.N, k.K, t.mode);
+    CHECK(plan_traversal(&c, k.N, true, k.K).mode != 6, "even/odd");
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> all = {{"scratch", scratch}, {"solver_buffers", solver_buffers},
                                                 {"refused_calls", refused_calls}, {"refused_host_memory", refused_host_memory},
@@ -465,7 +485,7 @@ int main(int argc, char **argv) {
                                                 {"unconverged_source", unconverged_source},
                                                 {"counted_applications", counted_applications},
                                                 {"column_extents", column_extents},
-                                                {"block_lanes", block_lanes}};
+                                                {"block_lanes", block_lanes}, {"march_rule", march_rule}};
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;
   it->second();

@@ -43,7 +43,7 @@ def host_paths(tmp_path_factory):
 
 @pytest.mark.parametrize("scenario", ["scratch", "solver_buffers", "refused_calls", "refused_host_memory",
                                       "streamed_conn", "one_by_one", "unconverged_source", "counted_applications",
-                                      "column_extents", "block_lanes"])
+                                      "column_extents", "block_lanes", "march_rule"])
 def test_host_path(host_paths, scenario):
     r = subprocess.run([str(host_paths), scenario], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
