@@ -322,8 +322,10 @@ int launch_psi(cvchip_ctx *c, double2 *psi, const Field &dn, const SrcLinks &L, 
 
 // Sites of a slab: enough blocks for several rounds of the chip, and pieces of conn
 // (8 MB) that the host copies while the next slabs are computed.  The whole
-// contraction at 40x20^3: 13.9 ms with 24-column Psi fields per nu and one copy at
-// the end; with this, 6.1 ms at 32000 and 64000 sites, 8.1 ms at 8000.
+// contraction with 8000 / 16000 / 32000 / 64000 sites at least: 32x16^3 3.08 / 2.74 /
+// 2.76 / 2.98 ms, 40x20^3 8.04 / 6.34 / 6.10 / 6.16, 96x12^3 3.62 / 3.36 / 3.19 / 4.54,
+// 20x30x18x22 5.03 / 4.78 / 4.64 / 6.68, 48x24^3 12.9 / 12.5 / 13.0 / 18.4 (13.9 ms at
+// 40x20^3 with 24-column Psi fields per nu and one copy at the end).
 constexpr uint32_t kSlabSites = 32000;
 
 // conn (host [V][16][2]) and contact from device up / dn sets of 60 columns
@@ -347,9 +349,9 @@ int contract_fields(cvchip_ctx *c, double *conn, double contact[8], const Field 
   uint32_t *dysp = nullptr;
   int rc = 0;
   auto fail = [&](hipError_t e, const char *w) { return hip_fail(e, w, __FILE__, __LINE__); };
-  // Slabs of nt time slices: the combined columns of a slab and of the slice after
-  // it (18 KB a site) are formed, contracted while they are still in the 256 MB MALL
-  // where the slices are that small, and overwritten by the next slab's.
+  // Slabs of nt time slices: the combined columns of a slab and of the slice after it
+  // (18 KB a site, 737 MB at 40x20^3: they go through HBM, not the 256 MB MALL) are
+  // formed, contracted, and overwritten by the next slab's.
   const uint32_t T = (uint32_t)c->lat.T, slice = V / T;
   const uint32_t nt = std::min(T, (kSlabSites + slice - 1) / slice);
   Slab B{nullptr, slice, nt == T ? T : nt + 1};

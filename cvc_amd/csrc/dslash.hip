@@ -446,7 +446,11 @@ __device__ __forceinline__ void hop_pipelined(cplx<typename IO::real> acc[12], R
 // second wave instead: FP32 bounded after three hops (48x24^3, 2 / 4 / 6 rhs: 136 /
 // 232 / 346 us against 142 / 243 / 363 us unbounded; one rhs 72 against 66 us), FP64
 // after three and six (48x24^3, 1 / 2 / 4 / 7 rhs: 185 / 265 / 444 / 752 us, after four
-// hops at one wave 166 / 262 / 473 / 892 us, unbounded 169 / 265 / 481 / 880 us).
+// hops at one wave 166 / 262 / 473 / 892 us, unbounded 169 / 265 / 481 / 880 us).  These
+// are the whole-lattice kernels, none of which spills; the bounds were not measured on
+// the even/odd ones, which do: FP32 127-156 registers with one rhs (616 B of
+// scratch) and 3-32 with more, FP16 50-103, FP64 21-76 from three rhs (up to 10
+// below).
 template <typename IO, int RECON, int H, bool LDSL, bool LDSS, bool EO, bool FEW>
 __device__ __forceinline__ void hop_plain(cplx<typename IO::real> acc[12], const NbLoader<IO, LDSS> &ld,
                                           const cplx<typename IO::real> *__restrict__ U,
@@ -463,8 +467,8 @@ __device__ __forceinline__ void hop_plain(cplx<typename IO::real> acc[12], const
 
 // Minimum resident waves per SIMD the register allocation must allow (the
 // compiler otherwise hoists every neighbour load and ends at one wave).  Links from
-// memory (few rhs) in FP32 and FP16: two, at three the FP32 kernel spills (48x24^3,
-// one / six rhs: 96 / 472 us against 66 / 346 us).
+// memory (few rhs) in FP32 and FP16: two, at three the whole-lattice FP32 kernel
+// spills (48x24^3, one / six rhs: 96 / 472 us against 66 / 346 us).
 #ifndef CVC_DSLASH_WAVES64
 #define CVC_DSLASH_WAVES64 1
 #endif
@@ -1145,8 +1149,9 @@ static void best_columns(const Lattice &L, int N, int K, bool eo, uint32_t &bx, 
 // automatic), bits 20-23 the x extent of mode 4's and the automatic columns (0: 4 or
 // 1 in mode 4; its t extent in bits 16-19 does not change the order); for mode 5, bits 16-19 are log2 of the column's z extent
 // (0: 8) and bits 20-23 its x extent (0: 4).
-// Automatic: N >= 8 the columns of best_columns; below, XCD chunks of a slice
-// (one rhs at 64x32^3: 0.46 ms against 0.51-0.57 ms for the other traversals).
+// Automatic: N >= 8 the columns of best_columns; below, XCD chunks of a slice: over 1,
+// 2, 4 and 7 rhs in each precision on six lattices (16^4 to 64x32^3) the best columns
+// of each case take 0.97 to 1.04 times as long in the geometric mean (0.81 to 1.15).
 // K: complexes per 16 bytes of the operator's spinors (1 FP64, 2 FP32, 4
 // FP16+norm).  The FP32 operator of 8 to 20 rhs on the whole lattice marches in t
 // (mode 6, marches of 4 slices) where the 8 x 8 patches of a cross-section divide
@@ -1584,10 +1589,14 @@ int reduce_stage1(cvchip_ctx *c, const double *part, int nblk, int rows, int slo
     *n = nblk;
     return 0;
   }
+  if (slot < 0 || slot >= kReduceSlots || rows > kReduceRows) {
+    set_error("partial sums: slot %d of %d, %d rows of %d", slot, kReduceSlots, rows, kReduceRows);
+    return CVCHIP_ERR_STATE;
+  }
   // every slot at the size of a full set of rows, so that no call grows the
   // scratch under another's result
-  const size_t room = (size_t)5 * 256 * kSegMax;
-  CVC_TRY(ensure_red2(c, sizeof(double) * 3 * room));
+  const size_t room = (size_t)kReduceRows * kSegMax;
+  CVC_TRY(ensure_red2(c, sizeof(double) * kReduceSlots * room));
   double *seg = (double *)c->red2.ptr + slot * room;
   hipLaunchKernelGGL(k_reduce_seg, dim3(rows * G), dim3(256), 0, c->stream, part, nblk, G, seg);
   CVC_HIP(hipGetLastError());

@@ -751,7 +751,8 @@ static int solve_setup(cvchip_ctx *c, Solve &S, int N, int64_t V = 0) {
   S.nt = (size_t)S.VN * 192 >= ((size_t)128 << 20) ? 1 : 0;
   // room for the operator's partials too (its traversal has its own block count)
   const size_t nb_max = std::max<size_t>(S.nblk, dslash_blocks(c, N));
-  // (two launches' norms side by side in Op::apply_omega)
+  // (side by side in Op::apply_omega: the 2 rows of <r2,s>, then the 5 of one launch or
+  // the 1 and 3 of two: at most 7)
   CVC_TRY(ensure_red(c, sizeof(double) * (nb_max * 7 * N + 64 * 256)));
   CVC_TRY(solve_buffers(c, c->solve_bufs));
   S.st = (RhsState *)c->solve_bufs.st;

@@ -251,8 +251,10 @@ __global__ void k_reduce_partials(const double *__restrict__ part, int nblk, int
                                   double *__restrict__ res);
 
 // First stage alone, for kernels that add the rest of each row themselves: *out / *n
-// are the rows and their length, either part itself or segment sums in the
-// context's second scratch (half `slot` of it: two results may be in use at once).
+// are the rows and their length, either part itself or segment sums in slot `slot`
+// of the context's second scratch.  The results of kReduceSlots calls with different
+// slots may be in use at once, for up to kReduceRows rows each.
+constexpr int kReduceSlots = 3, kReduceRows = 5 * 256;
 int reduce_stage1(cvchip_ctx *c, const double *part, int nblk, int rows, int slot, const double **out, int *n);
 
 int reduce_partials(cvchip_ctx *c, const double *part, int nblk, int Q, int N, double *res);
